@@ -1,14 +1,14 @@
 // bf16 GEMM on gfx950 matrix cores: C[M,N] = A[M,K] * B[K,N] (+ R[M,N]), all row-major, fp32
 // accumulation, one bf16 rounding at the store.
 //
-// Workgroup tiles of 256x256, 256x192, 256x128, 128x128 or 64x128 (Shape below), 4 waves in a 2x2
-// arrangement, each wave owning WM x WN v_mfma_f32_32x32x16_bf16 accumulators (256 fp32 per lane
-// for 256x256 tiles, held in AGPRs).
+// Workgroup tiles of 256x256, 256x192, 256x128, 128x256, 128x128 or 64x128 (Shape below), 4 waves in
+// a 2x2 arrangement, each wave owning WM x WN v_mfma_f32_32x32x16_bf16 accumulators (256 fp32 per
+// lane for 256x256 tiles, held in AGPRs).
 //
-// Operands move HBM -> LDS with buffer_load_dwordx4 ... lds (no VGPR staging).  256-row tiles stage
-// 64 K columns at a time (a whole 128-byte line of every A row) -- 256x128 tiles in a ring of three
-// slots, 256x256 and 256x192 tiles in rings of three A slots and two B slots (160 / 144 KB) -- and
-// 128x128 and smaller tiles 32 columns in rings of four slots.  Each stage's DMAs run two (or three)
+// Operands move HBM -> LDS with buffer_load_dwordx4 ... lds (no VGPR staging), 64 K columns at a time
+// (a whole 128-byte line of every A row; the grouped mode's 128x128 tiles 32): 256x128 and 128x256
+// tiles in a ring of three slots, 256x256 and 256x192 tiles in rings of three A slots and two B slots
+// (160 / 144 KB), 128x128 and 64x128 tiles in rings of four.  Each stage's DMAs run two (or three)
 // stages ahead and spread over a whole K step's MFMAs, into the slots the previous step's barrier
 // freed.  A and B keep their global layouts in LDS with 16-byte chunks XOR-swizzled per row, so
 // every fragment read is bank-conflict free:
@@ -29,8 +29,10 @@
 // grouped (the MoE grouped GEMM: a program table maps row tiles to weights).
 //
 // Tile order is XCD-aware: hardware hands workgroup i to XCD i % 8, so ids are remapped to give
-// each XCD a contiguous range of tiles, walked in groups of 8 tile-rows for L2 reuse.
+// each XCD a contiguous range of tiles, walked in groups of 8 tile-rows for L2 reuse; split-K walks
+// one K slice's tiles after the other, so that an XCD's workgroups share their slice's panels.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "ptb_common.h"
@@ -43,8 +45,9 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kGroupM = 8;
-// K past the end the DMA stream may address (the deepest ring: 4 stages of 32 or 2 of 64)
-constexpr int kRunAhead = 128;
+// K past the end the DMA stream may address: two 64-deep stages (three 32-deep ones), or three in the
+// four-slot rings of 64-deep stages
+constexpr int kRunAhead = 128, kRunAheadDeep = 192;
 // Widest C (columns) the epilogue addresses: a 256-row tile of it stays within 2^31 bytes, so its
 // 32-bit store offsets, and the 0x80000000 that marks a column outside C, stay in range.
 constexpr int64_t kMaxOutCols = int64_t(1) << 22;
@@ -55,12 +58,14 @@ typedef short i16x8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 
 // Tile shape: the 4 waves sit 2x2, each owning WM x WN blocks of 32x32, so the workgroup tile is
-// BM = 64*WM rows by BN = 64*WN columns (256x256, 256x192, 256x128, 128x128 or 64x128).  A stage
-// holds BK of K: 32 (a 64-byte piece of every A row; 128x128 and 64x128 tiles) in rings of 4 slots,
-// or 64 (a whole 128-byte line of every A row: the L2 serves a request per line, and a half-line
-// request costs a whole one) in rings of 3 slots (256x128 tiles) or of 3 A slots and 2 B slots
-// (256x256, 256x192).  Stage
-// kt + DIST, DIST = NSA - 1 = 2 or 3, refills the slots of stage kt-1, which the barrier of step
+// BM = 64*WM rows by BN = 64*WN columns (256x256, 256x192, 256x128, 128x256, 128x128 or 64x128).  A
+// stage holds BK of K: 64 (a whole 128-byte line of every A row: the L2 serves a request per line,
+// and a half-line request costs a whole one) in rings of 3 slots (256x128, 128x256), of 3 A slots and
+// 2 B slots (256x256, 256x192) or of 4 slots (128x128, 64x128: a workgroup of these is alone on its
+// CU and its step's MFMAs are short, so a third stage in flight pays: 4.5% over 3 slots), or 32 (the
+// grouped mode's 128x128 tiles, two workgroups a CU) in rings of 4 slots.  64-deep stages took
+// one-round shapes of 128x128 tiles from 53 to 42 us (640x4096x6144) and 48 to 39 us
+// (1024x4096x4096).  Stage kt + DIST, DIST = NSA - 1 = 2 or 3, refills the slots of stage kt-1, which the barrier of step
 // kt-1 freed, so the stage's DMAs spread over all of step kt's MFMAs; with two B slots, its B part
 // waits for the barrier of step kt and spreads over the slice after it.
 template <int WM, int WN, int BKT>
@@ -71,7 +76,7 @@ struct Shape {
   // refills a slot only after the barrier that frees it (the "hybrid" schedule below); every other
   // ring is one slot deeper than its DMA distance.
   static constexpr bool kHybrid = BK == 64 && WM * WN >= 12;
-  static constexpr int NSA = BK == 64 ? 3 : 4;
+  static constexpr int NSA = BK == 64 && WM * WN >= 8 ? 3 : 4;
   static constexpr int NSB = kHybrid ? 2 : NSA;
   static constexpr int NS = NSA;
   static constexpr int DIST = NSA - 1;
@@ -121,8 +126,8 @@ struct Groups {
 constexpr int kMaxPrograms = 256;
 constexpr int kMaxDedupGroups = 1024;   // group tables up to this size have repeated programs skipped
 
-// Split-K mode: workgroup (tile, blockIdx.y = s) multiplies K columns [s*kchunk, s*kchunk + kchunk)
-// and stores its fp32 partial tile at part + s*M*N; splitk_finish sums the partials.
+// Split-K mode: workgroup (tile, slice s) multiplies K columns [s*kchunk, s*kchunk + kchunk) and
+// stores its fp32 partial tile at part + s*M*N; splitk_finish sums the partials.
 // SwiGLU mode (the gate_up GEMM with silu(gate) * up fused into its epilogue): B is [K, 2*I] with
 // gate columns [0, I) and up columns [I, 2I); a 256x256 workgroup tile's B columns alternate in
 // 32-wide blocks between gate and up columns of the same 128 output columns, so each wave's
@@ -148,9 +153,13 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
   // ---- tile selection: tile id -> (first row, first column); ids are spread so that each XCD
   //      takes a contiguous range of tiles, walked in groups of kGroupM tile-rows
   const int ntiles = tiles_m * tiles_n;
-  auto tile_origin = [&](int id, int& tm0, int& tn0) __attribute__((always_inline)) {
-    int pid = id;
-    if ((ntiles & 7) == 0) pid = (pid & 7) * (ntiles >> 3) + (pid >> 3);
+  // XCD x takes ids x, x + 8, ...: the n / 8 (one more for the first n % 8) consecutive positions
+  // from x * (n / 8) + min(x, n % 8)
+  auto xcd_position = [](int id, int n) __attribute__((always_inline)) {
+    const int x = id & 7;
+    return x * (n >> 3) + min(x, n & 7) + (id >> 3);
+  };
+  auto tile_origin = [&](int pid, int& tm0, int& tn0) __attribute__((always_inline)) {
     const int width = kGroupM * tiles_n;
     const int first_m = (pid / width) * kGroupM;
     const int gsize = min(tiles_m - first_m, kGroupM);
@@ -164,6 +173,7 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
   uint16_t* C = C_in;
   int M = M_in, m0, n0;
   int Kl = K;    // the K columns this workgroup multiplies
+  int slice = 0; // split-K: this workgroup's K slice
   if constexpr (MODE == kGrouped) {
     __shared__ int pref[kMaxPrograms + 1];
     __shared__ int wsum[kThreads / 64];
@@ -214,13 +224,16 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
     m0 = 0;
     n0 = tn * BN;
   } else {
+    int pid = xcd_position(blockIdx.x, PERSIST ? ntiles : int(gridDim.x));
     if constexpr (MODE == kSplit) {
-      const int k0 = int(blockIdx.y) * kchunk;
+      slice = pid / ntiles;
+      pid -= slice * ntiles;
+      const int k0 = slice * kchunk;
       Kl = min(kchunk, K - k0);
       A = A_in + k0;
       B = B_in + int64_t(k0) * N;
     }
-    tile_origin(blockIdx.x, m0, n0);
+    tile_origin(pid, m0, n0);
   }
 
   const int tid = threadIdx.x;
@@ -229,7 +242,7 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
 
   // ---- loaders: A tile rows past M read as zero (num_records); B columns past N are read from
   //      the next row or as zero, and only feed columns of C that are never stored
-  const int koff = MODE == kSplit ? int(blockIdx.y) * kchunk : 0;   // this split's first K column
+  const int koff = MODE == kSplit ? slice * kchunk : 0;   // this slice's first K column
   auto make_rsrc_a = [&](int tm0) __attribute__((always_inline)) {
     return make_rsrc(A + int64_t(tm0) * K, uint32_t(int64_t(min(BM, M - tm0)) * K - koff) * 2u);
   };
@@ -479,7 +492,7 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
   const int next_id = tile_id + int(gridDim.x);
   const bool has_next = PERSIST && next_id < ntiles;
   int nm0 = 0, nn0 = 0;
-  if (has_next) tile_origin(next_id, nm0, nn0);
+  if (has_next) tile_origin(xcd_position(next_id, ntiles), nm0, nn0);
   auto prefetch_next = [&]() __attribute__((always_inline)) {
     if (has_next) {
       rsrc_a = make_rsrc_a(nm0);
@@ -491,25 +504,7 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
 
   // ---- epilogue: accumulator (i, j, r) of lane holds C row m0 + wm*BM/2 + i*32 + lane%32,
   //      column n0 + wn*BN/2 + j*32 + 8*(r/4) + 4*(lane/32) + r%4: 4 consecutive columns per r/4
-  if constexpr (MODE == kSplit) {
-#pragma unroll
-    for (int i = 0; i < WM; ++i) {
-      const int row = m0 + wm * (BM / 2) + i * 32 + fr;
-      if (row >= M) continue;
-#pragma unroll
-      for (int j = 0; j < WN; ++j) {
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int col = n0 + wn * (BN / 2) + j * 32 + 8 * g + 4 * h;
-          if (col >= N) continue;  // N % 8 == 0: a 4-column group is all in or all out
-          *reinterpret_cast<f32x4v*>(part + int64_t(blockIdx.y) * M * N + int64_t(row) * N + col) =
-              f32x4v{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-        }
-      }
-    }
-    return;
-  }
-  // Plain, grouped and SwiGLU tiles leave through the LDS, which is free now (every DMA has landed
+  // Tiles leave through the LDS, which is free now (every DMA has landed
   // and, past the barrier, no wave reads a stage): a wave writes one 32-row block of its results
   // (bf16; fp32 where a residual is still to be added, and in the persistent walk) (WJ 32-column
   // blocks; value(i, jj, g) gives
@@ -606,7 +601,39 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
       }
     }
   };
-  if constexpr (MODE == kSwiGLU) {
+  if constexpr (MODE == kSplit) {
+    // the slice's fp32 partial sums, staged the same way: whole rows of WN * 128 bytes a store
+    // instruction (16 bytes into each of 32 rows straight from the accumulators)
+    constexpr int WC = WN * 32, kPitch = WC * 4 + 16, LPR = WC / 4, RPI = 64 / LPR;
+    static_assert(64 % LPR == 0, "whole rows per instruction (no split-K form of 96-column waves)");
+    static_assert(4 * 32 * kPitch <= Sh::kSmemBytes, "the staging regions fit in the ring's LDS");
+    uint8_t* const stage = smem + wave * (32 * kPitch);
+    const int rl = lane / LPR, c4 = lane % LPR;
+    const int gcol = n0 + wn * (BN / 2) + 4 * c4;
+    const __amdgpu_buffer_rsrc_t rsrc_p =
+        __builtin_amdgcn_make_buffer_rsrc(part + int64_t(slice) * M * N + int64_t(m0) * N, 0,
+                                          uint32_t(min(BM, M - m0)) * uint32_t(N) * 4u, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < WM; ++i) {
+      const int r0 = wm * (BM / 2) + i * 32 + rl;
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<f32x4v*>(stage + fr * kPitch + (j * 32 + 8 * g + 4 * h) * 4) =
+              f32x4v{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+      u32x4 sv[32 / RPI];
+#pragma unroll
+      for (int t = 0; t < 32 / RPI; ++t)
+        sv[t] = *reinterpret_cast<const u32x4*>(stage + (t * RPI + rl) * kPitch + c4 * 16);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < 32 / RPI; ++t) {
+        const uint32_t off = gcol < N ? (uint32_t(r0 + t * RPI) * uint32_t(N) + uint32_t(gcol)) * 4u : 0x80000000u;
+        __builtin_amdgcn_raw_buffer_store_b128(sv[t], rsrc_p, off, 0, 0);
+      }
+    }
+  } else if constexpr (MODE == kSwiGLU) {
     // pair jp of this wave: gate acc[i][2jp], up acc[i][2jp+1] -> output columns
     // n0 + 32*(wn*WN/2 + jp) + 8*(r/4) + 4*(lane/32) + r%4 of C [M, N/2]
     store_staged(std::integral_constant<int, WN / 2>{}, [&](int i, int jp, int g) __attribute__((always_inline)) {
@@ -643,19 +670,12 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
   }   // tile walk
 }
 
-// 256x256 and 256x128 tiles take 64-deep stages (whole-line A requests), 128x128 tiles 32-deep
-// ones.  For 256x256 tiles the 3 A + 2 B slot rings beat 32-deep stages in 4-slot rings (same box:
-// 4096x4096x12288 314.6 -> 306.8 us, SwiGLU 2048x4096x24576 305.7 -> 297.8 us, 2048x4096x6144
-// 89.7 -> 86.5 us).
-template <int WM, int WN>
-constexpr int kBKOf = WM * WN >= 8 ? 64 : 32;
-
 int cu_count();
 
 template <int WM, int WN>
 int launch_gemm(const void* a, const void* b, const void* residual, void* c, int64_t m, int64_t n, int64_t k,
                 hipStream_t s) {
-  using Sh = Shape<WM, WN, kBKOf<WM, WN>>;
+  using Sh = Shape<WM, WN, 64>;
   const int64_t tm = (m + Sh::BM - 1) / Sh::BM, tn = (n + Sh::BN - 1) / Sh::BN;
   if (tm * tn > 0x7fffffff) return PTB_ERR_GRID;
   const dim3 grid(unsigned(tm * tn)), block(kThreads);
@@ -671,11 +691,11 @@ int launch_gemm(const void* a, const void* b, const void* residual, void* c, int
     }
   }
   if (residual)
-    gemm_bf16_kernel<WM, WN, true, kPlain, kBKOf<WM, WN>><<<grid, block, 0, s>>>(
+    gemm_bf16_kernel<WM, WN, true, kPlain, 64><<<grid, block, 0, s>>>(
         static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), static_cast<const uint16_t*>(residual),
         static_cast<uint16_t*>(c), int(m), int(n), int(k), int(tm), int(tn), none, nullptr, 0);
   else
-    gemm_bf16_kernel<WM, WN, false, kPlain, kBKOf<WM, WN>><<<grid, block, 0, s>>>(
+    gemm_bf16_kernel<WM, WN, false, kPlain, 64><<<grid, block, 0, s>>>(
         static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), nullptr, static_cast<uint16_t*>(c), int(m),
         int(n), int(k), int(tm), int(tn), none, nullptr, 0);
   return launch_status();
@@ -687,58 +707,68 @@ int cu_count() {
   return cus;
 }
 
-// Tile shape (wm x wn waves of 64x64 blocks: 4x4 = 256x256, 4x3 = 256x192, 4x2 = 256x128,
-// 2x2 = 128x128, 1x2 = 64x128) and K split of a GEMM.
+// Tile shape (BM = 64 wm rows by BN = 64 wn columns) and K split of a GEMM.
 struct GemmPlan {
   int wm, wn, splits;
   int64_t kchunk;   // K columns per split
 };
 
-// Split-K cost model for 64x128 tiles, fitted to the bundle's 97 GEMM shapes with M >= 8 (each
-// (tile, split) timed on MI355X by HIP-graph replay): a launch costs kLaunchUs; a workgroup streams
-// its (64 + 128) x K/S operand bytes at min(kWgBpus, kChipBpus / workgroups); a split adds the
-// finish launch and 8 bytes of partial traffic (written, then read) per output per slice.
-constexpr double kLaunchUs = 2.5, kFinishUs = 1.5;
-constexpr double kWgBpus = 90e3;       // bytes per us one workgroup streams
-constexpr double kChipBpus = 25e6;     // L2 -> CU bytes per us over the chip
-constexpr double kPartialBpus = 2.5e6;
+// Cost model of a plan, in us.  A round of workgroups (one a CU) costs `step` per 64-deep K step
+// plus `load` x (share of the CUs busy: they share the chip's power and L2 bandwidth) and `fixed` for
+// its prologue and epilogue.  Reading the operands and writing C takes kMemUs plus kMemUsPerMB; the
+// two overlap partly, which their root sum of squares follows.  A split adds the finish launch,
+// kFinishUs, and writing and reading 4 bytes per output and slice at kPartialUsPerMB.  Fitted by
+// least squares to 3969 (shape, tile, split) times on MI355X over 239 shapes with M 1 .. 4096, K
+// 64 .. 12288 and N 128 .. 24576: 4.7% rms error, and the plans it picks run within 0.9% (geometric
+// mean) of the best measured plan of each shape, 1.23x faster than the previous rule's plans (one
+// pass of 128x128 tiles where those covered 3/4 of the CUs, splits of 64x128 tiles only; both with
+// 32-deep stages): 640x12288x4096 147 -> 71 us, 1280x12288x4096 237 -> 114, 384x12288x4096 105 -> 50,
+// 640x4096x6144 53 -> 42, 2048x4096x12288 173 -> 150, 32x4096x6144 16 -> 14.5, 3000x8192x512 65 -> 36.
+struct TileCost {
+  int wm, wn;
+  double step, load, fixed;
+};
+constexpr TileCost kTiles[] = {{4, 4, 0.816, 0.464, 6.29}, {4, 3, 0.620, 0.511, 5.89}, {4, 2, 0.555, 0.203, 3.72},
+                               {2, 4, 0.592, 0.250, 3.92}, {2, 2, 0.358, 0.196, 2.42}, {1, 2, 0.296, 0.141, 1.68}};
+constexpr double kMemUs = 3.3, kMemUsPerMB = 0.106, kFinishUs = 1.9, kPartialUsPerMB = 0.148;
+constexpr int kMaxSplits = 8;
+constexpr int64_t kFitK = 16384;   // past it (the fit ends at 12288) splits keep to the narrow rule below
 
-// The largest tile that still gives every CU a tile: 256x256, else 256x128 (from 3/4 of the CUs:
-// one round of them beats 1.5 rounds of 128x128 tiles, 8192x3072x768 48.6 -> 35.3 us); then
-// 128x128 while its tiles cover 3/4 of the CUs (or 64x128 ones would need a second round); else
-// 64x128 (column tiles stay 128 wide: the B swizzle spans 16 chunks), its K split S ways (S fills at
-// most one round, slices at least 256 deep, K >= 1024) when the model above says the split pays:
-// over those 97 shapes the model's plans run 1.13x faster (geometric mean) than one pass of
-// 128x128 tiles or 128x128 splits, within 0.3% of the best measured plan.  Where 256x256 tiles
-// leave CUs idle but 256x128 ones would need a second round, 256x192 tiles when one round of them
-// covers more CUs (the fused q|k|v projection, 2048x4096x6144: 256 tiles against 192), else 256x256:
-// a 256x256 workgroup moves ~1.4x the flops per CU of a 256x128 one, so one round of it beats two
-// of the smaller.
+// The cheapest plan by the model.  Splits: K at least 1024 and slices at least 128 deep (below, the
+// finish launch costs more than the shorter slices save), all in one round of workgroups; a K past
+// the fitted range is split only when 128x128 tiles would leave a quarter of the CUs idle.  256-row
+// and 128-row tiles need 256 rows of A within the 32-bit buffer offsets, and the four-slot rings
+// their deeper run past the end of a slice of B.
 GemmPlan gemm_plan(int64_t m, int64_t n, int64_t k, bool may_split) {
   const int64_t cus = cu_count();
   auto tiles = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
-  const int64_t t256 = tiles(256, 256), t256x192 = tiles(256, 192), t256x128 = tiles(256, 128);
-  const int64_t t128 = tiles(128, 128), t64 = tiles(64, 128);
-  if (t256 < cus && t256x128 > cus && t256x192 <= cus && t256x192 > t256) return {4, 3, 1, k};
-  if (t256 >= cus || t256x128 > cus) return {4, 4, 1, k};
-  if (4 * t256x128 >= 3 * cus) return {4, 2, 1, k};
-  if (4 * t128 >= 3 * cus || (t64 > cus && 2 * t128 >= cus)) return {2, 2, 1, k};
-  int best_s = 1;
-  double best_t = 0.0;
-  for (int sp = 1; sp <= 8; sp *= 2) {
-    if (sp > 1 && (!may_split || k < 1024 || k / sp < 256 || t64 * sp > cus)) continue;
-    const double wgs = double(t64 * sp);
-    const double rate = std::min(kWgBpus, kChipBpus / std::min(wgs, double(cus)));
-    double t = kLaunchUs + double(k) / sp * (64 + 128) * 2 / rate;
-    if (sp > 1) t += kFinishUs + sp * double(m) * double(n) * 8 / kPartialBpus;
-    if (sp == 1 || t < best_t) {
-      best_t = t;
-      best_s = sp;
+  if (k < 1024 || (k > kFitK && 4 * tiles(128, 128) >= 3 * cus)) may_split = false;
+  const double mem = kMemUs + kMemUsPerMB * 2e-6 * (double(k) * double(n) + double(m) * (double(k) + double(n)));
+  const double partial = kPartialUsPerMB * 8e-6 * double(m) * double(n);
+  const bool tall = int64_t(256) * k * 2 < (int64_t(1) << 32);
+  GemmPlan best{1, 2, 1, k};
+  double best_t = -1.0;
+  for (const TileCost& c : kTiles) {
+    if (c.wm > 1 && !tall) continue;
+    const int64_t t = tiles(64 * c.wm, 64 * c.wn);
+    const int run_ahead = c.wm * c.wn >= 8 ? kRunAhead : kRunAheadDeep;
+    for (int sp = 1; sp <= (may_split && c.wn != 3 ? kMaxSplits : 1); ++sp) {
+      if (sp > 1 && (t * sp > cus || k / sp < 128)) break;
+      const int64_t kc = sp == 1 ? k : ((k + sp - 1) / sp + 63) / 64 * 64;
+      const int64_t splits = (k + kc - 1) / kc;
+      if ((kc + run_ahead) * n * 2 >= (int64_t(1) << 32)) continue;
+      const int64_t w = t * splits, full = (w - 1) / cus;
+      const double steps = double((kc + 63) / 64), last = double(w - full * cus) / double(cus);
+      const double body = double(full) * (steps * (c.step + c.load) + c.fixed) + steps * (c.step + c.load * last) + c.fixed;
+      double us = std::sqrt(body * body + mem * mem);
+      if (splits > 1) us += kFinishUs + partial * double(splits);
+      if (best_t < 0.0 || us < best_t) {
+        best_t = us;
+        best = GemmPlan{c.wm, c.wn, int(splits), kc};
+      }
     }
   }
-  if (best_s == 1) return {1, 2, 1, k};
-  const int64_t kc = ((k + best_s - 1) / best_s + 63) / 64 * 64;
-  return {1, 2, int((k + kc - 1) / kc), kc};
+  return best;
 }
 
 int launch_planned(const GemmPlan& p, const void* a, const void* b, const void* residual, void* c, int64_t m,
@@ -746,6 +776,7 @@ int launch_planned(const GemmPlan& p, const void* a, const void* b, const void* 
   if (p.wm == 4 && p.wn == 3) return launch_gemm<4, 3>(a, b, residual, c, m, n, k, s);
   if (p.wm == 4 && p.wn == 4) return launch_gemm<4, 4>(a, b, residual, c, m, n, k, s);
   if (p.wm == 4 && p.wn == 2) return launch_gemm<4, 2>(a, b, residual, c, m, n, k, s);
+  if (p.wm == 2 && p.wn == 4) return launch_gemm<2, 4>(a, b, residual, c, m, n, k, s);
   if (p.wm == 2 && p.wn == 2) return launch_gemm<2, 2>(a, b, residual, c, m, n, k, s);
   return launch_gemm<1, 2>(a, b, residual, c, m, n, k, s);
 }
@@ -771,27 +802,19 @@ PTB_EXPORT int ptb_gemm_bf16(const void* a, const void* b, const void* residual,
 
 namespace {
 
-// C = bf16(sum_s P[s] (+ R)), 4 consecutive elements per thread.
-// Eight slices' loads go out before any is added (a plain loop waits for each in turn); the sum
-// keeps the slice order, P_0 + P_1 + ... .
-__global__ __launch_bounds__(256) void splitk_finish(const float* __restrict__ P, int splits, int64_t mn,
+// C = bf16(sum_s P[s] (+ R)), 4 consecutive elements per thread, the slices in order, P_0 + P_1 + ...;
+// all S loads go out before the first add.
+template <int S>
+__global__ __launch_bounds__(256) void splitk_finish(const float* __restrict__ P, int64_t mn,
                                                      const uint16_t* __restrict__ R, uint16_t* __restrict__ C) {
   const int64_t q = (int64_t(blockIdx.x) * 256 + threadIdx.x) * 4;
   if (q >= mn) return;
-  f32x4v acc = {0.f, 0.f, 0.f, 0.f};
-  for (int s0 = 0; s0 < splits; s0 += 8) {
-    f32x4v v[8];
+  f32x4v v[S];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int sl = s0 + u < splits ? s0 + u : splits - 1;
-      v[u] = *reinterpret_cast<const f32x4v*>(P + int64_t(sl) * mn + q);
-    }
+  for (int u = 0; u < S; ++u) v[u] = *reinterpret_cast<const f32x4v*>(P + int64_t(u) * mn + q);
+  f32x4v acc = v[0];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int sl = s0 + u;
-      acc = sl == 0 ? v[u] : (sl < splits ? acc + v[u] : acc);
-    }
-  }
+  for (int u = 1; u < S; ++u) acc = acc + v[u];
   if (R) {
     const u32x2 rr = *reinterpret_cast<const u32x2*>(R + q);
     acc.x += bf16_lo(rr[0]);
@@ -802,13 +825,38 @@ __global__ __launch_bounds__(256) void splitk_finish(const float* __restrict__ P
   *reinterpret_cast<u32x2*>(C + q) = u32x2{pack_bf16x2(acc.x, acc.y), pack_bf16x2(acc.z, acc.w)};
 }
 
+template <int WM, int WN>
+int launch_split(const GemmPlan& p, const uint16_t* a, const uint16_t* b, const uint16_t* residual, uint16_t* c,
+                 float* part, int64_t m, int64_t n, int64_t k, hipStream_t s) {
+  using Sh = Shape<WM, WN, 64>;
+  const int64_t tm = (m + Sh::BM - 1) / Sh::BM, tn = (n + Sh::BN - 1) / Sh::BN;   // at most a tile a CU
+  const Groups none{nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
+  gemm_bf16_kernel<WM, WN, false, kSplit, 64><<<dim3(unsigned(tm * tn * p.splits)), dim3(kThreads), 0, s>>>(
+      a, b, nullptr, nullptr, int(m), int(n), int(k), int(tm), int(tn), none, part, int(p.kchunk));
+  const int64_t mn = m * n;
+  const dim3 grid(unsigned((mn / 4 + 255) / 256)), block(256);
+  static_assert(kMaxSplits == 8, "a finish kernel for every split count");
+  switch (p.splits) {
+    case 2: splitk_finish<2><<<grid, block, 0, s>>>(part, mn, residual, c); break;
+    case 3: splitk_finish<3><<<grid, block, 0, s>>>(part, mn, residual, c); break;
+    case 4: splitk_finish<4><<<grid, block, 0, s>>>(part, mn, residual, c); break;
+    case 5: splitk_finish<5><<<grid, block, 0, s>>>(part, mn, residual, c); break;
+    case 6: splitk_finish<6><<<grid, block, 0, s>>>(part, mn, residual, c); break;
+    case 7: splitk_finish<7><<<grid, block, 0, s>>>(part, mn, residual, c); break;
+    default: splitk_finish<8><<<grid, block, 0, s>>>(part, mn, residual, c); break;
+  }
+  return launch_status();
+}
+
+size_t plan_workspace(const GemmPlan& p, int64_t m, int64_t n) {
+  return p.splits < 2 ? 0 : size_t(p.splits) * size_t(m) * size_t(n) * sizeof(float);
+}
+
 }  // namespace
 
 PTB_EXPORT size_t ptb_gemm_bf16_workspace_bytes(int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || n <= 0 || k <= 0 || m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff) return 0;
-  const GemmPlan p = gemm_plan(m, n, k, true);
-  if (p.splits < 2) return 0;
-  return size_t(p.splits) * size_t(m) * size_t(n) * sizeof(float);
+  return plan_workspace(gemm_plan(m, n, k, true), m, n);
 }
 
 PTB_EXPORT int ptb_gemm_bf16_ws(const void* a, const void* b, const void* residual, void* c, int64_t m, int64_t n,
@@ -818,26 +866,22 @@ PTB_EXPORT int ptb_gemm_bf16_ws(const void* a, const void* b, const void* residu
   const GemmPlan p = gemm_plan(m, n, k, true);
   if (p.splits < 2) return ptb_gemm_bf16(a, b, residual, c, m, n, k, stream);   // no split for this shape
   if (!a || !b || !c || !workspace) return PTB_ERR_NULL;
-  if (workspace_bytes < ptb_gemm_bf16_workspace_bytes(m, n, k)) return PTB_ERR_WORKSPACE;
-  using Sh = Shape<1, 2, kBKOf<1, 2>>;   // the split plans use 64x128 tiles
-  if ((k + kRunAhead) * n * 2 >= (int64_t(1) << 32) || int64_t(Sh::BM) * k * 2 >= (int64_t(1) << 32))
+  if (workspace_bytes < plan_workspace(p, m, n)) return PTB_ERR_WORKSPACE;
+  // B and a tile's rows of A within 32-bit buffer offsets (the plan takes 64-row tiles past K = 2^23)
+  if ((k + kRunAhead) * n * 2 >= (int64_t(1) << 32) || int64_t(64) * k * 2 >= (int64_t(1) << 32))
     return PTB_ERR_UNSUPPORTED;
   if (!aligned16(a) || !aligned16(b) || !aligned16(c) || !aligned16(workspace) || (residual && !aligned16(residual)))
     return PTB_ERR_ALIGN;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int64_t tm = (m + Sh::BM - 1) / Sh::BM, tn = (n + Sh::BN - 1) / Sh::BN;
-  if (tm * tn > 0x7fffffff) return PTB_ERR_GRID;
-  const Groups none{nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
+  auto ap = static_cast<const uint16_t*>(a), bp = static_cast<const uint16_t*>(b);
+  auto rp = static_cast<const uint16_t*>(residual);
+  auto cp = static_cast<uint16_t*>(c);
   float* part = static_cast<float*>(workspace);
-  const int splits = p.splits;
-  const dim3 grid(unsigned(tm * tn), unsigned(splits));
-  gemm_bf16_kernel<1, 2, false, kSplit, kBKOf<1, 2>><<<grid, dim3(kThreads), 0, s>>>(
-        static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), nullptr, nullptr, int(m), int(n), int(k),
-        int(tm), int(tn), none, part, int(p.kchunk));
-  const int64_t mn = m * n;
-  splitk_finish<<<dim3(unsigned((mn / 4 + 255) / 256)), dim3(256), 0, s>>>(
-      part, splits, mn, static_cast<const uint16_t*>(residual), static_cast<uint16_t*>(c));
-  return launch_status();
+  if (p.wm == 4 && p.wn == 4) return launch_split<4, 4>(p, ap, bp, rp, cp, part, m, n, k, s);
+  if (p.wm == 4) return launch_split<4, 2>(p, ap, bp, rp, cp, part, m, n, k, s);
+  if (p.wm == 2 && p.wn == 4) return launch_split<2, 4>(p, ap, bp, rp, cp, part, m, n, k, s);
+  if (p.wm == 2) return launch_split<2, 2>(p, ap, bp, rp, cp, part, m, n, k, s);
+  return launch_split<1, 2>(p, ap, bp, rp, cp, part, m, n, k, s);
 }
 
 PTB_EXPORT int ptb_gemm_swiglu_bf16(const void* a, const void* b, void* c, int64_t m, int64_t inter, int64_t k,
@@ -855,7 +899,7 @@ PTB_EXPORT int ptb_gemm_swiglu_bf16(const void* a, const void* b, void* c, int64
   const int64_t tm = (m + 255) / 256, tn = inter / 128;
   if (tm * tn > 0x7fffffff) return PTB_ERR_GRID;
   const Groups none{nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
-  gemm_bf16_kernel<4, 4, false, kSwiGLU, kBKOf<4, 4>><<<dim3(unsigned(tm * tn)), dim3(kThreads), 0,
+  gemm_bf16_kernel<4, 4, false, kSwiGLU, 64><<<dim3(unsigned(tm * tn)), dim3(kThreads), 0,
                                                         static_cast<hipStream_t>(stream)>>>(
       static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), nullptr, static_cast<uint16_t*>(c), int(m),
       int(n), int(k), int(tm), int(tn), none, nullptr, 0);

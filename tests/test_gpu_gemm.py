@@ -119,6 +119,38 @@ def test_gemm_bundle_inputs_exact_products():
     assert bits_equal(c, oracle.gemm(a, b))
 
 
+@pytest.mark.parametrize("m,k,n,resid", [
+    (1308, 64, 5408, True),       # 128x256 tiles, one K step: every stage past the first runs past K
+    (1893, 128, 4176, False),     # 128x256 tiles, ragged in M and N, 255 tiles (not a multiple of 8)
+    (1849, 512, 4152, True),      # the same, eight steps of the three-step loop
+    (2357, 64, 792, False),       # 128x128 tiles, one step of the four-step loop
+    (1491, 320, 1896, True),      # 128x128 tiles, five steps: a remainder of one
+    (1, 640, 4512, False),        # 64x128 tiles, one row, ten steps: a remainder of two
+    (110, 896, 56, True),         # 64x128 tiles, one ragged column tile
+    (9, 2304, 8, True),           # 64x128 tiles split 8 ways, a single tile
+    (355, 1216, 16, False),       # split 7 ways, the last slice a step shorter
+    (72, 1792, 5480, True),       # 128x128 tiles split 4 ways, ragged
+    (385, 4160, 4104, True),      # 256x128 tiles split
+    (262, 4416, 3744, False),     # 128x256 tiles split 5 ways, 45 tiles a slice
+    (387, 7104, 5592, True),      # 256x256 tiles split 5 ways, 44 tiles a slice
+])
+def test_gemm_planned_tiles_stay_inside_c(m, k, n, resid):
+    """Every tile shape and split of the plan at ragged sizes, step counts around the loops' turns and
+    tile counts that do not divide by the XCDs: small-integer operands make every partial sum exact in
+    fp32 (|sum| <= 9 * 12288 + 9 < 2^24), so the result is the oracle's bit for bit whatever the tiling,
+    and a NaN-filled guard after C's last element stays NaN."""
+    g = torch.Generator().manual_seed(m + n)
+    a = torch.randint(-3, 4, (m, k), generator=g).to(torch.bfloat16)
+    b = torch.randint(-3, 4, (k, n), generator=g).to(torch.bfloat16)
+    r = torch.randint(-9, 10, (m, n), generator=g).to(torch.bfloat16) if resid else None
+    guard = torch.full((m * n + 8192,), float("nan"), dtype=torch.bfloat16, device=DEV)
+    c = guard[: m * n].view(m, n)
+    ops.gemm(a.to(DEV), b.to(DEV), None if r is None else r.to(DEV), out=c)
+    assert bool(guard[m * n:].isnan().all()), "the GEMM wrote past C"
+    rows = torch.arange(m) if m * k * n < 2e9 else sample_rows(m, 6)
+    assert bits_equal(c.cpu()[rows], oracle.gemm(a[rows], b, None if r is None else r[rows]))
+
+
 def test_gemm_refuses_bad_k():
     a = torch.zeros((4, 100), dtype=torch.bfloat16, device=DEV)
     b = torch.zeros((100, 64), dtype=torch.bfloat16, device=DEV)
