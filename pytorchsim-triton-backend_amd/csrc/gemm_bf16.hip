@@ -126,13 +126,29 @@ struct Groups {
 constexpr int kMaxPrograms = 256;
 constexpr int kMaxDedupGroups = 1024;   // group tables up to this size have repeated programs skipped
 
+// The column of B (from the tile's first gate column; up columns I further) that a SwiGLU tile of WN
+// blocks a wave stages as its 16-byte chunk c.  Even WN: 32-wide blocks alternate between gate and up,
+// so a wave's accumulators 2jp and 2jp + 1 are the gate and up of the same 32 outputs.  WN = 3 (48
+// outputs a wave): block 0 the first 32 gate columns, block 2 their up columns, block 1 the last 16
+// gate columns, then their up columns, which a lane holds 8 accumulator registers apart.
+template <int WN>
+__device__ __forceinline__ int swiglu_col(int c, int inter) {
+  if constexpr (WN == 3) {
+    const int w = c / 12, r = c % 12;
+    return 48 * w + (r < 6 ? 8 * r : inter + (r < 8 ? 8 * (r - 2) : 8 * (r - 8)));
+  } else {
+    const int b = c >> 2;
+    return ((b & 1) ? inter : 0) + 32 * (b >> 1) + 8 * (c & 3);
+  }
+}
+
 // Split-K mode: workgroup (tile, slice s) multiplies K columns [s*kchunk, s*kchunk + kchunk) and
 // stores its fp32 partial tile at part + s*M*N; splitk_finish sums the partials.
 // SwiGLU mode (the gate_up GEMM with silu(gate) * up fused into its epilogue): B is [K, 2*I] with
-// gate columns [0, I) and up columns [I, 2I); a 256x256 workgroup tile's B columns alternate in
-// 32-wide blocks between gate and up columns of the same 128 output columns, so each wave's
-// accumulator pairs (j even: gate, j + 1: up) cover the same outputs and the epilogue stores
-// bf16(silu(bf16(gate)) * bf16(up)), as a separate silu_mul would compute it from the bf16 GEMM.
+// gate columns [0, I) and up columns [I, 2I); a workgroup tile's BN columns of B are the gate and up
+// columns of the same BN / 2 output columns, laid out so that a lane holds both of every output (see
+// swiglu_col), and the epilogue stores bf16(silu(bf16(gate)) * bf16(up)), as a separate silu_mul
+// would compute it from the bf16 GEMM.
 enum { kPlain = 0, kGrouped = 1, kSplit = 2, kSwiGLU = 3 };
 
 
@@ -267,11 +283,7 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
     const int piece = 64 * (wave * Sh::kDmaB + t) + lane;
     const int k = piece / Sh::kBSlots;
     const int bchunk = (piece % Sh::kBSlots) ^ b_swz<BN>(k);
-    int bcol = bchunk * 8;
-    if constexpr (MODE == kSwiGLU) {   // 32-wide block b: gate (b even) or up (b odd) of pair b / 2
-      const int b = bchunk >> 2;
-      bcol = ((b & 1) ? N / 2 : 0) + 32 * (b >> 1) + 8 * (bchunk & 3);
-    }
+    const int bcol = MODE == kSwiGLU ? swiglu_col<WN>(bchunk, N / 2) : bchunk * 8;
     b_voff[t] = uint32_t(k * N + bcol) * 2u;
   }
   const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(smem));
@@ -375,7 +387,7 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
   static_assert(!PERSIST || (WM == 4 && WN == 4 && BKT == 64 && !RESID && MODE == kPlain),
                 "the persistent walk is for plain 256x256 tiles (the SwiGLU form has no registers to spare)");
   // stores of the epilogue's second half, issued after the next tile's stage-0 DMAs
-  constexpr int kStoresAfter = (WM / 2) * 4 * (MODE == kSwiGLU ? WN / 2 : WN);
+  constexpr int kStoresAfter = (WM / 2) * 4 * WN;
   int tile_id = blockIdx.x;
   bool pre0 = false;   // this tile's stage 0 went out during the previous tile's epilogue
   for (;;) {
@@ -506,19 +518,17 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
   //      column n0 + wn*BN/2 + j*32 + 8*(r/4) + 4*(lane/32) + r%4: 4 consecutive columns per r/4
   // Tiles leave through the LDS, which is free now (every DMA has landed
   // and, past the barrier, no wave reads a stage): a wave writes one 32-row block of its results
-  // (bf16; fp32 where a residual is still to be added, and in the persistent walk) (WJ 32-column
-  // blocks; value(i, jj, g) gives
-  // the 4 fp32 columns 8g + 4*(lane/32) .. +3 of
-  // block jj for row lane%32) into a private, padded region and reads it back 4 columns a lane, so
+  // (bf16; fp32 where a residual is still to be added, and in the persistent walk) (NG groups of
+  // 8 columns; value(i, gg) gives the 4 fp32 columns 8gg + 4*(lane/32) .. +3 for row lane%32) into a private, padded region and reads it back 4 columns a lane, so
   // each store writes whole rows of its block (in the accumulator layout one store instruction
   // writes 16 bytes into each of 32 rows, which took 12% of a 256x256 tile's time) and the
   // residual is read the same way.  The region is the wave's own and LDS operations of a wave
   // complete in order, so no barrier separates its writes from its reads.  Rows past M and columns
   // past `cols` fall outside the buffer resources (stores dropped, loads 0): no branches.
   __syncthreads();
-  auto store_staged = [&](auto wj, auto value, uint16_t* out, int ldc, int cols, int col0) __attribute__((always_inline)) {
-    constexpr int WJ = decltype(wj)::value;
-    constexpr int WC = WJ * 32;           // columns of a wave's block
+  auto store_staged = [&](auto ng, auto value, uint16_t* out, int ldc, int cols, int col0) __attribute__((always_inline)) {
+    constexpr int NG = decltype(ng)::value;
+    constexpr int WC = NG * 8;            // columns of a wave's block
     // without a residual to add, each value is rounded to bf16 before it is staged (the rounding
     // the store would make anyway), halving the staged bytes; with one, the fp32 sum needs fp32.
     // The persistent walk keeps fp32 staging: its bf16 form needs registers it does not have
@@ -527,7 +537,8 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
     constexpr int kEl = kF32Stage ? 4 : 2;   // bytes per staged value
     constexpr int kPitch = WC * kEl + 16; // bytes per staged row: rows start 4 banks apart
     constexpr int LPR = WC / 4;           // lanes per row, 4 columns each
-    constexpr int RPI = 64 / LPR;         // rows per instruction (96 columns: 2 rows, 48 lanes)
+    // rows per instruction (96 columns: 2 rows on 48 lanes; 48 columns: 4 rows on 48 lanes)
+    constexpr int RPI = LPR == 12 ? 4 : 64 / LPR;
     static_assert(32 % RPI == 0, "whole instructions per 32-row block");
     static_assert(4 * 32 * kPitch <= Sh::kSmemBytes, "the staging regions fit in the ring's LDS");
     // a persistent walk keeps A slot 0 and B slot 0 free for the next tile's first stage: waves 0-2
@@ -560,16 +571,14 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
         for (int t = 0; t < 32 / RPI; ++t) rr[t] = __builtin_amdgcn_raw_buffer_load_b64(rsrc_r, voff[t], 0, 0);
       }
 #pragma unroll
-      for (int jj = 0; jj < WJ; ++jj)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const f32x4v v = value(i, jj, g);
-          if constexpr (kF32Stage)
-            *reinterpret_cast<f32x4v*>(stage + fr * kPitch + (jj * 32 + 8 * g + 4 * h) * 4) = v;
-          else
-            *reinterpret_cast<u32x2*>(stage + fr * kPitch + (jj * 32 + 8 * g + 4 * h) * 2) =
-                u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-        }
+      for (int gg = 0; gg < NG; ++gg) {
+        const f32x4v v = value(i, gg);
+        if constexpr (kF32Stage)
+          *reinterpret_cast<f32x4v*>(stage + fr * kPitch + (8 * gg + 4 * h) * 4) = v;
+        else
+          *reinterpret_cast<u32x2*>(stage + fr * kPitch + (8 * gg + 4 * h) * 2) =
+              u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      }
       // every staged row of the block read back before the first conversion: the reads' latencies
       // overlap instead of adding up pair by pair
       using Staged = std::conditional_t<kF32Stage, f32x4v, u32x2>;
@@ -634,14 +643,16 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
       }
     }
   } else if constexpr (MODE == kSwiGLU) {
-    // pair jp of this wave: gate acc[i][2jp], up acc[i][2jp+1] -> output columns
-    // n0 + 32*(wn*WN/2 + jp) + 8*(r/4) + 4*(lane/32) + r%4 of C [M, N/2]
-    store_staged(std::integral_constant<int, WN / 2>{}, [&](int i, int jp, int g) __attribute__((always_inline)) {
+    // output columns n0 + wn*BN/4 + 8*gg + 4*(lane/32) + e of C [M, N/2]: gate and up where swiglu_col
+    // put them
+    store_staged(std::integral_constant<int, 2 * WN>{}, [&](int i, int gg) __attribute__((always_inline)) {
+      const int gj = WN == 3 ? gg >> 2 : 2 * (gg >> 2), uj = WN == 3 ? (gg < 4 ? 2 : 1) : gj + 1;
+      const int gr = 4 * (gg & 3), ur = WN == 3 && gg >= 4 ? gr + 8 : gr;
       float gv[4], uv[4], bv[4], q[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        gv[e] = bf16_to_f32(f32_to_bf16(acc[i][2 * jp][4 * g + e]));
-        uv[e] = bf16_to_f32(f32_to_bf16(acc[i][2 * jp + 1][4 * g + e]));
+        gv[e] = bf16_to_f32(f32_to_bf16(acc[i][gj][gr + e]));
+        uv[e] = bf16_to_f32(f32_to_bf16(acc[i][uj][ur + e]));
         bv[e] = __builtin_amdgcn_exp2f(-gv[e] * 1.4426950408889634f) + 1.0f;
         q[e] = silu_quotient(gv[e], bv[e]);
       }
@@ -657,7 +668,8 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
       return o;
     }, C, N / 2, N / 2, n0 + wn * (BN / 4));
   } else {
-    store_staged(std::integral_constant<int, WN>{}, [&](int i, int j, int g) __attribute__((always_inline)) {
+    store_staged(std::integral_constant<int, 4 * WN>{}, [&](int i, int gg) __attribute__((always_inline)) {
+      const int j = gg >> 2, g = gg & 3;
       return f32x4v{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
     }, C, N, N, n0 + wn * (BN / 2));
   }
@@ -884,6 +896,22 @@ PTB_EXPORT int ptb_gemm_bf16_ws(const void* a, const void* b, const void* residu
   return launch_split<1, 2>(p, ap, bp, rp, cp, part, m, n, k, s);
 }
 
+namespace {
+
+template <int WM, int WN>
+int launch_swiglu(const void* a, const void* b, void* c, int64_t m, int64_t n, int64_t k, hipStream_t s) {
+  using Sh = Shape<WM, WN, 64>;
+  const int64_t tm = (m + Sh::BM - 1) / Sh::BM, tn = (n + Sh::BN - 1) / Sh::BN;
+  if (tm * tn > 0x7fffffff) return PTB_ERR_GRID;
+  const Groups none{nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
+  gemm_bf16_kernel<WM, WN, false, kSwiGLU, 64><<<dim3(unsigned(tm * tn)), dim3(kThreads), 0, s>>>(
+      static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), nullptr, static_cast<uint16_t*>(c), int(m),
+      int(n), int(k), int(tm), int(tn), none, nullptr, 0);
+  return launch_status();
+}
+
+}  // namespace
+
 PTB_EXPORT int ptb_gemm_swiglu_bf16(const void* a, const void* b, void* c, int64_t m, int64_t inter, int64_t k,
                                     void* stream) {
   if (m < 0 || inter < 0 || k < 0) return PTB_ERR_SHAPE;
@@ -896,14 +924,19 @@ PTB_EXPORT int ptb_gemm_swiglu_bf16(const void* a, const void* b, void* c, int64
       n > kMaxOutCols)
     return PTB_ERR_UNSUPPORTED;
   if (!aligned16(a) || !aligned16(b) || !aligned16(c)) return PTB_ERR_ALIGN;
-  const int64_t tm = (m + 255) / 256, tn = inter / 128;
-  if (tm * tn > 0x7fffffff) return PTB_ERR_GRID;
-  const Groups none{nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
-  gemm_bf16_kernel<4, 4, false, kSwiGLU, 64><<<dim3(unsigned(tm * tn)), dim3(kThreads), 0,
-                                                        static_cast<hipStream_t>(stream)>>>(
-      static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), nullptr, static_cast<uint16_t*>(c), int(m),
-      int(n), int(k), int(tm), int(tn), none, nullptr, 0);
-  return launch_status();
+  // The tiles of the [m, 2*inter] product by the plain GEMM's model, whose pick was within 0.2%
+  // (geometric mean) of the best tile over 100 (tokens, hidden, inter) points and 1.7x faster than
+  // 256x256 tiles throughout: 1 token of 4096 -> 12288 84 -> 46 us (96 workgroups of which one row is
+  // wanted -> 192 of 64x128), 200 tokens 84.5 -> 65 (192 of 256x128), 640 167 -> 130 (128x256), 1024
+  // 184 -> 171 (two even rounds of 256x192), 2048 unchanged.
+  const GemmPlan p = gemm_plan(m, n, k, false);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (p.wm == 4 && p.wn == 4) return launch_swiglu<4, 4>(a, b, c, m, n, k, s);
+  if (p.wm == 4 && p.wn == 3) return launch_swiglu<4, 3>(a, b, c, m, n, k, s);
+  if (p.wm == 4) return launch_swiglu<4, 2>(a, b, c, m, n, k, s);
+  if (p.wm == 2 && p.wn == 4) return launch_swiglu<2, 4>(a, b, c, m, n, k, s);
+  if (p.wm == 2) return launch_swiglu<2, 2>(a, b, c, m, n, k, s);
+  return launch_swiglu<1, 2>(a, b, c, m, n, k, s);
 }
 
 PTB_EXPORT int ptb_grouped_gemm_bf16(const void* a, const void* b, const int32_t* group, const int32_t* start,

@@ -298,6 +298,27 @@ def test_gemm_odd_step_count(m, k, n, resid):
     assert_close(got, want, RTOL, ATOL * rms(want), f"gemm {m}x{k}x{n}")
 
 
+@pytest.mark.parametrize("m,k,inter", [
+    (1, 64, 128),         # 64x128 tiles, one row, one step
+    (130, 320, 256),      # 64x128 tiles, five steps
+    (129, 320, 5504),     # 128x128 tiles, the second row tile one row
+    (1669, 320, 1280),    # 256x128 tiles
+    (515, 320, 5632),     # 128x256 tiles, the last row tile three rows
+    (2047, 448, 2176),    # 256x192 tiles (96 outputs each): the last one covers 64 of its 96
+    (2500, 192, 3200),    # 256x256 tiles
+])
+def test_gemm_swiglu_every_tile(m, k, inter):
+    """The SwiGLU epilogue of every tile shape of the plan, ragged in M and (256x192) in the outputs:
+    bit for bit the GEMM followed by silu_mul, and nothing past C."""
+    a = randn((m, k), 61, std=1 / 16).to(DEV)
+    b = randn((k, 2 * inter), 62, std=1 / 4).to(DEV)
+    guard = torch.full((m * inter + 8192,), float("nan"), dtype=torch.bfloat16, device=DEV)
+    c = guard[: m * inter].view(m, inter)
+    ops.gemm_swiglu(a, b, out=c)
+    assert bool(guard[m * inter:].isnan().all()), "the GEMM wrote past C"
+    assert bits_equal(c.cpu(), ops.silu_mul(ops.gemm(a, b, split_k=False)).cpu())
+
+
 def test_gemm_swiglu_odd_step_count():
     """The SwiGLU-fused GEMM with K = 1088 (17 steps of 64: a remainder of five) equals the GEMM +
     silu_mul pair."""
