@@ -330,7 +330,8 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
   const int qi = qw0 + fr;             // this lane's query
 
   // ---- K/V loaders: instruction t of this wave fills key rows 4*(kDmaT*wave + t) .. +3 of a tile;
-  //      lane L writes row L/16, slot L%16, so it fetches the chunk that belongs in that slot
+  //      lane L writes row L/16, slot L%16, so it fetches the chunk that belongs in that slot; the
+  //      wave's instructions fill consecutive KB, so they go out as a run (offsets less 1024 * t)
   const uint32_t kv_bytes = uint32_t(S) * D * 2u;
   const i32x4 rsrc_k = make_rsrc(kp, kv_bytes);
   const i32x4 rsrc_v = make_rsrc(vp, uint32_t((int64_t(S) - 1) * vrow * 2 + D * 2));
@@ -339,8 +340,8 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
   for (int t = 0; t < kDmaT; ++t) {
     const int key = 4 * (kDmaT * wave + t) + (lane >> 4);
     const int slot = lane & 15;
-    k_voff[t] = uint32_t(key * D + ((slot ^ (key & 15)) * 8)) * 2u;
-    v_voff[t] = uint32_t(int64_t(key) * vrow + ((slot ^ (4 * (key & 3))) * 8)) * 2u;
+    k_voff[t] = uint32_t(key * D + ((slot ^ (key & 15)) * 8)) * 2u - 1024u * t;
+    v_voff[t] = uint32_t(int64_t(key) * vrow + ((slot ^ (4 * (key & 3))) * 8)) * 2u - 1024u * t;
   }
   const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(smem));
   // par = kb & 1, a compile-time constant at every call, so stage addresses fold into the LDS
@@ -349,13 +350,8 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
     const uint32_t st = lds0 + uint32_t(decltype(par)::value) * kStageBytes;
     const uint32_t soff = uint32_t(kb) * uint32_t(kTileBytes);
     const uint32_t soff_v = uint32_t(int64_t(kb) * BKV * vrow * 2);
-#pragma unroll
-    for (int t = 0; t < kDmaT; ++t)
-      dma16(rsrc_k, __builtin_amdgcn_readfirstlane(st + (wave * kDmaT + t) * 1024), k_voff[t], soff);
-#pragma unroll
-    for (int t = 0; t < kDmaT; ++t)
-      dma16(rsrc_v, __builtin_amdgcn_readfirstlane(st + kTileBytes + (wave * kDmaT + t) * 1024), v_voff[t],
-            soff_v);
+    dma16_run(rsrc_k, __builtin_amdgcn_readfirstlane(st + wave * kDmaT * 1024), k_voff, soff);
+    dma16_run(rsrc_v, __builtin_amdgcn_readfirstlane(st + kTileBytes + wave * kDmaT * 1024), v_voff, soff_v);
   };
 
   // ---- fragment addressing

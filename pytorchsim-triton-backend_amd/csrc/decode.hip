@@ -823,14 +823,16 @@ __global__ __launch_bounds__(64) void attn_decode_mfma(const uint16_t* __restric
   // so it fetches the chunk that belongs in that slot.  K row r keeps chunk c in slot c ^ (r & 15)
   // (a fragment read's 16 lanes take 16 rows); V row r keeps chunk c in slot c ^ (4 * (r & 3)) (a
   // transposing read's 16 lanes take 4 rows x 4 chunks).
-  // Offsets stay in the VGPR operand (soffset 0), which the buffer range check covers.
-  uint32_t koff[8];
+  // A tile goes out as two runs of four instructions (their offsets less 1024 * (i % 4)).
+  // Offsets stay in the VGPR operand and the offset field (soffset 0), which the buffer range check
+  // covers.
+  uint32_t koff[2][4], voff[2][4];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int r = 4 * i + g4;
-    koff[i] = uint32_t(r * 256 + ((l16 ^ (r & 15)) << 4));
+    koff[i / 4][i % 4] = uint32_t(r * 256 + ((l16 ^ (r & 15)) << 4)) - 1024u * (i % 4);
+    voff[i / 4][i % 4] = uint32_t(r * 256 + ((l16 ^ (4 * g4)) << 4)) - 1024u * (i % 4);
   }
-  const uint32_t vdma = uint32_t(g4 * 256 + ((l16 ^ (4 * g4)) << 4));
   auto issue = [&](int s, auto par) __attribute__((always_inline)) {
     constexpr int P = decltype(par)::value;
     const int key0 = (range * steps + s) * kWKeys;
@@ -844,11 +846,9 @@ __global__ __launch_bounds__(64) void attn_decode_mfma(const uint16_t* __restric
     }
     const uint32_t st = lds0 + uint32_t(P * 2 * kWTile);
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      dma16(rk, __builtin_amdgcn_readfirstlane(st + i * 1024), koff[i], 0);
+    for (int i = 0; i < 2; ++i) dma16_run(rk, __builtin_amdgcn_readfirstlane(st + i * 4096), koff[i], 0);
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      dma16(rv, __builtin_amdgcn_readfirstlane(st + kWTile + i * 1024), vdma + i * 1024, 0);
+    for (int i = 0; i < 2; ++i) dma16_run(rv, __builtin_amdgcn_readfirstlane(st + kWTile + i * 4096), voff[i], 0);
   };
   issue(0, std::integral_constant<int, 0>{});
 

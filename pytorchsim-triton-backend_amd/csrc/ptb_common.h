@@ -220,9 +220,32 @@ __device__ __forceinline__ i32x4 make_rsrc(const void* base, uint32_t bytes) {
 // 16 bytes per lane from global (buffer resource, byte offsets voff + soff) straight into LDS at
 // lds_base + 16 * lane (buffer_load_dwordx4 ... lds, no VGPR staging); lds_base is wave-uniform.
 // The compiler does not see the LDS write: callers order it with wait_vmcnt + a barrier.
+// The s_nop is the wait state gfx9 needs between a scalar write of m0 and an LDS-bound load that reads
+// it (the compiler, which puts one there itself, cannot see into the asm block).
 __device__ __forceinline__ void dma16(i32x4 rsrc, uint32_t lds_base, uint32_t voff, uint32_t soff) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                :: "s"(lds_base), "v"(voff), "s"(rsrc), "s"(soff) : "memory", "m0");
+}
+
+// A run of N (2 or 4) such loads into consecutive KB of LDS: the i-th reads byte offset
+// voff[i] + 1024 * i + soff into lds_base + 1024 * i + 16 * lane.  The instruction's offset field
+// advances the global and the LDS address alike, so one m0 write and one wait state serve the run.
+template <int N>
+__device__ __forceinline__ void dma16_run(i32x4 rsrc, uint32_t lds_base, const uint32_t (&voff)[N], uint32_t soff) {
+  static_assert(N == 2 || N == 4, "runs of two or four");
+  if constexpr (N == 2)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
+                 "buffer_load_dwordx4 %1, %3, %4 offen lds\n\t"
+                 "buffer_load_dwordx4 %2, %3, %4 offen offset:1024 lds"
+                 :: "s"(lds_base), "v"(voff[0]), "v"(voff[1]), "s"(rsrc), "s"(soff) : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
+                 "buffer_load_dwordx4 %1, %5, %6 offen lds\n\t"
+                 "buffer_load_dwordx4 %2, %5, %6 offen offset:1024 lds\n\t"
+                 "buffer_load_dwordx4 %3, %5, %6 offen offset:2048 lds\n\t"
+                 "buffer_load_dwordx4 %4, %5, %6 offen offset:3072 lds"
+                 :: "s"(lds_base), "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(rsrc), "s"(soff)
+                 : "memory", "m0");
 }
 
 template <int N>
