@@ -158,9 +158,9 @@ int ptb_slice_add_bf16(const void* x, float* out, int64_t first, int64_t count, 
 int ptb_gemm_bf16(const void* a, const void* b, const void* residual, void* c, int64_t m, int64_t n,
                   int64_t k, void* stream);
 
-/* The same GEMM with a caller workspace for split-K: when the output's 64x128 tiles leave CUs idle
- * (and K >= 1024), K may be cut into 2, 4 or 8 slices (at least 256 deep, tiles x slices within the
- * CUs, as a fitted cost model of the workgroups' operand streaming and the partial traffic decides)
+/* The same GEMM with a caller workspace for split-K: where the plan's tiles would leave CUs idle (and
+ * K >= 1024), K may be cut into 2 to 8 slices (at least 128 deep, tiles x slices within the CUs, as a
+ * fitted cost model of the tiles' K steps, the operand traffic and the partials decides)
  * multiplied by separate workgroups into fp32 partials that a finish pass sums (+ residual) and
  * rounds once.  ptb_gemm_bf16_workspace_bytes is 0 for shapes that do not split; then
  * ptb_gemm_bf16_ws is ptb_gemm_bf16.  A split shape refuses a NULL workspace (PTB_ERR_NULL) or one
@@ -201,6 +201,14 @@ int ptb_quant_weight_e4m3(const float* w, void* wq_t, float* scale, int64_t k, i
 int ptb_gemm_fp8_scaled(const void* aq, const float* sa, const void* wq_t, const float* sw, void* c,
                         int64_t m, int64_t n, int64_t k, void* stream);
 
+/* The same GEMM with a caller workspace (16-byte aligned) for split-K: shapes whose tiles would leave
+ * CUs idle may cut K into 2 to 8 slices, multiplied by separate workgroups into fp32 partials that a
+ * finish pass sums, scales and rounds once.  ptb_gemm_fp8_workspace_bytes is 0 for shapes that do not
+ * split; then ptb_gemm_fp8_scaled_ws is ptb_gemm_fp8_scaled and takes a NULL workspace.  A split shape
+ * refuses a NULL workspace (PTB_ERR_NULL) or one shorter than that (PTB_ERR_WORKSPACE). */
+size_t ptb_gemm_fp8_workspace_bytes(int64_t m, int64_t n, int64_t k);
+int ptb_gemm_fp8_scaled_ws(const void* aq, const float* sa, const void* wq_t, const float* sw, void* c, int64_t m,
+                           int64_t n, int64_t k, void* workspace, size_t workspace_bytes, void* stream);
 
 /* Flash-attention forward, head-major layout: q/o [batch*hq, seq, head_dim], k/v [batch*hkv, seq,
  * head_dim]; q head h reads kv head h / (hq / hkv).  Online softmax in fp32 with P rounded to bf16

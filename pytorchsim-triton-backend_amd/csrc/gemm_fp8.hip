@@ -5,23 +5,28 @@
 //                  Wt[N,K] (K contiguous), which is how the GEMM streams it
 //   gemm_fp8     : C[m,n] = bf16( (sum_k Aq[m,k] * Wt[n,k]) * sa[m] * sw[n] ), fp32 accumulation
 //
-// The GEMM uses v_mfma_f32_32x32x64_f8f6f4 (both operands e4m3, no block scales): a 256xBN
-// workgroup tile (BN = 256, or 128 when 256x256 tiles would leave CUs idle), 4 waves in a 2x2
-// arrangement, each wave 128 x BN/2 as 32x32 accumulators.  Both operands are K-contiguous; a stage
+// The GEMM uses v_mfma_f32_32x32x64_f8f6f4 (both operands e4m3, no block scales): a BM x BN workgroup
+// tile (256x256, 256x128, 128x128 or 64x128, and the split of K, by the cost model of fp8_plan), 4
+// waves in a 2x2
+// arrangement, each wave BM/2 x BN/2 as 32x32 accumulators.  Both operands are K-contiguous; a stage
 // holds 128 bytes (= 128 K) of every tile row, so each row's DMA is one whole 128-byte line and the
 // L2 serves one request per line (a 64-byte stage row costs the L2 a request slot for half a line:
 // the request rate, not the bytes, bounded the 64-byte form).  Operands move HBM -> LDS with
-// buffer_load_dwordx4 ... lds into a ring of NS stages (3 x 48 KB at BN = 128, 2 x 64 KB at
-// BN = 256).  Within a row the eight 16-byte chunks sit XOR-swizzled by (row >> 1) & 7, so the
+// buffer_load_dwordx4 ... lds into a ring of NS stages (2 x 64 KB for 256x256, 3 x 48 KB for 256x128,
+// 4 x 32 KB and 4 x 24 KB for 128x128 and 64x128).  Within a row the eight 16-byte chunks sit XOR-swizzled by (row >> 1) & 7, so the
 // 128-bit fragment reads (16 lanes a phase, 16 different rows) are bank-conflict free.  A stage is
 // two MFMA K substeps of 64: substep 0's MFMAs run with substep 1's fragment reads folded in; the
 // barrier that follows publishes the next stage and frees this one; substep 1's MFMAs then run with
-// the reads of the next stage's substep 0.  The refill DMAs of a three-stage ring go into the slot
+// the reads of the next stage's substep 0.  The refill DMAs of a ring of three or more stages go into the slot
 // the previous step freed and spread over both substeps (bunched into one substep they queue in the
 // address unit and stall the MFMAs: config 4 85 -> 82 us); a two-stage ring refills the slot its
 // own barrier frees, during substep 1.  MFMAs take W as the first operand, so accumulators hold C^T blocks and each lane
 // stores 4 consecutive columns of a row of C at once.
+//
+// Up to 32 rows of A against a weight small enough that a second launch would show run gemm_fp8_rows
+// instead: no LDS staging, one launch, the waves of a workgroup splitting K.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "ptb_common.h"
@@ -30,41 +35,44 @@ using namespace ptb;
 
 namespace {
 
-constexpr int BM = 256, BK = 128;   // BK in bytes (= fp8 elements) per stage
+constexpr int BK = 128;   // bytes (= fp8 elements) of K per stage
 constexpr int kThreads = 256;
 
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
-template <int BN>
+template <int BM, int BN>
 struct Cfg {
-  static constexpr int NS = BN == 256 ? 2 : 3;         // LDS ring depth
-  static constexpr int WNT = BN / 64;                  // 32-wide column tiles per wave
-  static constexpr int kABytes = BM * BK;              // 32 KB
+  static constexpr int WMT = BM / 64, WNT = BN / 64;   // 32-row / 32-column blocks per wave
+  static constexpr int kABytes = BM * BK;
   static constexpr int kWBytes = BN * BK;
   static constexpr int kStageBytes = kABytes + kWBytes;
+  static constexpr int NS = BM == 256 ? (BN == 256 ? 2 : 3) : 4;   // LDS ring depth
   static constexpr int kDmaA = BM / 8 / 4;             // DMA instructions per wave per stage (8 rows each)
   static constexpr int kDmaW = BN / 8 / 4;
   static constexpr int kDma = kDmaA + kDmaW;
-  static constexpr int kPieces = 2 * (4 + WNT);        // 128-bit fragment reads per wave per substep
-  static constexpr int kMfma = 4 * WNT;                // MFMAs per wave per substep
+  static constexpr int kPieces = 2 * (WMT + WNT);      // 128-bit fragment reads per wave per substep
+  static constexpr int kMfma = WMT * WNT;              // MFMAs per wave per substep
+  static_assert(NS * kStageBytes <= 160 * 1024, "the ring fits the LDS");
 };
 
-template <int BN>
+template <int BM, int BN>
 struct Frags {
-  i32x8 a[4];
-  i32x8 w[Cfg<BN>::WNT];
-  u32x4 lo[4 + Cfg<BN>::WNT];
+  i32x8 a[Cfg<BM, BN>::WMT];
+  i32x8 w[Cfg<BM, BN>::WNT];
+  u32x4 lo[Cfg<BM, BN>::WMT + Cfg<BM, BN>::WNT];
 };
 
 __device__ __forceinline__ int fp8_swz(int row) { return (row >> 1) & 7; }
 
-template <int BN>
+// SPLIT: workgroup (tile, slice s) multiplies K columns [s*kchunk, s*kchunk + kchunk) and stores its
+// fp32 partial sums, unscaled, at part + s*M*N (fp8_finish sums, scales and rounds them).
+template <int BM, int BN, bool SPLIT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_fp8_kernel(
-    const uint8_t* __restrict__ A, const float* __restrict__ SA, const uint8_t* __restrict__ W,
+    const uint8_t* __restrict__ A_in, const float* __restrict__ SA, const uint8_t* __restrict__ W_in,
     const float* __restrict__ SW, uint16_t* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n,
-    int group_m) {
-  using G = Cfg<BN>;
-  constexpr int NS = G::NS;
+    int group_m, float* __restrict__ part, int kchunk) {
+  using G = Cfg<BM, BN>;
+  constexpr int NS = G::NS, WMT = G::WMT, WNT = G::WNT;
   // stage kt+DIST refills the slot of stage kt+DIST-NS: with a three-stage ring that is stage kt-1,
   // freed by step kt-1's barrier, so the stage's DMAs spread over both substeps of step kt; with
   // two stages, stage kt's own slot, freed only by step kt's barrier (the DMAs go in substep 1)
@@ -72,9 +80,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
   constexpr bool kSpread = DIST < NS;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[NS * G::kStageBytes];
 
+  // XCD x (ids x, x + 8, ...) takes consecutive positions; a split's slices follow one another
   const int ntiles = tiles_m * tiles_n;
-  int pid = blockIdx.x;
-  if ((ntiles & 7) == 0) pid = (pid & 7) * (ntiles >> 3) + (pid >> 3);
+  const int xcd = int(blockIdx.x) & 7;
+  int pid = xcd * int(gridDim.x >> 3) + min(xcd, int(gridDim.x & 7)) + int(blockIdx.x >> 3);
+  int koff = 0, Kl = K;   // the K columns of this workgroup: [koff, koff + Kl)
+  int slice = 0;
+  if constexpr (SPLIT) {
+    slice = pid / ntiles;
+    pid -= slice * ntiles;
+    koff = slice * kchunk;
+    Kl = min(kchunk, K - koff);
+  }
+  const uint8_t* A = A_in + koff;
+  const uint8_t* W = W_in + koff;
   const int width = group_m * tiles_n;
   const int first_m = (pid / width) * group_m;
   const int gsize = min(tiles_m - first_m, group_m);
@@ -88,14 +107,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
   // the tile's row scales: one load a thread, issued ahead of the prologue's DMAs and held in a
   // register until the epilogue puts it in LDS, so the epilogue waits on no global load per
   // 32-row block (and nothing waits on this load before then)
-  static_assert(BM == kThreads, "one row scale per thread");
-  __shared__ float sa_tile[BM];
-  const float sa_mine = SA[min(m0 + tid, M - 1)];
+  static_assert(BM <= kThreads, "at most one row scale per thread");
+  __shared__ float sa_tile[SPLIT ? 1 : BM];
+  const float sa_mine = SPLIT ? 0.f : SA[min(m0 + tid % BM, M - 1)];   // threads past BM repeat, unused
 
   // loaders: rows past M (A) or N (W) read as zero through num_records; stages past K read other
   // rows' bytes or zeros into slots nobody reads any more (the DMA stream runs ahead without a branch)
-  const i32x4 rsrc_a = make_rsrc(A + int64_t(m0) * K, uint32_t(min(BM, M - m0)) * uint32_t(K));
-  const i32x4 rsrc_w = make_rsrc(W + int64_t(n0) * K, uint32_t(min(BN, N - n0)) * uint32_t(K));
+  const i32x4 rsrc_a = make_rsrc(A + int64_t(m0) * K, uint32_t(min(BM, M - m0)) * uint32_t(K) - uint32_t(koff));
+  const i32x4 rsrc_w = make_rsrc(W + int64_t(n0) * K, uint32_t(min(BN, N - n0)) * uint32_t(K) - uint32_t(koff));
   // DMA instruction d of this wave covers rows 8*(kDma_op*wave + d) .. +8; lane -> row lane/8,
   // slot lane%8 holding chunk (lane%8) ^ swz(row)
   auto voff_of = [&](int row) { return uint32_t(row * K + (((lane & 7) ^ fp8_swz(row)) << 4)); };
@@ -118,31 +137,31 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
       dma16(rsrc_w, st + G::kABytes + wave_w + (d - G::kDmaA) * 1024, w_voff[d - G::kDmaA], soff);
   };
 
-  f32x16 acc[4][G::WNT];
+  f32x16 acc[WMT][WNT];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < WMT; ++i)
 #pragma unroll
-    for (int j = 0; j < G::WNT; ++j)
+    for (int j = 0; j < WNT; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
   // lane -> row (or column) lane % 32, K half (32 bytes = chunks 4ks + 2h, 4ks + 2h + 1) lane / 32
   const int fr = lane & 31, h = lane >> 5;
-  int row_off[4 + G::WNT], row_sw[4 + G::WNT];
+  int row_off[WMT + WNT], row_sw[WMT + WNT];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = wm * 128 + i * 32 + fr;
+  for (int i = 0; i < WMT; ++i) {
+    const int m = wm * (BM / 2) + i * 32 + fr;
     row_off[i] = m * BK;
     row_sw[i] = fp8_swz(m);
   }
 #pragma unroll
-  for (int j = 0; j < G::WNT; ++j) {
+  for (int j = 0; j < WNT; ++j) {
     const int n = wn * (BN / 2) + j * 32 + fr;
-    row_off[4 + j] = G::kABytes + n * BK;
-    row_sw[4 + j] = fp8_swz(n);
+    row_off[WMT + j] = G::kABytes + n * BK;
+    row_sw[WMT + j] = fp8_swz(n);
   }
   // piece p of substep ks: operand row t = p / 2, half c = p % 2 (chunk 4ks + 2h + c)
-  auto read_piece = [&](const uint8_t* st, int ks, int p, Frags<BN>& f) __attribute__((always_inline)) {
+  auto read_piece = [&](const uint8_t* st, int ks, int p, Frags<BM, BN>& f) __attribute__((always_inline)) {
     const int t = p >> 1, c = p & 1;
     const u32x4 v = *reinterpret_cast<const u32x4*>(st + row_off[t] + (((4 * ks + 2 * h + c) ^ row_sw[t]) << 4));
     if (c == 0) {
@@ -150,19 +169,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
     } else {
       const i32x8 x = i32x8{int(f.lo[t][0]), int(f.lo[t][1]), int(f.lo[t][2]), int(f.lo[t][3]),
                             int(v[0]), int(v[1]), int(v[2]), int(v[3])};
-      if (t < 4) f.a[t] = x;
-      else f.w[t - 4] = x;
+      if (t < WMT) f.a[t] = x;
+      else f.w[t - WMT] = x;
     }
   };
-  auto mfma_one = [&](const Frags<BN>& f, int u) __attribute__((always_inline)) {
-    const int i = u / G::WNT, j = u % G::WNT;
+  auto mfma_one = [&](const Frags<BM, BN>& f, int u) __attribute__((always_inline)) {
+    const int i = u / WNT, j = u % WNT;
     acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.w[j], f.a[i], acc[i][j], 0, 0, 0, 0, 0, 0);
   };
 
-  const int nk = K / BK;
+  const int nk = Kl / BK;
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, 1>;
   using S2 = std::integral_constant<int, 2 % NS>;
+  using S3 = std::integral_constant<int, 3 % NS>;
 #pragma unroll
   for (int d = 0; d < G::kDma; ++d) dma_one(0, d, S0{});
 #pragma unroll
@@ -173,15 +193,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
   }
   wait_vmcnt<(DIST - 1) * G::kDma>();   // stage 0 landed (this wave's part)
   __syncthreads();                    // ... and everyone's
-  Frags<BN> f0, f1;
+  Frags<BM, BN> f0, f1;
 #pragma unroll
   for (int p = 0; p < G::kPieces; ++p) read_piece(smem, 0, p, f0);
 
   // Reads are issued in the order the MFMAs first use the operands (MFMA u multiplies A row block
   // u / WNT by W column block u % WNT): A0, W0 .. W(WNT-1), A1, A2, A3, two 128-bit pieces each,
-  // two pieces per MFMA from the start of a substep, so the next substep's first MFMAs find their
-  // operands landed instead of waiting on the LDS.  The refill DMAs spread over the whole substep.
+  // two pieces per MFMA (PPM: as many as the small tiles need) from the start of a substep, so the
+  // next substep's first MFMAs find their operands landed instead of waiting on the LDS.  The refill
+  // DMAs spread over the whole substep.
   constexpr int U = G::kMfma, P = G::kPieces, D = G::kDma;
+  constexpr int PPM = P > 2 * U ? (P + U - 1) / U : 2;
   constexpr int NPRE = [] {   // DMAs of stage kt+DIST issued before step kt's barrier
     int n = 0;
     for (int o = 0; o < D; ++o)
@@ -190,7 +212,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
   }();
   auto piece_of = [](int q) constexpr {
     const int o = q >> 1;   // operand in first-use order
-    const int t = o == 0 ? 0 : (o <= G::WNT ? 4 + (o - 1) : o - G::WNT);
+    const int t = o == 0 ? 0 : (o <= WNT ? WMT + (o - 1) : o - WNT);
     return 2 * t + (q & 1);
   };
   auto step = [&](int kt, auto stg) __attribute__((always_inline)) {
@@ -203,7 +225,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
     for (int u = 0; u < U; ++u) {
       mfma_one(f0, u);
 #pragma unroll
-      for (int q = 2 * u; q < 2 * u + 2; ++q)
+      for (int q = PPM * u; q < PPM * u + PPM; ++q)
         if (q < P) read_piece(st, 1, piece_of(q), f1);
       if constexpr (kSpread) {
 #pragma unroll
@@ -222,7 +244,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
     for (int u = 0; u < U; ++u) {
       mfma_one(f1, u);
 #pragma unroll
-      for (int q = 2 * u; q < 2 * u + 2; ++q)
+      for (int q = PPM * u; q < PPM * u + PPM; ++q)
         if (q < P) read_piece(nst, 0, piece_of(q), f0);
 #pragma unroll
       for (int d = 0; d < D; ++d)
@@ -235,14 +257,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
     step(kt, S0{});
     step(kt + 1, S1{});
     if constexpr (NS > 2) step(kt + 2, S2{});
+    if constexpr (NS > 3) step(kt + 3, S3{});
   }
   if (kt < nk) step(kt, S0{});
   if constexpr (NS > 2) {
     if (kt + 1 < nk) step(kt + 1, S1{});
   }
+  if constexpr (NS > 3) {
+    if (kt + 2 < nk) step(kt + 2, S2{});
+  }
   wait_vmcnt<0>();
 
-  // accumulator (i, j, r) of lane holds C row m0 + wm*128 + i*32 + lane%32, columns
+  // accumulator (i, j, r) of lane holds C row m0 + wm*BM/2 + i*32 + lane%32, columns
   // n0 + wn*BN/2 + j*32 + 8*(r/4) + 4*(lane/32) + r%4.  Each value is scaled, (acc * sa) * sw, and
   // rounded to bf16 where it sits, then the tile leaves through the LDS, which is free once every
   // DMA has landed and, past the barrier, no wave reads a stage: a wave writes one 32-row block of
@@ -251,18 +277,51 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
   // into each of 32 rows).  The region is the wave's own and LDS operations of a wave complete in
   // order, so no barrier separates its writes from its reads.  Rows past M and columns past N fall
   // outside the output's buffer resource (stores dropped), so the stores need no branches.
-  sa_tile[tid] = sa_mine;
-  // the weight scales of this lane's accumulator columns: 4 consecutive ones per (j, g)
-  f32x4v swc[G::WNT][4];
+  if constexpr (SPLIT) {
+    // the slice's fp32 sums, staged the same way
+    __syncthreads();
+    constexpr int WCS = WNT * 32, kPitchS = WCS * 4 + 16, LPRS = WCS / 4, RPIS = 64 / LPRS;
+    static_assert(4 * 32 * kPitchS <= NS * G::kStageBytes, "the staging regions fit in the ring's LDS");
+    uint8_t* const st32 = smem + wave * (32 * kPitchS);
+    const int rls = lane / LPRS, cs = lane % LPRS;
+    const int col = n0 + wn * (BN / 2) + 4 * cs;
+    const __amdgpu_buffer_rsrc_t rsrc_p =
+        __builtin_amdgcn_make_buffer_rsrc(part + int64_t(slice) * M * N + int64_t(m0) * N, 0,
+                                          uint32_t(min(BM, M - m0)) * uint32_t(N) * 4u, 0x00020000);
 #pragma unroll
-  for (int j = 0; j < G::WNT; ++j)
+    for (int i = 0; i < WMT; ++i) {
+#pragma unroll
+      for (int j = 0; j < WNT; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<f32x4v*>(st32 + fr * kPitchS + (j * 32 + 8 * g + 4 * h) * 4) =
+              f32x4v{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+      u32x4 sv[32 / RPIS];
+#pragma unroll
+      for (int t = 0; t < 32 / RPIS; ++t)
+        sv[t] = *reinterpret_cast<const u32x4*>(st32 + (t * RPIS + rls) * kPitchS + cs * 16);
+      __builtin_amdgcn_sched_barrier(0);
+      const int r0 = wm * (BM / 2) + i * 32 + rls;
+#pragma unroll
+      for (int t = 0; t < 32 / RPIS; ++t) {
+        const uint32_t off = col < N ? (uint32_t(r0 + t * RPIS) * uint32_t(N) + uint32_t(col)) * 4u : 0x80000000u;
+        __builtin_amdgcn_raw_buffer_store_b128(sv[t], rsrc_p, off, 0, 0);
+      }
+    }
+    return;
+  }
+  if (tid < BM) sa_tile[tid] = sa_mine;
+  // the weight scales of this lane's accumulator columns: 4 consecutive ones per (j, g)
+  f32x4v swc[WNT][4];
+#pragma unroll
+  for (int j = 0; j < WNT; ++j)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const int c = n0 + wn * (BN / 2) + j * 32 + 8 * g + 4 * h;
       swc[j][g] = *reinterpret_cast<const f32x4v*>(SW + (c < N ? c : 0));
     }
   __syncthreads();
-  constexpr int WC = G::WNT * 32;       // columns of a wave's block
+  constexpr int WC = WNT * 32;       // columns of a wave's block
   constexpr int kPitch = WC * 2 + 16;   // bytes per staged bf16 row: rows start 4 banks apart
   constexpr int LPR = WC / 4;           // lanes per row, 4 columns each
   constexpr int RPI = 64 / LPR;         // rows per instruction
@@ -273,11 +332,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
   const __amdgpu_buffer_rsrc_t rsrc_c = __builtin_amdgcn_make_buffer_rsrc(
       C + int64_t(m0) * N, 0, uint32_t(min(BM, M - m0)) * uint32_t(N) * 2u, 0x00020000);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r0 = wm * 128 + i * 32 + rl;   // tile row of this lane's first stored row
-    const float sa = sa_tile[wm * 128 + i * 32 + fr];
+  for (int i = 0; i < WMT; ++i) {
+    const int r0 = wm * (BM / 2) + i * 32 + rl;   // tile row of this lane's first stored row
+    const float sa = sa_tile[wm * (BM / 2) + i * 32 + fr];
 #pragma unroll
-    for (int j = 0; j < G::WNT; ++j)
+    for (int j = 0; j < WNT; ++j)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const f32x4v w4 = swc[j][g];
@@ -297,6 +356,109 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
       __builtin_amdgcn_raw_buffer_store_b64(v[t], rsrc_c, off, 0, 0);
     }
   }
+}
+
+// ---- few rows
+// M <= 16 MB rows of A against 16 columns (rows of Wt) a workgroup: kRowWaves waves take every
+// kRowWaves-th 128-wide K step, each lane holding 32 bytes of one row of Wt (lane % 16) and of MB rows of
+// A per step straight from global memory (16 + 16 bytes 64 apart: the K order within a step is the same
+// for both operands, so it does not matter to the dot product), UN steps' loads issued before the first
+// MFMA.  The waves' sums meet in LDS in wave order.  Bound by the stream of W and, at 16 rows, by A from
+// L2 beside it (each workgroup reads all of A): 16x4096x4096 29.7 -> 6.7 us (5.7 at one row), 16x512x512
+// 7.1 -> 2.8 us against the 256x128 tiles that ran before; W is read once a call (streaming policy).
+// Waves with contiguous K ranges, or a K start rotated by workgroup, measured the same.
+constexpr int kRowWaves = 8;
+template <int MB>
+__global__ __launch_bounds__(64 * kRowWaves) void gemm_fp8_rows(const uint8_t* __restrict__ A,
+                                                                const float* __restrict__ SA,
+                                                                const uint8_t* __restrict__ W,
+                                                                const float* __restrict__ SW,
+                                                                uint16_t* __restrict__ C, int M, int N, int K) {
+  constexpr int UN = MB == 1 ? 6 : 4;
+  __shared__ float red[kRowWaves][MB * 256];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int n0 = blockIdx.x * 16;   // N % 16 == 0
+  const int r = lane & 15, g = lane >> 4;
+  const uint8_t* const wp = W + int64_t(n0 + r) * K + 16 * g;
+  const uint8_t* ap[MB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i) ap[i] = A + int64_t(min(16 * i + r, M - 1)) * K + 16 * g;   // rows past M repeat, unused
+  auto join = [](const u32x4& a, const u32x4& b) __attribute__((always_inline)) {
+    return i32x8{int(a[0]), int(a[1]), int(a[2]), int(a[3]), int(b[0]), int(b[1]), int(b[2]), int(b[3])};
+  };
+  auto load_w = [&](int k) __attribute__((always_inline)) {
+    const u32x4* p = reinterpret_cast<const u32x4*>(wp + k * BK);
+    return join(__builtin_nontemporal_load(p), __builtin_nontemporal_load(p + 4));
+  };
+  auto load_a = [&](int i, int k) __attribute__((always_inline)) {
+    const u32x4* p = reinterpret_cast<const u32x4*>(ap[i] + k * BK);
+    return join(p[0], p[4]);
+  };
+  f32x4 acc[MB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int nk = K / BK;
+  int k = wave;
+  for (; k + (UN - 1) * kRowWaves < nk; k += UN * kRowWaves) {
+    i32x8 w[UN], x[UN][MB];
+#pragma unroll
+    for (int u = 0; u < UN; ++u) w[u] = load_w(k + u * kRowWaves);
+#pragma unroll
+    for (int u = 0; u < UN; ++u)
+#pragma unroll
+      for (int i = 0; i < MB; ++i) x[u][i] = load_a(i, k + u * kRowWaves);
+    __builtin_amdgcn_sched_barrier(0);   // every load out before the first MFMA waits
+#pragma unroll
+    for (int u = 0; u < UN; ++u)
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+        acc[i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w[u], x[u][i], acc[i], 0, 0, 0, 0, 0, 0);
+  }
+  for (; k < nk; k += kRowWaves) {
+    const i32x8 w = load_w(k);
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+      acc[i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w, load_a(i, k), acc[i], 0, 0, 0, 0, 0, 0);
+  }
+  // W is the first operand: the lane holds row 16 i + r of A, columns n0 + 4 g .. + 3
+#pragma unroll
+  for (int i = 0; i < MB; ++i) *reinterpret_cast<f32x4*>(&red[wave][(16 * i + r) * 16 + 4 * g]) = acc[i];
+  __syncthreads();
+  if (tid < MB * 128) {   // two columns a thread
+    const int m = tid >> 3, c = 2 * (tid & 7);
+    float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+    for (int v = 0; v < kRowWaves; ++v) {
+      s0 += red[v][m * 16 + c];
+      s1 += red[v][m * 16 + c + 1];
+    }
+    if (m < M) {
+      const float sa = SA[m];
+      *reinterpret_cast<uint32_t*>(C + int64_t(m) * N + n0 + c) =
+          pack_bf16x2((s0 * sa) * SW[n0 + c], (s1 * sa) * SW[n0 + c + 1]);
+    }
+  }
+}
+
+// C = bf16((sum_s P[s] * sa) * sw), 4 columns a thread, the slices in order; all S loads go out before
+// the first add.
+template <int S>
+__global__ __launch_bounds__(256) void fp8_finish(const float* __restrict__ P, int mn, int N,
+                                                  const float* __restrict__ SA, const float* __restrict__ SW,
+                                                  uint16_t* __restrict__ C) {
+  const int q = (int(blockIdx.x) * 256 + int(threadIdx.x)) * 4;
+  if (q >= mn) return;
+  f32x4v v[S];
+#pragma unroll
+  for (int u = 0; u < S; ++u) v[u] = *reinterpret_cast<const f32x4v*>(P + int64_t(u) * mn + q);
+  const int m = q / N;
+  const float sa = SA[m];
+  const f32x4v sw = *reinterpret_cast<const f32x4v*>(SW + (q - m * N));   // N % 16 == 0: one row of C
+  f32x4v acc = v[0];
+#pragma unroll
+  for (int u = 1; u < S; ++u) acc = acc + v[u];
+  *reinterpret_cast<u32x2*>(C + q) = u32x2{pack_bf16x2((acc.x * sa) * sw.x, (acc.y * sa) * sw.y),
+                                           pack_bf16x2((acc.z * sa) * sw.z, (acc.w * sa) * sw.w)};
 }
 
 // ---- per-row activation quantiser
@@ -643,7 +805,7 @@ int fp8_check(const void* aq, const float* sa, const void* wq_t, const float* sw
   if (k == 0) return PTB_ERR_UNSUPPORTED;
   if (m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff) return PTB_ERR_SHAPE;
   if (k % 128 || n % 16) return PTB_ERR_UNSUPPORTED;
-  if (int64_t(BM) * k >= (int64_t(1) << 32)) return PTB_ERR_UNSUPPORTED;  // 32-bit buffer offsets
+  if (int64_t(256) * k >= (int64_t(1) << 32)) return PTB_ERR_UNSUPPORTED;  // 32-bit buffer offsets
   // a 256-row tile of C within 2^31 bytes: the epilogue's 32-bit store offsets, and the 0x80000000
   // that marks a column outside C, stay in range
   if (n > (int64_t(1) << 22)) return PTB_ERR_UNSUPPORTED;
@@ -652,33 +814,152 @@ int fp8_check(const void* aq, const float* sa, const void* wq_t, const float* sw
   return 1;   // go on
 }
 
+// Tile (rows 0: gemm_fp8_rows) and K split of an fp8 GEMM.
+struct Fp8Plan {
+  int bm, bn, splits;
+  int64_t kchunk;   // K columns per split
+};
+
+// Cost model of a plan, in us, of the form of the bf16 GEMM's: a round of workgroups (one a CU) costs
+// `step` per 128-deep K step plus `load` x (share of the CUs busy) and `fixed`; memory traffic overlaps
+// it (root sum of squares); a split adds its finish launch and fp32 partials.  gemm_fp8_rows costs its
+// launch, then the larger of W's stream (slower the more rows of A come from L2 beside it) and the
+// serial steps of a wave.  Fitted to 1777 (shape, plan) times on MI355X over 230 shapes (M 1 .. 8192, K
+// 128 .. 12288, N 128 .. 12288): 4.9% rms error, the picks within 1.1% (geometric mean) of each shape's
+// best measured plan and 2.1x faster than 256x256 / 256x128 tiles in one pass throughout:
+// 16x12288x4096 80 -> 14.5 us, 64x4096x4096 30 -> 11, 300x4096x4096 30 -> 15.5, 700x12288x4096 80 -> 51,
+// 2048x512x512 7.5 -> 5.  128x256 tiles were never the best by more than 3%.
+struct Fp8Tile {
+  int bm, bn;
+  double step, load, fixed;
+};
+constexpr Fp8Tile kFp8Tiles[] = {
+    {256, 256, 1.078, 0.256, 6.32}, {256, 128, 0.554, 0.300, 4.09}, {128, 128, 0.312, 0.187, 2.69}, {64, 128, 0.267, 0.141, 1.64}};
+constexpr double kMemUs = 3.24, kMemUsPerMB = 0.137, kFinishUs = 1.57, kPartialUsPerMB = 0.165;
+constexpr double kRowsUs = 1.62, kRowsStepUs = 0.785, kRowsUsPerMB = 0.224, kRowsUsPerMBRow = 0.0046, kRowsBlockUs = 0.225;
+constexpr int kMaxSplits = 8;
+
+// Splits stay in one round of workgroups, in slices of at least a 128-deep step of a K of at least 512.
+// 64x128 tiles stay in one round too: past it the larger tiles' fewer bytes per flop decide, and the
+// model, which does not see L2 misses, was up to 6% wrong there.
+Fp8Plan fp8_plan(int64_t m, int64_t n, int64_t k, bool may_split) {
+  const int64_t cus = device_cus();
+  const double mb = 1e-6 * double(k) * double(n);
+  const double mem = kMemUs + kMemUsPerMB * (mb + 1e-6 * double(m) * (double(k) + 2.0 * double(n)));
+  const double partial = kPartialUsPerMB * 8e-6 * double(m) * double(n);
+  Fp8Plan best{256, 128, 1, k};
+  double best_t = -1.0;
+  if (m <= 32) {
+    const double stream = mb * (kRowsUsPerMB + kRowsUsPerMBRow * double(m));
+    const double chain = kRowsStepUs * double((k / BK + kRowWaves - 1) / kRowWaves);
+    best_t = kRowsUs + std::sqrt(stream * stream + chain * chain) + kRowsBlockUs * double((m + 15) / 16);
+    best = Fp8Plan{0, 16, 1, k};
+  }
+  for (const Fp8Tile& c : kFp8Tiles) {
+    const int64_t t = ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn);
+    if (c.bm == 64 && t > cus) continue;
+    for (int sp = 1; sp <= (may_split && k >= 512 ? kMaxSplits : 1); ++sp) {
+      if (sp > 1 && (t * sp > cus || k / sp < BK)) break;
+      const int64_t kc = sp == 1 ? k : ((k + sp - 1) / sp + BK - 1) / BK * BK;
+      const int64_t splits = (k + kc - 1) / kc, w = t * splits, full = (w - 1) / cus;
+      const double steps = double(kc / BK), last = double(w - full * cus) / double(cus);
+      const double body = double(full) * (steps * (c.step + c.load) + c.fixed) + steps * (c.step + c.load * last) + c.fixed;
+      double us = std::sqrt(body * body + mem * mem);
+      if (splits > 1) us += kFinishUs + partial * double(splits);
+      if (best_t < 0.0 || us < best_t) {
+        best_t = us;
+        best = Fp8Plan{c.bm, c.bn, int(splits), kc};
+      }
+    }
+  }
+  return best;
+}
+
+size_t fp8_workspace(const Fp8Plan& p, int64_t m, int64_t n) {
+  return p.splits < 2 ? 0 : size_t(p.splits) * size_t(m) * size_t(n) * sizeof(float);
+}
+
+struct Fp8Args {
+  const uint8_t* a;
+  const float* sa;
+  const uint8_t* w;
+  const float* sw;
+  uint16_t* c;
+  int64_t m, n, k;
+};
+
+template <int BM, int BN>
+int launch_fp8(const Fp8Plan& p, const Fp8Args& g, float* part, hipStream_t s) {
+  const int64_t tm = (g.m + BM - 1) / BM, tn = (g.n + BN - 1) / BN;
+  if (tm * tn > 0x7fffffff) return PTB_ERR_GRID;
+  // Tile order: each XCD takes consecutive positions, walked in groups of group_m tile-rows.  At
+  // 256x128 tiles a group of 4 rows makes an XCD's 32 resident tiles a 4x8 block, whose A and W panels
+  // (4 x 256 rows + 8 x 128 rows of K) are the fewest bytes its L2 must fetch; 256x256 tiles take 8.
+  const int group_m = BN == 256 ? 8 : 4;
+  const dim3 block(kThreads);
+  if (p.splits < 2) {
+    gemm_fp8_kernel<BM, BN, false><<<dim3(unsigned(tm * tn)), block, 0, s>>>(
+        g.a, g.sa, g.w, g.sw, g.c, int(g.m), int(g.n), int(g.k), int(tm), int(tn), group_m, nullptr, 0);
+    return launch_status();
+  }
+  gemm_fp8_kernel<BM, BN, true><<<dim3(unsigned(tm * tn * p.splits)), block, 0, s>>>(
+      g.a, g.sa, g.w, g.sw, nullptr, int(g.m), int(g.n), int(g.k), int(tm), int(tn), group_m, part, int(p.kchunk));
+  const int mn = int(g.m * g.n), n = int(g.n);   // at most a tile a CU: within 32 bits
+  const dim3 grid(unsigned((mn / 4 + 255) / 256));
+  static_assert(kMaxSplits == 8, "a finish kernel for every split count");
+  switch (p.splits) {
+    case 2: fp8_finish<2><<<grid, 256, 0, s>>>(part, mn, n, g.sa, g.sw, g.c); break;
+    case 3: fp8_finish<3><<<grid, 256, 0, s>>>(part, mn, n, g.sa, g.sw, g.c); break;
+    case 4: fp8_finish<4><<<grid, 256, 0, s>>>(part, mn, n, g.sa, g.sw, g.c); break;
+    case 5: fp8_finish<5><<<grid, 256, 0, s>>>(part, mn, n, g.sa, g.sw, g.c); break;
+    case 6: fp8_finish<6><<<grid, 256, 0, s>>>(part, mn, n, g.sa, g.sw, g.c); break;
+    case 7: fp8_finish<7><<<grid, 256, 0, s>>>(part, mn, n, g.sa, g.sw, g.c); break;
+    default: fp8_finish<8><<<grid, 256, 0, s>>>(part, mn, n, g.sa, g.sw, g.c); break;
+  }
+  return launch_status();
+}
+
+int launch_fp8_plan(const Fp8Plan& p, const Fp8Args& g, float* part, hipStream_t s) {
+  if (p.bm == 0) {
+    const dim3 grid(unsigned(g.n / 16)), block(64 * kRowWaves);
+    if (g.m <= 16) gemm_fp8_rows<1><<<grid, block, 0, s>>>(g.a, g.sa, g.w, g.sw, g.c, int(g.m), int(g.n), int(g.k));
+    else gemm_fp8_rows<2><<<grid, block, 0, s>>>(g.a, g.sa, g.w, g.sw, g.c, int(g.m), int(g.n), int(g.k));
+    return launch_status();
+  }
+  if (p.bm == 256 && p.bn == 256) return launch_fp8<256, 256>(p, g, part, s);
+  if (p.bm == 256) return launch_fp8<256, 128>(p, g, part, s);
+  if (p.bm == 128) return launch_fp8<128, 128>(p, g, part, s);
+  return launch_fp8<64, 128>(p, g, part, s);
+}
+
 }  // namespace
 
 PTB_EXPORT int ptb_gemm_fp8_scaled(const void* aq, const float* sa, const void* wq_t, const float* sw, void* c,
                                    int64_t m, int64_t n, int64_t k, void* stream) {
   const int st = fp8_check(aq, sa, wq_t, sw, c, m, n, k);
   if (st <= 0) return st;
-  // 256x256 tiles unless that leaves CUs idle, then 256x128
-  const int64_t tm = (m + BM - 1) / BM;
-  const bool wide = tm * ((n + 255) / 256) >= device_cus();
-  const int bn = wide ? 256 : 128;
-  const int64_t tn = (n + bn - 1) / bn;
-  if (tm * tn > 0x7fffffff) return PTB_ERR_GRID;
-  const dim3 grid(unsigned(tm * tn)), block(kThreads);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const uint8_t* a8 = static_cast<const uint8_t*>(aq);
-  const uint8_t* w8 = static_cast<const uint8_t*>(wq_t);
-  uint16_t* c16 = static_cast<uint16_t*>(c);
-  // Tile order: ids are spread so that each XCD takes a contiguous range of tiles, walked in groups
-  // of group_m tile-rows.  At 256x128 tiles a group of 4 rows makes an XCD's 32 resident tiles a 4x8
-  // block, whose A and W panels (4 x 256 rows + 8 x 128 rows of K) are the fewest bytes its L2 must
-  // fetch; 256x256 tiles keep groups of 8.
-  const int group_m = wide ? 8 : 4;
-  if (wide)
-    gemm_fp8_kernel<256><<<grid, block, 0, s>>>(a8, sa, w8, sw, c16, int(m), int(n), int(k), int(tm), int(tn),
-                                                group_m);
-  else
-    gemm_fp8_kernel<128><<<grid, block, 0, s>>>(a8, sa, w8, sw, c16, int(m), int(n), int(k), int(tm), int(tn),
-                                                group_m);
-  return launch_status();
+  const Fp8Args g{static_cast<const uint8_t*>(aq), sa, static_cast<const uint8_t*>(wq_t), sw,
+                  static_cast<uint16_t*>(c), m, n, k};
+  return launch_fp8_plan(fp8_plan(m, n, k, false), g, nullptr, static_cast<hipStream_t>(stream));
+}
+
+PTB_EXPORT size_t ptb_gemm_fp8_workspace_bytes(int64_t m, int64_t n, int64_t k) {
+  if (m <= 0 || n <= 0 || k <= 0 || m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff) return 0;
+  return fp8_workspace(fp8_plan(m, n, k, true), m, n);
+}
+
+PTB_EXPORT int ptb_gemm_fp8_scaled_ws(const void* aq, const float* sa, const void* wq_t, const float* sw, void* c,
+                                      int64_t m, int64_t n, int64_t k, void* workspace, size_t workspace_bytes,
+                                      void* stream) {
+  const int st = fp8_check(aq, sa, wq_t, sw, c, m, n, k);
+  if (st <= 0) return st;
+  const Fp8Plan p = fp8_plan(m, n, k, true);
+  if (p.splits > 1) {
+    if (!workspace) return PTB_ERR_NULL;
+    if (workspace_bytes < fp8_workspace(p, m, n)) return PTB_ERR_WORKSPACE;
+    if (!aligned16(workspace)) return PTB_ERR_ALIGN;
+  }
+  const Fp8Args g{static_cast<const uint8_t*>(aq), sa, static_cast<const uint8_t*>(wq_t), sw,
+                  static_cast<uint16_t*>(c), m, n, k};
+  return launch_fp8_plan(p, g, static_cast<float*>(workspace), static_cast<hipStream_t>(stream));
 }

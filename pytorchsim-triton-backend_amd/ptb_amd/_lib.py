@@ -113,6 +113,8 @@ SIGNATURES = {
     "ptb_quant_rows_e4m3": (_c_int, [_vp, _vp, _vp, _c_i64, _c_i64, _vp]),
     "ptb_quant_weight_e4m3": (_c_int, [_vp, _vp, _vp, _c_i64, _c_i64, _vp]),
     "ptb_gemm_fp8_scaled": (_c_int, [_vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _vp]),
+    "ptb_gemm_fp8_workspace_bytes": (_c_size, [_c_i64, _c_i64, _c_i64]),
+    "ptb_gemm_fp8_scaled_ws": (_c_int, [_vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _vp, _c_size, _vp]),
     "ptb_rmsnorm_f32": (_c_int, [_vp, _vp, _vp, _c_i64, _c_i64, _c_f32, _vp]),
     "ptb_col_rms_f32": (_c_int, [_vp, _vp, _c_i64, _c_i64, _c_f32, _vp]),
     "ptb_softmax_rows_f32": (_c_int, [_vp, _vp, _c_i64, _c_i64, _vp]),

@@ -273,8 +273,10 @@ def gemm_fp8(aq: torch.Tensor, sa: torch.Tensor, wq_t: torch.Tensor, sw: torch.T
     if k != k2 or sa.numel() != m or sw.numel() != n:
         raise ValueError("shapes: aq [M,K], sa [M], wq_t [N,K], sw [N]")
     c = _out(out, (m, n), BF16, aq)
-    _lib.call("ptb_gemm_fp8_scaled", aq.data_ptr(), sa.data_ptr(), wq_t.data_ptr(), sw.data_ptr(), c.data_ptr(),
-              m, n, k, _stream(aq))
+    need = _lib.load().ptb_gemm_fp8_workspace_bytes(m, n, k)   # 0 unless the plan splits K
+    ws = torch.empty(need, dtype=torch.uint8, device=aq.device) if need else None
+    _lib.call("ptb_gemm_fp8_scaled_ws", aq.data_ptr(), sa.data_ptr(), wq_t.data_ptr(), sw.data_ptr(), c.data_ptr(),
+              m, n, k, None if ws is None else ws.data_ptr(), need, _stream(aq))
     return c
 
 

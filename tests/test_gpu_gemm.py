@@ -203,6 +203,63 @@ def test_gemm_fp8(m, k, n):
     assert_close(c[rows], want, RTOL, ATOL * scale, f"gemm_fp8 {m}x{k}x{n}")
 
 
+@pytest.mark.parametrize("m,k,n", [
+    (1, 128, 16),        # few rows: one step, seven waves idle
+    (16, 1024, 528),     # a step a wave
+    (7, 7296, 112),      # 57 steps: a whole batch of 6 a wave, then 9 more steps
+    (17, 4480, 80),      # two blocks of 16 rows, 35 steps
+    (32, 256, 848),
+    (33, 128, 64),       # 64x128 tiles, one step: three stages past K
+    (205, 384, 224),     # three steps, ragged in M and N
+    (419, 640, 32),      # five steps of the four-step loop
+    (40, 4224, 16),      # split 7 ways, one ragged tile
+    (67, 2176, 2368),    # split 3 ways, the last slice a step shorter
+    (398, 128, 4640),    # 128x128 tiles
+    (601, 384, 3488),
+    (463, 5120, 2112),   # 128x128 tiles split
+    (1026, 512, 3632),   # 256x128 tiles, an odd tile count for the XCDs
+    (397, 11008, 4112),  # 256x128 tiles split
+    (644, 8704, 5392),   # 256x256 tiles split
+    (1747, 1664, 4640),  # 256x256 tiles
+])
+def test_gemm_fp8_planned_tiles_stay_inside_c(m, k, n):
+    """Every tile shape and split of the fp8 plan and the few-row kernel at ragged sizes and around
+    their loops' step counts: small integers (exact in e4m3) and powers of two as scales make every sum
+    exact in fp32 (|sum| <= 9 * 12288 < 2^24), so the result is the oracle's bit for bit; a NaN-filled
+    guard after C's last element stays NaN."""
+    g = torch.Generator().manual_seed(m + n)
+    a = torch.randint(-3, 4, (m, k), generator=g).float().to(torch.float8_e4m3fn)
+    w = torch.randint(-3, 4, (n, k), generator=g).float().to(torch.float8_e4m3fn)
+    sa = 2.0 ** torch.randint(-3, 4, (m,), generator=g).float()
+    sw = 2.0 ** torch.randint(-6, 2, (n,), generator=g).float()
+    guard = torch.full((m * n + 8192,), float("nan"), dtype=torch.bfloat16, device=DEV)
+    c = guard[: m * n].view(m, n)
+    ops.gemm_fp8(a.to(DEV), sa.to(DEV), w.to(DEV), sw.to(DEV), out=c)
+    assert bool(guard[m * n:].isnan().all()), "the GEMM wrote past C"
+    rows = torch.arange(m) if m * k * n < 2e9 else sample_rows(m, 6)
+    assert bits_equal(c.cpu()[rows], oracle.gemm_fp8(a[rows], sa[rows], w, sw))
+
+
+def test_gemm_fp8_workspace_is_checked():
+    """A split shape refuses a missing, short or misaligned workspace; the entry without one takes it."""
+    m, k, n = 67, 2176, 2368
+    lib = _lib.load()
+    need = lib.ptb_gemm_fp8_workspace_bytes(m, n, k)
+    assert need > 0 and lib.ptb_gemm_fp8_workspace_bytes(2048, 4096, 12288) == 0
+    a = torch.ones((m, k), device=DEV).to(torch.float8_e4m3fn)
+    w = torch.ones((n, k), device=DEV).to(torch.float8_e4m3fn)
+    sa, sw = torch.ones(m, device=DEV), torch.ones(n, device=DEV)
+    c = torch.empty((m, n), dtype=torch.bfloat16, device=DEV)
+    ws = torch.empty(need + 16, dtype=torch.uint8, device=DEV)
+    s = torch.cuda.current_stream().cuda_stream
+    args = (a.data_ptr(), sa.data_ptr(), w.data_ptr(), sw.data_ptr(), c.data_ptr(), m, n, k)
+    assert lib.ptb_gemm_fp8_scaled_ws(*args, None, 0, s) == _lib.PTB_ERR_NULL
+    assert lib.ptb_gemm_fp8_scaled_ws(*args, ws.data_ptr(), need - 1, s) == _lib.PTB_ERR_WORKSPACE
+    assert lib.ptb_gemm_fp8_scaled_ws(*args, ws.data_ptr() + 4, need, s) == _lib.PTB_ERR_ALIGN
+    assert lib.ptb_gemm_fp8_scaled(*args, s) == _lib.PTB_OK
+    assert bool((c == k).all())
+
+
 @pytest.mark.parametrize("m,k,n,resid", [
     (128, 2048, 128, False), (8, 2048, 768, False), (512, 2048, 128, True), (32, 3072, 768, False),
     (1000, 4096, 264, True), (64, 1024, 2048, False), (256, 12288, 512, True),
