@@ -740,8 +740,10 @@ struct TileCost {
   int wm, wn;
   double step, load, fixed;
 };
-constexpr TileCost kTiles[] = {{4, 4, 0.816, 0.464, 6.29}, {4, 3, 0.620, 0.511, 5.89}, {4, 2, 0.555, 0.203, 3.72},
+constexpr TileCost kTiles[] = {{4, 4, 0.830, 0.500, 6.29}, {4, 3, 0.620, 0.511, 5.89}, {4, 2, 0.555, 0.203, 3.72},
                                {2, 4, 0.592, 0.250, 3.92}, {2, 2, 0.358, 0.196, 2.42}, {1, 2, 0.296, 0.141, 1.68}};
+// (256x256's step and load a little above the fit's 0.816 and 0.464: at 1664x12288x4096 the fit took two
+// slices of 256x256 tiles, 1.4% of the layer slower than one pass of 256x128 ones)
 constexpr double kMemUs = 3.3, kMemUsPerMB = 0.106, kFinishUs = 1.9, kPartialUsPerMB = 0.148;
 constexpr int kMaxSplits = 8;
 constexpr int64_t kFitK = 16384;   // past it (the fit ends at 12288) splits keep to the narrow rule below

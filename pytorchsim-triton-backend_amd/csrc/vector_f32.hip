@@ -4,6 +4,9 @@
 // hold inputs and outputs in fp32 with tolerances down to rtol 1e-5: nothing is rounded below fp32.
 // Rows move as 128-bit chunks of 4 floats with coalesced loads and stores; reductions are wave DPP /
 // permlane steps plus one LDS pass across waves.
+#include <algorithm>
+#include <type_traits>
+
 #include "ptb_common.h"
 
 using namespace ptb;
@@ -185,65 +188,178 @@ __global__ __launch_bounds__(kBlock) void silu_mul_f32(const float* __restrict__
 }
 
 // ---------------------------------------------------------------- SwiGLU block
-// o = silu(x @ wg) * (x @ wu) for fp32 x [M, K], wg / wu [K, N]: 64x64 output tiles, 256 threads each
-// owning a 4x4 block of both products, K in steps of 16 through LDS.  fp32 FMA (the operands are
-// fp32; the reference case checks at rtol 1e-3).
-constexpr int kSwT = 64, kSwK = 16;
-__global__ __launch_bounds__(kBlock) void swiglu_f32(const float* __restrict__ x, const float* __restrict__ wg,
-                                                     const float* __restrict__ wu, float* __restrict__ o, int M,
-                                                     int N, int K) {
-  __shared__ float xs[kSwK][kSwT + 4];
-  __shared__ float gs[kSwK][kSwT];
-  __shared__ float us[kSwK][kSwT];
-  const int m0 = blockIdx.y * kSwT, n0 = blockIdx.x * kSwT;
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  float ag[4][4] = {}, au[4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += kSwK) {
-    // x tile [64 rows][16 k] stored k-major; wg/wu tiles [16 k][64 n]
-    for (int e = threadIdx.x; e < kSwT * kSwK; e += kBlock) {
-      const int r = e / kSwK, kk = e % kSwK;
-      const int gm = m0 + r, gk = k0 + kk;
-      xs[kk][r] = (gm < M && gk < K) ? x[int64_t(gm) * K + gk] : 0.f;
-      const int kr = e / kSwT, nn = e % kSwT;
-      const int gk2 = k0 + kr, gn = n0 + nn;
-      const bool ok = gk2 < K && gn < N;
-      gs[kr][nn] = ok ? wg[int64_t(gk2) * N + gn] : 0.f;
-      us[kr][nn] = ok ? wu[int64_t(gk2) * N + gn] : 0.f;
-    }
-    __syncthreads();
+// o = silu(x @ wg) * (x @ wu) for fp32 x [M, K], wg / wu [K, N] on v_mfma_f32_32x32x2_f32 (fp32 operands
+// and accumulation): a wave owns a 32x32 block of both products, WR waves tile a workgroup's 32 WR
+// rows x 32 columns and WK waves split each K slab of WK * KW columns.  Slabs pass through registers
+// into two LDS buffers, the next slab's loads in flight under the current one's MFMAs; loads are dwords,
+// so any size and 4-byte alignment takes this path.  Within a slab a lane's half (lane / 32) takes KW / 2
+// consecutive k of its wave's KW: the order is the same for both operands, and x rows are then read
+// four k at a time.  The K-split waves' sums meet in LDS, in wave order (splitting K also keeps the
+// error against 64 bits below the plain fp32 sum's, 4e-7 .. 7e-7 relative against 9e-7 at K = 1024).
+// Bound by the fp32 matrix rate (64 cycles an MFMA) and, per slab, by the barrier and the staging around
+// its 256 .. 1024 cycles of MFMAs; measured beside its predecessor, one FMA per lane, product and k over
+// 4x4 outputs a thread: 777x1024x2816 (m, k, n) 245 -> 102 us, 2048x2048x4096 1000 -> 594 (116 TFLOP/s of
+// the 141 that a large fp32 library product reaches here), 1x2048x4096 395 -> 30.  Four waves of 64x64
+// outputs, without the K split, were no faster and lost accuracy.
+template <int WR, int WK, int KW>
+struct SwShape {
+  static constexpr int kThreads = 64 * WR * WK;
+  static constexpr int BM = 32 * WR, BN = 32, KS = WK * KW;
+  static constexpr int kPitchA = KS + 4;                      // floats: rows start 4 banks apart
+  static constexpr int kA = BM * kPitchA, kB = KS * 2 * BN;   // floats; a B row is 32 gate | 32 up
+  static constexpr int kSlab = kA + kB, kRed = WK * WR * 2048;
+  static constexpr int kSmem = 2 * kSlab > kRed ? 2 * kSlab : kRed;
+  static constexpr int kLoadA = BM * KS / kThreads, kLoadB = KS * BN / kThreads;   // kLoadB of each product
+  static_assert(KW % 8 == 0 && kThreads % KS == 0 && kThreads % BN == 0, "a thread keeps its k of A and column of B");
+  static_assert(BM * KS % kThreads == 0 && KS * BN % kThreads == 0, "whole loads per thread");
+};
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_range(const float* p, int64_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, uint32_t(bytes < 0xfffffffcll ? bytes : 0xfffffffcll),
+                                           0x00020000);
+}
+__device__ __forceinline__ float buffer_f32(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+}
+// WIDE: byte offsets within a workgroup's rows of x or a slab of the weights may pass 2^32.
+template <int WR, int WK, int KW, bool WIDE>
+__global__ __launch_bounds__(64 * WR * WK) void swiglu_f32(
+    const float* __restrict__ x, const float* __restrict__ wg, const float* __restrict__ wu, float* __restrict__ o,
+    int M, int N, int K) {
+  using Sh = SwShape<WR, WK, KW>;
+  using Off = std::conditional_t<WIDE, int64_t, uint32_t>;
+  __shared__ __attribute__((aligned(16))) float smem[Sh::kSmem];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wk = wave % WK, wr = wave / WK;
+  const int m0 = int(blockIdx.y) * Sh::BM, n0 = int(blockIdx.x) * Sh::BN;
+  const int col = lane & 31, h = lane >> 5;
+
+  // Loads: thread -> k ka of rows ra0, ra0 + kThreads / KS, ... of x; column cb of rows kb0, kb0 +
+  // kThreads / BN, ... of each weight.  Rows past M and columns past N repeat the last one (their
+  // outputs are not stored); k past K reads as zero, which only the last slab has to test.
+  constexpr int kStepA = Sh::kThreads / Sh::KS, kStepB = Sh::kThreads / Sh::BN;
+  const int ka = tid % Sh::KS, ra0 = tid / Sh::KS, cb = tid % Sh::BN, kb0 = tid / Sh::BN;
+  Off aoff[Sh::kLoadA], boff[Sh::kLoadB];
 #pragma unroll
-    for (int kk = 0; kk < kSwK; ++kk) {
-      float a[4], bg[4], bu[4];
+  for (int i = 0; i < Sh::kLoadA; ++i) aoff[i] = (Off(min(m0 + ra0 + i * kStepA, M - 1) - m0) * Off(K) + Off(ka)) * 4;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = xs[kk][ty * 4 + i];
+  for (int i = 0; i < Sh::kLoadB; ++i) boff[i] = (Off(kb0 + i * kStepB) * Off(N) + Off(min(n0 + cb, N - 1))) * 4;
+  float ra[Sh::kLoadA], rg[Sh::kLoadB], ru[Sh::kLoadB];
+  auto load = [&](int64_t k0) __attribute__((always_inline)) {
+    const float* const px = x + int64_t(m0) * K + k0;
+    const float* const pg = wg + k0 * N;
+    const float* const pu = wu + k0 * N;
+    if constexpr (WIDE) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        bg[j] = gs[kk][tx * 4 + j];
-        bu[j] = us[kk][tx * 4 + j];
+      for (int i = 0; i < Sh::kLoadA; ++i) ra[i] = k0 + ka < K ? px[aoff[i] / 4] : 0.f;
+#pragma unroll
+      for (int i = 0; i < Sh::kLoadB; ++i) {
+        const bool in = k0 + kb0 + i * kStepB < K;
+        rg[i] = in ? pg[boff[i] / 4] : 0.f;
+        ru[i] = in ? pu[boff[i] / 4] : 0.f;
       }
+    } else {
+      // the ranges end at the last element: rows of the weights past K read as zero; x past K within a
+      // row reads the next row and is zeroed below (an infinity there must not meet a zero weight)
+      const auto rx = make_range(px, (int64_t(M - m0) * K - k0) * 4);
+      const auto rwg = make_range(pg, (K - k0) * N * 4), rwu = make_range(pu, (K - k0) * N * 4);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < Sh::kLoadA; ++i) ra[i] = buffer_f32(rx, aoff[i]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          ag[i][j] = fmaf(a[i], bg[j], ag[i][j]);
-          au[i][j] = fmaf(a[i], bu[j], au[i][j]);
-        }
+      for (int i = 0; i < Sh::kLoadB; ++i) rg[i] = buffer_f32(rwg, boff[i]);
+#pragma unroll
+      for (int i = 0; i < Sh::kLoadB; ++i) ru[i] = buffer_f32(rwu, boff[i]);
+    }
+  };
+  // x past K, zeroed once its loads are waited for
+  auto zero_tail = [&](int64_t k0) __attribute__((always_inline)) {
+    if (!WIDE && k0 + Sh::KS > K) {
+#pragma unroll
+      for (int i = 0; i < Sh::kLoadA; ++i) ra[i] = k0 + ka < K ? ra[i] : 0.f;
+    }
+  };
+  auto store = [&](float* slab) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < Sh::kLoadA; ++i) slab[(ra0 + i * kStepA) * Sh::kPitchA + ka] = ra[i];
+    float* const b = slab + Sh::kA + kb0 * (2 * Sh::BN) + cb;
+#pragma unroll
+    for (int i = 0; i < Sh::kLoadB; ++i) {
+      b[i * kStepB * 2 * Sh::BN] = rg[i];
+      b[i * kStepB * 2 * Sh::BN + 32] = ru[i];
+    }
+  };
+  f32x16 ag, au;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) ag[e] = au[e] = 0.f;
+  auto compute = [&](const float* slab) __attribute__((always_inline)) {
+    const float* pa = slab + (32 * wr + col) * Sh::kPitchA + wk * KW + h * (KW / 2);
+    const float* pb = slab + Sh::kA + (wk * KW + h * (KW / 2)) * (2 * Sh::BN) + col;
+    // every fragment of the slab requested before the first MFMA, which waits for its own only
+    f32x4v a[KW / 8];
+    float bg[KW / 2], bu[KW / 2];
+#pragma unroll
+    for (int s = 0; s < KW / 2; ++s) {
+      if (s % 4 == 0) a[s / 4] = *reinterpret_cast<const f32x4v*>(pa + s);
+      bg[s] = pb[s * 2 * Sh::BN];
+      bu[s] = pb[s * 2 * Sh::BN + 32];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < KW / 2; ++s) {
+      ag = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s / 4][s % 4], bg[s], ag, 0, 0, 0);
+      au = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s / 4][s % 4], bu[s], au, 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // slab s in buffer s % 2: the next slab's loads run under this one's MFMAs and go into the other
+  // buffer, which every wave left before the barrier that ended the previous slab
+  load(0);
+  zero_tail(0);
+  store(smem);
+  __syncthreads();
+  int buf = 0;
+  for (int64_t k0 = 0; k0 < K; k0 += Sh::KS) {
+    const bool more = k0 + Sh::KS < K;
+    if (more) load(k0 + Sh::KS);
+    compute(smem + buf * Sh::kSlab);
+    buf ^= 1;
+    if (more) {
+      zero_tail(k0 + Sh::KS);
+      store(smem + buf * Sh::kSlab);
     }
     __syncthreads();
   }
+  // accumulator e of lane: row 8 (e / 4) + 4 h + e % 4 of the wave's block, column lane % 32;
+  // the slabs are done with: the waves' sums take their place
+  float* const red = smem + wave * 2048;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int gm = m0 + ty * 4 + i;
-    if (gm >= M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int gn = n0 + tx * 4 + j;
-      if (gn < N) {
-        const float g = ag[i][j];
-        o[int64_t(gm) * N + gn] = (g / (1.0f + exp_e(-g))) * au[i][j];
-      }
-    }
+  for (int e = 0; e < 16; ++e) {
+    const int r = 8 * (e >> 2) + 4 * h + (e & 3);
+    red[r * 32 + col] = ag[e];
+    red[1024 + r * 32 + col] = au[e];
   }
+  __syncthreads();
+  for (int t = tid; t < Sh::BM * Sh::BN; t += Sh::kThreads) {
+    const int r = t >> 5, c = t & 31;
+    const float* p = smem + (r >> 5) * WK * 2048 + (r & 31) * 32 + c;
+    float g = p[0], u = p[1024];
+#pragma unroll
+    for (int w = 1; w < WK; ++w) {
+      g += p[w * 2048];
+      u += p[w * 2048 + 1024];
+    }
+    if (m0 + r < M && n0 + c < N) o[int64_t(m0 + r) * N + n0 + c] = (g / (1.0f + exp_e(-g))) * u;
+  }
+}
+
+template <int WR, int WK, int KW, bool WIDE>
+int launch_swiglu_f32(const float* x, const float* wg, const float* wu, float* o, int64_t m, int64_t n, int64_t k,
+                      hipStream_t s) {
+  using Sh = SwShape<WR, WK, KW>;
+  const int64_t gx = (n + Sh::BN - 1) / Sh::BN, gy = (m + Sh::BM - 1) / Sh::BM;
+  if (gx > 0x7fffffff || gy > 65535) return PTB_ERR_GRID;
+  swiglu_f32<WR, WK, KW, WIDE><<<dim3(unsigned(gx), unsigned(gy)), dim3(Sh::kThreads), 0, s>>>(x, wg, wu, o, int(m),
+                                                                                            int(n), int(k));
+  return launch_status();
 }
 
 bool aligned_rows(const void* p, int64_t cols) { return aligned16(p) && cols % 4 == 0; }
@@ -327,9 +443,18 @@ PTB_EXPORT int ptb_swiglu_f32(const float* x, const float* wg, const float* wu, 
   if (m == 0 || n == 0) return PTB_OK;
   if (!x || !wg || !wu || !o) return PTB_ERR_NULL;
   if (m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff) return PTB_ERR_SHAPE;
-  const int64_t gx = (n + kSwT - 1) / kSwT, gy = (m + kSwT - 1) / kSwT;
-  if (gx > 0x7fffffff || gy > 65535) return PTB_ERR_GRID;
-  swiglu_f32<<<dim3(unsigned(gx), unsigned(gy)), dim3(kBlock), 0, static_cast<hipStream_t>(stream)>>>(
-      x, wg, wu, o, int(m), int(n), int(k));
-  return launch_status();
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  // By the number of 32x32 output blocks: up to two a CU, one block a workgroup of eight waves (few
+  // rows are bound by the latency of the weights: 1x2048x4096 30 us against 38 with four waves); to nine
+  // a CU, one block to four waves (200x1024x2816 38 us against 41 with eight); past it 64x32 outputs to
+  // four waves, which read less per product (2048x2048x4096 594 us against 668 with 32x32).  64-bit
+  // offsets only where a workgroup's rows of x or a slab of the weights may pass 4 GB.
+  const int64_t blocks = ((m + 31) / 32) * ((n + 31) / 32);
+  int dev = 0, cus = 256;
+  if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  if (k >= (int64_t(1) << 24) || n >= (int64_t(1) << 24))
+    return launch_swiglu_f32<2, 2, 16, true>(x, wg, wu, o, m, n, k, s);
+  if (blocks <= 2 * int64_t(cus)) return launch_swiglu_f32<1, 8, 8, false>(x, wg, wu, o, m, n, k, s);
+  if (blocks <= 9 * int64_t(cus)) return launch_swiglu_f32<1, 4, 8, false>(x, wg, wu, o, m, n, k, s);
+  return launch_swiglu_f32<2, 2, 16, false>(x, wg, wu, o, m, n, k, s);
 }

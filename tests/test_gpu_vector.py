@@ -257,3 +257,36 @@ def test_swiglu_f32_ragged(m, n, k):
     wu = randn((k, n), 9, dtype=torch.float32, std=0.1)
     o = ops.swiglu_f32(x.to(DEV), wg.to(DEV), wu.to(DEV)).cpu()
     assert_close(o, oracle.swiglu_f32(x, wg, wu), 1e-4, 1e-5, f"swiglu f32 {m}x{n}x{k}")
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 1, 1),            # one output, a tail of one k
+    (33, 65, 64),         # eight waves a 32x32 block: one whole slab, ragged blocks
+    (5, 31, 257),         # four slabs and a tail of one
+    (700, 800, 40),       # four waves a block (550 blocks): a slab and a tail of eight
+    (1500, 1601, 33),     # 64x32 outputs (2397 blocks): a slab and a tail of one, ragged both ways
+    (2049, 1200, 96),     # the same, whole slabs only
+])
+def test_swiglu_f32_blocks(m, n, k):
+    """Every workgroup shape of the fp32 SwiGLU at ragged sizes and slab tails.  Operands in {-1, 0, 1}
+    and {-2 .. 2} / 32 make both products exact in fp32 whatever the order of their sums, so only the
+    gate's exponential, sum, quotient and product round: within (|g| + 4) 2^-23 of the exact value, |g|
+    <= 2 * 257 / 32 < 17.  An infinity in one row of x, which the last k of the row before it is next to
+    in memory, stays in its row, and nothing is written past o."""
+    g = torch.Generator().manual_seed(m + n + k)
+    x = torch.randint(-1, 2, (m, k), generator=g).float()
+    wg, wu = (torch.randint(-2, 3, (k, n), generator=g).float() / 32 for _ in range(2))
+    guard = torch.full((m * n + 4096,), float("nan"), device=DEV)
+    o = guard[: m * n].view(m, n)
+    ops.swiglu_f32(x.to(DEV), wg.to(DEV), wu.to(DEV), out=o)
+    assert bool(guard[m * n:].isnan().all()), "the kernel wrote past o"
+    gate, up = x.double() @ wg.double(), x.double() @ wu.double()
+    want = gate / (1 + torch.exp(-gate)) * up
+    bound = (gate.abs() + 4) * 2.0 ** -23 * want.abs()
+    assert bool(((o.cpu().double() - want).abs() <= bound).all())
+    if m > 2:
+        first = o.clone()
+        x[2, 0] = float("inf")
+        ops.swiglu_f32(x.to(DEV), wg.to(DEV), wu.to(DEV), out=o)
+        keep = torch.arange(m) != 2
+        assert bits_equal(o.cpu()[keep], first.cpu()[keep])
