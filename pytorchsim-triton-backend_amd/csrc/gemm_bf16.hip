@@ -753,8 +753,7 @@ constexpr int64_t kFitK = 16384;   // past it (the fit ends at 12288) splits kee
 // the fitted range is split only when 128x128 tiles would leave a quarter of the CUs idle.  256-row
 // and 128-row tiles need 256 rows of A within the 32-bit buffer offsets, and the four-slot rings
 // their deeper run past the end of a slice of B.
-GemmPlan gemm_plan(int64_t m, int64_t n, int64_t k, bool may_split) {
-  const int64_t cus = cu_count();
+GemmPlan make_plan(int64_t m, int64_t n, int64_t k, bool may_split, int64_t cus) {
   auto tiles = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
   if (k < 1024 || (k > kFitK && 4 * tiles(128, 128) >= 3 * cus)) may_split = false;
   const double mem = kMemUs + kMemUsPerMB * 2e-6 * (double(k) * double(n) + double(m) * (double(k) + double(n)));
@@ -783,6 +782,21 @@ GemmPlan gemm_plan(int64_t m, int64_t n, int64_t k, bool may_split) {
     }
   }
   return best;
+}
+
+// The plan of a size is asked for twice a call, by the workspace query and by the launch: a thread
+// keeps its last one.
+GemmPlan gemm_plan(int64_t m, int64_t n, int64_t k, bool may_split) {
+  struct Last {
+    int64_t m = -1, n = 0, k = 0, cus = 0;
+    bool may_split = false;
+    GemmPlan plan{};
+  };
+  static thread_local Last last;
+  const int64_t cus = cu_count();
+  if (last.m != m || last.n != n || last.k != k || last.may_split != may_split || last.cus != cus)
+    last = Last{m, n, k, cus, may_split, make_plan(m, n, k, may_split, cus)};
+  return last.plan;
 }
 
 int launch_planned(const GemmPlan& p, const void* a, const void* b, const void* residual, void* c, int64_t m,

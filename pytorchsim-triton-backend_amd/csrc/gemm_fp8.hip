@@ -842,8 +842,7 @@ constexpr int kMaxSplits = 8;
 // Splits stay in one round of workgroups, in slices of at least a 128-deep step of a K of at least 512.
 // 64x128 tiles stay in one round too: past it the larger tiles' fewer bytes per flop decide, and the
 // model, which does not see L2 misses, was up to 6% wrong there.
-Fp8Plan fp8_plan(int64_t m, int64_t n, int64_t k, bool may_split) {
-  const int64_t cus = device_cus();
+Fp8Plan make_fp8_plan(int64_t m, int64_t n, int64_t k, bool may_split, int64_t cus) {
   const double mb = 1e-6 * double(k) * double(n);
   const double mem = kMemUs + kMemUsPerMB * (mb + 1e-6 * double(m) * (double(k) + 2.0 * double(n)));
   const double partial = kPartialUsPerMB * 8e-6 * double(m) * double(n);
@@ -873,6 +872,21 @@ Fp8Plan fp8_plan(int64_t m, int64_t n, int64_t k, bool may_split) {
     }
   }
   return best;
+}
+
+// The plan of a size is asked for twice a call, by the workspace query and by the launch: a thread
+// keeps its last one.
+Fp8Plan fp8_plan(int64_t m, int64_t n, int64_t k, bool may_split) {
+  struct Last {
+    int64_t m = -1, n = 0, k = 0, cus = 0;
+    bool may_split = false;
+    Fp8Plan plan{};
+  };
+  static thread_local Last last;
+  const int64_t cus = device_cus();
+  if (last.m != m || last.n != n || last.k != k || last.may_split != may_split || last.cus != cus)
+    last = Last{m, n, k, cus, may_split, make_fp8_plan(m, n, k, may_split, cus)};
+  return last.plan;
 }
 
 size_t fp8_workspace(const Fp8Plan& p, int64_t m, int64_t n) {

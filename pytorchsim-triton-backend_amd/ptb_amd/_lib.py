@@ -168,11 +168,14 @@ SIGNATURES.update({f"ptb_{fam}_args": _ARGS_SIG for fam in ARGS_FAMILIES})
 
 _lock = threading.Lock()
 _lib = None
+_fns = {}   # the loaded library's entry points by name (filled before _lib is set, never changed after)
 
 
 def load(path: Path | str | None = None) -> ctypes.CDLL:
     """Load (once) and return the library with every declared signature bound."""
     global _lib
+    if _lib is not None and path is None:
+        return _lib
     with _lock:
         if _lib is not None and path is None:
             return _lib
@@ -191,6 +194,7 @@ def load(path: Path | str | None = None) -> ctypes.CDLL:
             fn.restype = res
             fn.argtypes = args
         if path is None:
+            _fns.update({name: getattr(lib, name) for name in SIGNATURES})
             _lib = lib
         return lib
 
@@ -208,4 +212,6 @@ def check(fn: str, status: int) -> None:
 
 
 def call(fn: str, *args) -> None:
-    check(fn, getattr(load(), fn)(*args))
+    status = (_fns.get(fn) or getattr(load(), fn))(*args)
+    if status != PTB_OK:
+        check(fn, status)

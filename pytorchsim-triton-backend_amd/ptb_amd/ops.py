@@ -19,10 +19,15 @@ E4M3 = torch.float8_e4m3fn
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # the handle alone: a Stream object around it takes 1.9 us of an 8 us call to make
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _need(t: torch.Tensor, name: str, dtypes, ndim: int | None = None) -> None:
+    if (isinstance(t, torch.Tensor) and t.is_cuda and t.is_contiguous() and (ndim is None or t.dim() == ndim)
+            and (t.dtype in dtypes if isinstance(dtypes, tuple) else t.dtype == dtypes)):
+        return
+    # refused: the first reason, in this order
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
     if t.device.type != "cuda":
