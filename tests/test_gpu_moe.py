@@ -91,6 +91,27 @@ def test_sort_rows(rows, e, kind, desc):
     assert bits_equal(v.cpu(), wv) if kind == "float" else torch.equal(v.cpu(), wv)
 
 
+@pytest.mark.parametrize("e,lo,hi,desc", [
+    (257, 0, 128, False),               # 512 places, half of them padding; 8 of 16 waves have a segment
+    (1000, -5, 250, False),             # 255 key codes and the padding's: the counting sort's most
+    (1000, -5, 251, True),              # one more: the network
+    (4097, 7, 8, False),                # one key: positions in order
+    (16384, 0, 128, True),              # two chunks and a merge
+    (600, -2 ** 63, 2 ** 63 - 1, False),   # both ends of int64: the widest range
+])
+def test_sort_rows_key_ranges(e, lo, hi, desc):
+    """Few distinct keys take the counting sort, others the bitonic network: stable either way, the
+    range's ends included."""
+    g = gen(e)
+    x = torch.randint(lo, hi, (2 * e,), generator=g, dtype=I64)
+    for r in (0, e):
+        x[r + 3], x[r + 5] = lo, hi - 1 if hi < 2 ** 62 else hi
+    v, i = torch.empty_like(x, device=DEV), torch.empty(2 * e, dtype=I64, device=DEV)
+    moe.sort_rows(x.to(DEV), v, i, 2, desc)
+    wv, wi = oracle.sort_rows(x, 2, desc)
+    assert torch.equal(i.cpu(), wi) and torch.equal(v.cpu(), wv)
+
+
 @pytest.mark.parametrize("rows,e,k,largest", [(1024, 128, 8, True), (1, 128, 8, True), (4096, 128, 8, True),
                                               (100, 1000, 5, False), (7, 64, 64, True), (3, 100, 65, True),
                                               (5, 33, 8, False), (2, 300, 16, True), (9, 1024, 64, False)])
