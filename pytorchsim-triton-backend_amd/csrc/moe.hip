@@ -165,9 +165,15 @@ __global__ __launch_bounds__(kB) void expert_count(const int64_t* __restrict__ i
   for (int x = threadIdx.x; x < e; x += kB) hist[x] = 0;
   if (threadIdx.x < nr) mine[threadIdx.x] = ids[r0 + threadIdx.x];
   __syncthreads();
-  for (int64_t q = threadIdx.x; q < r0; q += kB) {
-    const int64_t id = ids[q];
-    if (id >= 0 && id < e) atomicAdd(&hist[id], 1);
+  // sixteen ids a thread in flight: one at a time, the last block of 16384 slots waits for 64 loads in
+  // turn (24 us, now 8.9; of 4096 slots 9 us, now 5.1)
+  for (int64_t q = threadIdx.x; q < r0; q += 16 * kB) {
+    int64_t id[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) id[u] = ids[q + u * kB < r0 ? q + u * kB : q];
+#pragma unroll
+    for (int u = 0; u < 16; ++u)
+      if (q + u * kB < r0 && id[u] >= 0 && id[u] < e) atomicAdd(&hist[id[u]], 1);
   }
   __syncthreads();
   const bool last = r0 + kSlotsPerBlock >= r;
