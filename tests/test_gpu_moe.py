@@ -383,3 +383,40 @@ def test_grouped_gemm_repeated_groups_fill_the_grid():
                      gemv=False)
     want = oracle.grouped_mm(a, b, group, starts, rows, k_dim, n, k_dim * n, c=c0)
     close_scaled(c.cpu(), want, "grouped gemm, repeated groups")
+
+
+@pytest.mark.parametrize("groups,n,k_dim,div", [
+    (128, 2056, 64, 32), (128, 2056, 192, 1), (128, 2056, 64, 1), (9, 520, 64, 1), (9, 264, 448, 4),
+    (40, 520, 64, 1), (40, 1544, 192, 1), (40, 1032, 320, 1),
+])
+def test_grouped_gemm_walk(groups, n, k_dim, div):
+    """The walk over the tiles of all programs: groups of 0 rows to two tiles and a remainder, at the edges
+    of 64- and 128-row tiles; walks of one tile a workgroup and of several; tiles of one, two and more K steps
+    (fewer than the ring's depth: the cursor runs several tiles ahead); column tiles with a remainder;
+    programs in another order than their groups.  Rows of no group keep C's values."""
+    sizes = torch.tensor([0, 1, 63, 64, 65, 127, 128, 129, 257], dtype=I32) // div
+    rows = sizes[(torch.arange(groups) * 5 + 3) % 9]
+    starts = torch.cumsum(rows + 1, 0).to(I32) - rows     # a row of no group before each
+    a_rows = int(rows.sum()) + groups
+    group = torch.randperm(groups, generator=gen(40)).to(I32)
+    a = (torch.randn(a_rows * k_dim, generator=gen(41)) / 8).to(BF16)
+    b = (torch.randn(groups * k_dim * n, generator=gen(42)) / 8).to(BF16)
+    c0 = torch.randn(a_rows * n, generator=gen(43)).to(BF16)
+    c = c0.to(DEV)
+    moe.grouped_gemm(a.to(DEV), b.to(DEV), group.to(DEV), starts.to(DEV), rows.to(DEV), c, k_dim, n, k_dim * n,
+                     gemv=False)
+    want = c0.clone().reshape(a_rows, n)
+    ad, bd = a.reshape(a_rows, k_dim).double(), b.reshape(groups, k_dim, n).double()
+    for g in range(groups):
+        s, r = int(starts[g]), int(rows[g])
+        want[s:s + r] = (ad[s:s + r] @ bd[g]).to(F32).to(BF16)
+    got = c.cpu().reshape(a_rows, n)
+    # both sides round once to bf16, so they may differ by an ulp (2^-7 of the value), plus the fp32 sum's
+    # own error, k roundings of at most sum |a b|
+    bound = want.abs().double() * 2 ** -7
+    for g in range(groups):
+        s, r = int(starts[g]), int(rows[g])
+        bound[s:s + r] += (ad[s:s + r].abs() @ bd[g].abs()) * k_dim * 2 ** -24
+    assert bool(((got.double() - want.double()).abs() <= bound).all())
+    gaps = starts.long() - 1
+    assert torch.equal(got[gaps], c0.reshape(a_rows, n)[gaps])
