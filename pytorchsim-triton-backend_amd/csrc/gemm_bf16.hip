@@ -636,10 +636,13 @@ constexpr int kMaxDedupGroups = 1024;   // group tables up to this size have rep
 // steps are no whole number of ring turns; that costs 16 address adds a stage.  Tiles are numbered
 // program by program, column by column, rows fastest, and XCD x takes a contiguous range, so row tiles
 // that share a weight panel run side by side on one L2.  128 experts, gate_up (2048 -> 1536) and down
-// (768 -> 2048) together: 64 routed rows 91 -> 81 us, 512 203 -> 190, 2048 243 -> 226, 4096 273 -> 268
-// (4.5 TB/s: three experts take a second row tile and a fourth round of tiles), 8192 315 -> 274, 16384
+// (768 -> 2048) together: 64 routed rows 91 -> 81 us, 512 203 -> 190, 2048 243 -> 226, 4096 273 -> 268,
+// 8192 315 -> 274, 16384
 // 406 -> 320, 32768 617 -> 441.
-template <int WM, int WN, int NS, int WGS>
+// STREAM (see grouped_plan): the weights of a group with one row tile go by the streaming policy, which
+// takes these (other boxes, popularity N(0, 0.5) in the log) to 128 rows 118 us (132 without), 512 181
+// (207), 2048 201 (224), 4096 219 (239), 8192 256 (279).
+template <int WM, int WN, int NS, int WGS, bool STREAM>
 __global__ __launch_bounds__(kThreads, WGS) void grouped_gemm_kernel(const uint16_t* __restrict__ A,
                                                                    const uint16_t* __restrict__ B,
                                                                    uint16_t* __restrict__ C, int N, int K, int tiles_n,
@@ -699,6 +702,7 @@ __global__ __launch_bounds__(kThreads, WGS) void grouped_gemm_kernel(const uint1
   // pref[p] <= id: each lane looks at four
   struct Tile {
     int first, rows, n0, g;
+    bool once;   // the group's only row tile: no other tile reads its weight columns
   };
   auto locate = [&](unsigned id) __attribute__((always_inline)) {
     const unsigned x = id & 7, n8 = total >> 3;
@@ -716,6 +720,7 @@ __global__ __launch_bounds__(kThreads, WGS) void grouped_gemm_kernel(const uint1
     t.first = __builtin_amdgcn_readfirstlane(pstart[p]) + mt * BM;
     t.rows = min(BM, rows - mt * BM);
     t.n0 = tn * BN;
+    t.once = rt == 1;
     t.g = __builtin_amdgcn_readfirstlane(pgroup[p]);
     return t;
   };
@@ -742,12 +747,14 @@ __global__ __launch_bounds__(kThreads, WGS) void grouped_gemm_kernel(const uint1
   // Past the last tile its resources are empty: such stages write zeros nobody reads
   unsigned next_load = tile;
   int lkt = nk, lslot = 0;
+  bool lonce = false;
   i32x4 rsrc_a = make_rsrc(A, 0), rsrc_b = make_rsrc(B, 0);
   auto advance = [&]() __attribute__((always_inline)) {   // before a stage's DMAs
     if (lkt == nk) {
       lkt = 0;
       if (next_load < total) {
         const Tile t = locate(next_load);
+        lonce = STREAM && t.once;
         rsrc_a = make_rsrc(A + int64_t(t.first) * K, uint32_t(int64_t(t.rows) * K) * 2u);
         rsrc_b = make_rsrc(B + int64_t(t.g) * gp.sbg + t.n0, uint32_t((int64_t(K) * N - t.n0) * 2));
         next_load += gridDim.x;
@@ -760,9 +767,14 @@ __global__ __launch_bounds__(kThreads, WGS) void grouped_gemm_kernel(const uint1
   };
   auto dma_one = [&](int t) __attribute__((always_inline)) {
     const uint32_t kt = lkt > nk ? 0u : uint32_t(lkt);
-    if (t < Sh::kDmaA) dma16(rsrc_a, wave_a + uint32_t(lslot * kABytes + t * 1024), a_voff[t], kt * (BK * 2u));
-    else dma16(rsrc_b, wave_b + uint32_t(lslot * kBBytes + (t - Sh::kDmaA) * 1024), b_voff[t - Sh::kDmaA],
-               kt * (BK * 2u) * uint32_t(N));
+    if (t < Sh::kDmaA) {
+      dma16(rsrc_a, wave_a + uint32_t(lslot * kABytes + t * 1024), a_voff[t], kt * (BK * 2u));
+    } else {
+      const int b = t - Sh::kDmaA;
+      const uint32_t at = wave_b + uint32_t(lslot * kBBytes + b * 1024), soff = kt * (BK * 2u) * uint32_t(N);
+      if (STREAM && lonce) dma16_once(rsrc_b, at, b_voff[b], soff);
+      else dma16(rsrc_b, at, b_voff[b], soff);
+    }
   };
   auto stage_out = [&]() __attribute__((always_inline)) {   // after a stage's DMAs
     lkt += lkt < nk ? 1 : 0;
@@ -1165,12 +1177,22 @@ int launch_swiglu(const void* a, const void* b, void* c, int64_t m, int64_t n, i
 // within 0.5% (geometric mean) of the best of the three over 79 (groups, rows, n, k) points, 2 to 128
 // groups and 24 to 16384 rows, at worst 1.1% slower and on average 1.09x faster than one workgroup a
 // 128x128 tile.
-int grouped_tile(int64_t groups, int64_t a_rows, int64_t n, int64_t k, int64_t cus) {
+struct GroupedPlan {
+  int tile;
+  bool stream;
+};
+// The weights go by the streaming policy, tile by tile where a group has one row tile, if a group's mean
+// rows fit one and the table's weights are more than the 256 MB last-level cache, which then keeps
+// little of them from one call to the next.  128 experts, gate_up / down: 4 rows each 134.4 -> 119.2 /
+// 72.7 -> 63.1 us, 32 150.9 -> 139.2 / 88.0 -> 80.3, 128 204 -> 202 / 109 -> 104; at 200 rows 255 -> 262
+// / 145 -> 146.  Weights that do fit: 32 experts of 6 MB (201 MB), 4 rows, the same weights each call 31.6
+// -> 35.0, other weights each call 38.8 -> 35.7.
+GroupedPlan grouped_plan(int64_t groups, int64_t a_rows, int64_t n, int64_t k, int64_t cus) {
   struct {
     int bm, bn;
     double step, load, fixed;
   } const tiles[] = {{128, 256, 0.592, 0.250, 3.92}, {128, 128, 0.340, 0.196, 2.42}, {64, 128, 0.296, 0.141, 1.68}};
-  if (groups <= 0) return 2;
+  if (groups <= 0) return {2, false};
   const double hit = double(groups) * (1.0 - std::exp(-double(a_rows) / double(groups)));
   const double mean = double(a_rows) / hit, steps = double(k / 64);
   int best = 0;
@@ -1185,16 +1207,19 @@ int grouped_tile(int64_t groups, int64_t a_rows, int64_t n, int64_t k, int64_t c
       best = i;
     }
   }
-  return best;
+  constexpr double kCacheBytes = double(int64_t(1) << 28);
+  return {best, mean <= tiles[best].bm && double(groups) * double(n) * double(k) * 2.0 > kCacheBytes};
 }
 
 // A workgroup for each of the tiles there can be, up to the CUs' WGS each.
 template <int WM, int WN, int NS, int WGS>
-int launch_grouped(const void* a, const void* b, void* c, int64_t n, int64_t k, const Groups& gp, hipStream_t s) {
+int launch_grouped(bool stream, const void* a, const void* b, void* c, int64_t n, int64_t k, const Groups& gp,
+                   hipStream_t s) {
   using Sh = Shape<WM, WN>;
   const int64_t tn = (n + Sh::BN - 1) / Sh::BN, tm = (int64_t(gp.a_rows) + Sh::BM - 1) / Sh::BM + gp.nprog;
   const int64_t grid = std::min<int64_t>(tm * tn, WGS * cu_count());
-  grouped_gemm_kernel<WM, WN, NS, WGS><<<dim3(unsigned(grid)), dim3(kThreads), 0, s>>>(
+  const auto kernel = stream ? grouped_gemm_kernel<WM, WN, NS, WGS, true> : grouped_gemm_kernel<WM, WN, NS, WGS, false>;
+  kernel<<<dim3(unsigned(grid)), dim3(kThreads), 0, s>>>(
       static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), static_cast<uint16_t*>(c), int(n), int(k),
       int(tn), gp);
   return launch_status();
@@ -1245,9 +1270,10 @@ PTB_EXPORT int ptb_grouped_gemm_bf16(const void* a, const void* b, const int32_t
   if (((a_rows + 127) / 128 + nprog) * ((n + 127) / 128) > 0x7fffffff) return PTB_ERR_GRID;
   const Groups gp{group, start, rows, int(nprog), int(ntab), int(nweights), int(a_rows), weight_stride};
   hipStream_t s = static_cast<hipStream_t>(stream);
-  switch (grouped_tile(std::min(nprog, std::min(ntab, nweights)), a_rows, n, k, cu_count())) {
-    case 0: return launch_grouped<2, 4, 3, 1>(a, b, c, n, k, gp, s);
-    case 1: return launch_grouped<2, 2, 4, 1>(a, b, c, n, k, gp, s);
-    default: return launch_grouped<1, 2, 3, 2>(a, b, c, n, k, gp, s);
+  const GroupedPlan p = grouped_plan(std::min(nprog, std::min(ntab, nweights)), a_rows, n, k, cu_count());
+  switch (p.tile) {
+    case 0: return launch_grouped<2, 4, 3, 1>(p.stream, a, b, c, n, k, gp, s);
+    case 1: return launch_grouped<2, 2, 4, 1>(p.stream, a, b, c, n, k, gp, s);
+    default: return launch_grouped<1, 2, 3, 2>(p.stream, a, b, c, n, k, gp, s);
   }
 }

@@ -227,6 +227,12 @@ __device__ __forceinline__ void dma16(i32x4 rsrc, uint32_t lds_base, uint32_t vo
                :: "s"(lds_base), "v"(voff), "s"(rsrc), "s"(soff) : "memory", "m0");
 }
 
+// The same with the streaming policy, for bytes that no later load of the launch finds in a cache.
+__device__ __forceinline__ void dma16_once(i32x4 rsrc, uint32_t lds_base, uint32_t voff, uint32_t soff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+               :: "s"(lds_base), "v"(voff), "s"(rsrc), "s"(soff) : "memory", "m0");
+}
+
 // A run of N (2 or 4) such loads into consecutive KB of LDS: the i-th reads byte offset
 // voff[i] + 1024 * i + soff into lds_base + 1024 * i + 16 * lane.  The instruction's offset field
 // advances the global and the LDS address alike, so one m0 write and one wait state serve the run.

@@ -420,3 +420,32 @@ def test_grouped_gemm_walk(groups, n, k_dim, div):
     assert bool(((got.double() - want.double()).abs() <= bound).all())
     gaps = starts.long() - 1
     assert torch.equal(got[gaps], c0.reshape(a_rows, n)[gaps])
+
+
+@pytest.mark.parametrize("groups,n,k_dim,sizes", [
+    (72, 1024, 2048, [0, 1, 3, 16, 63, 64, 65, 2]), (72, 1024, 2048, [0, 127, 64, 128, 65, 129, 33, 1]),
+    (72, 1024, 2048, [0, 257, 127, 128, 129, 65, 64, 1]), (130, 1096, 1024, [5, 64, 0, 63, 65, 40, 129, 2]),
+])
+def test_grouped_gemm_streamed_weights(groups, n, k_dim, sizes):
+    """Weights of more than the last-level cache's 256 MB, which groups of one row tile read by the streaming
+    policy and groups of two or three as usual, both in one walk, for each of the three tiles."""
+    assert groups * n * k_dim * 2 > 1 << 28
+    rows = torch.tensor(sizes, dtype=I32)[(torch.arange(groups) * 5 + 3) % 8]
+    starts = torch.cumsum(rows, 0).to(I32) - rows
+    a_rows = int(rows.sum())
+    g = torch.Generator(device=DEV).manual_seed(44)
+    a = (torch.randn(a_rows, k_dim, generator=g, device=DEV) / 8).to(BF16)
+    b = (torch.randn(groups, k_dim, n, generator=g, device=DEV) / 8).to(BF16)
+    c = torch.full((a_rows * n,), float("nan"), dtype=BF16, device=DEV)
+    group = torch.arange(groups, dtype=I32)
+    moe.grouped_gemm(a.view(-1), b.view(-1), group.to(DEV), starts.to(DEV), rows.to(DEV), c, k_dim, n, k_dim * n,
+                     gemv=False)
+    got = c.view(a_rows, n)
+    for i in range(groups):
+        s, r = int(starts[i]), int(rows[i])
+        if r:
+            af, bf = a[s:s + r].float(), b[i].float()
+            want = (af @ bf).to(BF16).double()
+            # an ulp of bf16 between two roundings, plus k fp32 roundings of at most sum |a b| on each side
+            bound = want.abs() * 2 ** -7 + (af.abs() @ bf.abs()).double() * k_dim * 2 ** -23
+            assert bool(((got[s:s + r].double() - want).abs() <= bound).all()), f"group {i} of {r} rows"
