@@ -801,7 +801,8 @@ __device__ __forceinline__ i16x4 lds_tr16(uint32_t addr) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_i16x4*>(size_t(addr)));
 }
 
-template <int G>
+// STREAM (kStreamBytes below): K and V go by the streaming policy.
+template <int G, bool STREAM>
 __global__ __launch_bounds__(64) void attn_decode_mfma(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kc,
                                                        const uint16_t* __restrict__ Vc, uint16_t* __restrict__ O,
                                                        float* __restrict__ part, int S, float c, int steps,
@@ -846,9 +847,10 @@ __global__ __launch_bounds__(64) void attn_decode_mfma(const uint16_t* __restric
     }
     const uint32_t st = lds0 + uint32_t(P * 2 * kWTile);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) dma16_run(rk, __builtin_amdgcn_readfirstlane(st + i * 4096), koff[i], 0);
+    for (int i = 0; i < 2; ++i) dma16_run<STREAM>(rk, __builtin_amdgcn_readfirstlane(st + i * 4096), koff[i], 0);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) dma16_run(rv, __builtin_amdgcn_readfirstlane(st + kWTile + i * 4096), voff[i], 0);
+    for (int i = 0; i < 2; ++i)
+      dma16_run<STREAM>(rv, __builtin_amdgcn_readfirstlane(st + kWTile + i * 4096), voff[i], 0);
   };
   issue(0, std::integral_constant<int, 0>{});
 
@@ -1011,10 +1013,18 @@ WavePlan wave_plan(int64_t seq) {
   return {int(steps), int((n + steps - 1) / steps)};
 }
 
+// K and V of more than the 256 MB last-level cache, which keeps none of them from one call to the next,
+// go by the streaming policy: 128 kv heads, 8192 keys, G = 4 (537 MB) 102 -> 96 us.  Smaller ones keep the
+// default, under which they may still be cached: 64 kv heads (268 MB), the same caches each call 45.1 us
+// against 48.5 streamed, other caches each call 52.9 against 50.0.
+constexpr int64_t kStreamBytes = int64_t(1) << 28;
+
 template <int G>
 void launch_attn_decode_mfma(const uint16_t* q, const uint16_t* k, const uint16_t* v, uint16_t* o, float* part,
                              int nkv, int seq, float c, const WavePlan& p, const QNorm& qn, hipStream_t s) {
-  attn_decode_mfma<G><<<dim3(unsigned(p.records), unsigned(nkv)), dim3(64), 0, s>>>(
+  const auto kernel =
+      int64_t(nkv) * seq * (2 * kD * 2) > kStreamBytes ? attn_decode_mfma<G, true> : attn_decode_mfma<G, false>;
+  kernel<<<dim3(unsigned(p.records), unsigned(nkv)), dim3(64), 0, s>>>(
       q, k, v, o, part, seq, c, p.steps, qn.w, qn.cos, qn.sin, qn.eps);
   if (p.records > 1) attn_decode_merge<G><<<dim3(unsigned(nkv), unsigned(G)), dim3(256), 0, s>>>(part, o, p.records);
 }

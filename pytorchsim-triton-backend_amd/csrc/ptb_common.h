@@ -236,23 +236,31 @@ __device__ __forceinline__ void dma16_once(i32x4 rsrc, uint32_t lds_base, uint32
 // A run of N (2 or 4) such loads into consecutive KB of LDS: the i-th reads byte offset
 // voff[i] + 1024 * i + soff into lds_base + 1024 * i + 16 * lane.  The instruction's offset field
 // advances the global and the LDS address alike, so one m0 write and one wait state serve the run.
-template <int N>
+// ONCE: the streaming policy, as dma16_once.
+#define PTB_DMA16_RUN(NT)                                                                                          \
+  if constexpr (N == 2)                                                                                            \
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"                                                               \
+                 "buffer_load_dwordx4 %1, %3, %4 offen" NT " lds\n\t"                                              \
+                 "buffer_load_dwordx4 %2, %3, %4 offen offset:1024" NT " lds"                                      \
+                 :: "s"(lds_base), "v"(voff[0]), "v"(voff[1]), "s"(rsrc), "s"(soff) : "memory", "m0");             \
+  else                                                                                                             \
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"                                                               \
+                 "buffer_load_dwordx4 %1, %5, %6 offen" NT " lds\n\t"                                              \
+                 "buffer_load_dwordx4 %2, %5, %6 offen offset:1024" NT " lds\n\t"                                  \
+                 "buffer_load_dwordx4 %3, %5, %6 offen offset:2048" NT " lds\n\t"                                  \
+                 "buffer_load_dwordx4 %4, %5, %6 offen offset:3072" NT " lds"                                      \
+                 :: "s"(lds_base), "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(rsrc), "s"(soff)    \
+                 : "memory", "m0")
+template <bool ONCE = false, int N>
 __device__ __forceinline__ void dma16_run(i32x4 rsrc, uint32_t lds_base, const uint32_t (&voff)[N], uint32_t soff) {
   static_assert(N == 2 || N == 4, "runs of two or four");
-  if constexpr (N == 2)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
-                 "buffer_load_dwordx4 %1, %3, %4 offen lds\n\t"
-                 "buffer_load_dwordx4 %2, %3, %4 offen offset:1024 lds"
-                 :: "s"(lds_base), "v"(voff[0]), "v"(voff[1]), "s"(rsrc), "s"(soff) : "memory", "m0");
-  else
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
-                 "buffer_load_dwordx4 %1, %5, %6 offen lds\n\t"
-                 "buffer_load_dwordx4 %2, %5, %6 offen offset:1024 lds\n\t"
-                 "buffer_load_dwordx4 %3, %5, %6 offen offset:2048 lds\n\t"
-                 "buffer_load_dwordx4 %4, %5, %6 offen offset:3072 lds"
-                 :: "s"(lds_base), "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(rsrc), "s"(soff)
-                 : "memory", "m0");
+  if constexpr (ONCE) {
+    PTB_DMA16_RUN(" nt");
+  } else {
+    PTB_DMA16_RUN("");
+  }
 }
+#undef PTB_DMA16_RUN
 
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {

@@ -152,6 +152,23 @@ def test_attention_decode_fused_qnorm_rope(nkv, g, s):
     assert_close(fused, want, RTOL, 2e-2, f"fused decode vs oracle {nkv}x{g}x{s}")
 
 
+@pytest.mark.parametrize("g", [1, 2, 3, 4, 6, 8])
+def test_attention_decode_streamed_cache(g):
+    """K and V just past the last-level cache's 256 MB take the streaming policy, the two halves of their heads
+    do not: the same bits, and a head of each end against the oracle."""
+    nkv, s = 70, 7501                            # a last step of 13 keys
+    assert nkv * s * 512 > 1 << 28 >= nkv // 2 * s * 512
+    r = torch.Generator(device=DEV).manual_seed(g)
+    q, k, v = (torch.randn(nkv, n, 128, generator=r, device=DEV).bfloat16() for n in (g, s, s))
+    got = ops.attention_decode(q, k, v)
+    h = nkv // 2
+    halves = torch.cat([ops.attention_decode(q[:h], k[:h], v[:h]), ops.attention_decode(q[h:], k[h:], v[h:])])
+    assert torch.equal(got, halves)
+    for i in (0, nkv - 1):
+        want = oracle.attention_decode(q[i:i + 1].cpu(), k[i:i + 1].cpu(), v[i:i + 1].cpu())
+        assert_close(got[i:i + 1].cpu(), want, RTOL, 2e-2, f"decode streamed head {i} x{g}")
+
+
 def test_attention_decode_workspace_reuse():
     """One caller workspace serves consecutive calls of different shapes (each call's records
     replace the last call's)."""
