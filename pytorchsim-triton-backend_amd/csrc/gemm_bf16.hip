@@ -637,11 +637,10 @@ constexpr int kMaxDedupGroups = 1024;   // group tables up to this size have rep
 // program by program, column by column, rows fastest, and XCD x takes a contiguous range, so row tiles
 // that share a weight panel run side by side on one L2.  128 experts, gate_up (2048 -> 1536) and down
 // (768 -> 2048) together: 64 routed rows 91 -> 81 us, 512 203 -> 190, 2048 243 -> 226, 4096 273 -> 268,
-// 8192 315 -> 274, 16384
-// 406 -> 320, 32768 617 -> 441.
-// STREAM (see grouped_plan): the weights of a group with one row tile go by the streaming policy, which
-// takes these (other boxes, popularity N(0, 0.5) in the log) to 128 rows 118 us (132 without), 512 181
-// (207), 2048 201 (224), 4096 219 (239), 8192 256 (279).
+// 8192 315 -> 274, 16384 406 -> 320, 32768 617 -> 441.
+// STREAM (see grouped_plan): the weights of a group with one row tile go by the streaming policy.  On
+// another box, with skewed groups, both GEMMs without and with it: 128 routed rows 132 -> 118 us, 512 207 ->
+// 181, 2048 224 -> 201, 4096 239 -> 219, 8192 279 -> 256.
 template <int WM, int WN, int NS, int WGS, bool STREAM>
 __global__ __launch_bounds__(kThreads, WGS) void grouped_gemm_kernel(const uint16_t* __restrict__ A,
                                                                    const uint16_t* __restrict__ B,
