@@ -162,9 +162,12 @@ int ptb_gemm_bf16(const void* a, const void* b, const void* residual, void* c, i
  * K >= 1024), K may be cut into 2 to 8 slices (at least 128 deep, tiles x slices within the CUs, as a
  * fitted cost model of the tiles' K steps, the operand traffic and the partials decides)
  * multiplied by separate workgroups into fp32 partials that a finish pass sums (+ residual) and
- * rounds once.  ptb_gemm_bf16_workspace_bytes is 0 for shapes that do not split; then
- * ptb_gemm_bf16_ws is ptb_gemm_bf16.  A split shape refuses a NULL workspace (PTB_ERR_NULL) or one
- * shorter than ptb_gemm_bf16_workspace_bytes (PTB_ERR_WORKSPACE).
+ * rounds once.  ptb_gemm_bf16_workspace_bytes is what the fastest split takes, 0 for shapes that do not
+ * split; then ptb_gemm_bf16_ws is ptb_gemm_bf16.  With a shorter workspace the fastest split that fits
+ * it runs, or one pass, as with none or one that is not 16-byte aligned -- except where few 64x128 tiles
+ * (at most half the CUs) and a long K make one pass much slower: there a NULL workspace is refused
+ * (PTB_ERR_NULL), as is one too short for the 2 to 8 slices of those tiles (PTB_ERR_WORKSPACE) or
+ * misaligned (PTB_ERR_ALIGN).
  * Replaces: the same kernels as ptb_gemm_bf16 (the small M x N gemm_<M>x<K>x<N>_bf16 shapes). */
 size_t ptb_gemm_bf16_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int ptb_gemm_bf16_ws(const void* a, const void* b, const void* residual, void* c, int64_t m, int64_t n, int64_t k,

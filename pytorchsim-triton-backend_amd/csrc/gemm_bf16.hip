@@ -997,10 +997,12 @@ constexpr int64_t kFitK = 16384;   // past it (the fit ends at 12288) splits kee
 // finish launch costs more than the shorter slices save), all in one round of workgroups; a K past
 // the fitted range is split only when 128x128 tiles would leave a quarter of the CUs idle.  256-row
 // and 128-row tiles need 256 rows of A within the 32-bit buffer offsets, and the four-slot rings
-// their deeper run past the end of a slice of B.
-GemmPlan make_plan(int64_t m, int64_t n, int64_t k, bool may_split, int64_t cus) {
+// their deeper run past the end of a slice of B.  The partials take at most `room` bytes (kAnyRoom: what
+// they need; 0: one pass).
+constexpr size_t kAnyRoom = ~size_t(0);
+GemmPlan make_plan(int64_t m, int64_t n, int64_t k, size_t room, int64_t cus) {
   auto tiles = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
-  if (k < 1024 || (k > kFitK && 4 * tiles(128, 128) >= 3 * cus)) may_split = false;
+  const bool may_split = room > 0 && k >= 1024 && (k <= kFitK || 4 * tiles(128, 128) < 3 * cus);
   const double mem = kMemUs + kMemUsPerMB * 2e-6 * (double(k) * double(n) + double(m) * (double(k) + double(n)));
   const double partial = kPartialUsPerMB * 8e-6 * double(m) * double(n);
   const bool tall = int64_t(256) * k * 2 < (int64_t(1) << 32);
@@ -1014,6 +1016,7 @@ GemmPlan make_plan(int64_t m, int64_t n, int64_t k, bool may_split, int64_t cus)
       if (sp > 1 && (t * sp > cus || k / sp < 128)) break;
       const int64_t kc = sp == 1 ? k : ((k + sp - 1) / sp + 63) / 64 * 64;
       const int64_t splits = (k + kc - 1) / kc;
+      if (splits > 1 && size_t(splits) * size_t(m) * size_t(n) * sizeof(float) > room) break;
       if ((kc + run_ahead) * n * 2 >= (int64_t(1) << 32)) continue;
       const int64_t w = t * splits, full = (w - 1) / cus;
       const double steps = double((kc + 63) / 64), last = double(w - full * cus) / double(cus);
@@ -1031,17 +1034,37 @@ GemmPlan make_plan(int64_t m, int64_t n, int64_t k, bool may_split, int64_t cus)
 
 // The plan of a size is asked for twice a call, by the workspace query and by the launch: a thread
 // keeps its last one.
-GemmPlan gemm_plan(int64_t m, int64_t n, int64_t k, bool may_split) {
+GemmPlan gemm_plan(int64_t m, int64_t n, int64_t k, size_t room) {
   struct Last {
     int64_t m = -1, n = 0, k = 0, cus = 0;
-    bool may_split = false;
+    size_t room = 0;
     GemmPlan plan{};
   };
   static thread_local Last last;
   const int64_t cus = cu_count();
-  if (last.m != m || last.n != n || last.k != k || last.may_split != may_split || last.cus != cus)
-    last = Last{m, n, k, cus, may_split, make_plan(m, n, k, may_split, cus)};
+  if (last.m != m || last.n != n || last.k != k || last.room != room || last.cus != cus)
+    last = Last{m, n, k, cus, room, make_plan(m, n, k, room, cus)};
   return last.plan;
+}
+
+// The K slices that ptb_gemm_bf16_ws asks a caller's workspace for: those of 64x128 tiles on at most half
+// of the CUs where a workgroup's operand stream (90 GB/s; 2.5 us to launch) gets shorter by more than the
+// finish launch (1.5 us) and the partials' traffic (2.5 TB/s) take.  Part of the call's contract, not of the plan: such a call is refused without
+// the room for them, and every other one runs with the room it has.
+int required_slices(int64_t m, int64_t n, int64_t k) {
+  const int64_t cus = cu_count(), t64 = ((m + 63) / 64) * ((n + 127) / 128);
+  auto stream = [&](int sp) { return 2.5 + double(k) / sp * (64 + 128) * 2 / 90e3; };
+  int best = 1;
+  double best_us = stream(1);
+  for (int sp = 2; sp <= 8 && k >= 1024 && k / sp >= 256 && t64 * sp <= cus; sp *= 2) {
+    const double us = stream(sp) + (1.5 + sp * double(m) * double(n) * 8 / 2.5e6);
+    if (us < best_us) {
+      best_us = us;
+      best = sp;
+    }
+  }
+  const int64_t kc = ((k + best - 1) / best + 63) / 64 * 64;
+  return int((k + kc - 1) / kc);
 }
 
 int launch_planned(const GemmPlan& p, const void* a, const void* b, const void* residual, void* c, int64_t m,
@@ -1070,7 +1093,7 @@ PTB_EXPORT int ptb_gemm_bf16(const void* a, const void* b, const void* residual,
     return PTB_ERR_UNSUPPORTED;
   if (!aligned16(a) || !aligned16(b) || !aligned16(c) || (residual && !aligned16(residual)))
     return PTB_ERR_ALIGN;
-  return launch_planned(gemm_plan(m, n, k, false), a, b, residual, c, m, n, k, static_cast<hipStream_t>(stream));
+  return launch_planned(gemm_plan(m, n, k, 0), a, b, residual, c, m, n, k, static_cast<hipStream_t>(stream));
 }
 
 namespace {
@@ -1128,22 +1151,32 @@ size_t plan_workspace(const GemmPlan& p, int64_t m, int64_t n) {
 
 PTB_EXPORT size_t ptb_gemm_bf16_workspace_bytes(int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || n <= 0 || k <= 0 || m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff) return 0;
-  return plan_workspace(gemm_plan(m, n, k, true), m, n);
+  return plan_workspace(gemm_plan(m, n, k, kAnyRoom), m, n);
 }
 
 PTB_EXPORT int ptb_gemm_bf16_ws(const void* a, const void* b, const void* residual, void* c, int64_t m, int64_t n,
                                 int64_t k, void* workspace, size_t workspace_bytes, void* stream) {
   if (m <= 0 || n <= 0 || k <= 0 || k % 64 || n % 8 || m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff)
     return ptb_gemm_bf16(a, b, residual, c, m, n, k, stream);   // refused or trivial there
-  const GemmPlan p = gemm_plan(m, n, k, true);
-  if (p.splits < 2) return ptb_gemm_bf16(a, b, residual, c, m, n, k, stream);   // no split for this shape
-  if (!a || !b || !c || !workspace) return PTB_ERR_NULL;
-  if (workspace_bytes < plan_workspace(p, m, n)) return PTB_ERR_WORKSPACE;
+  GemmPlan p = gemm_plan(m, n, k, kAnyRoom);
+  if (p.splits > 1) {
+    const size_t need = plan_workspace(p, m, n);
+    const size_t room = workspace && aligned16(workspace) ? workspace_bytes : 0;
+    const int required = required_slices(m, n, k);
+    if (required > 1) {
+      if (!a || !b || !c || !workspace) return PTB_ERR_NULL;
+      if (workspace_bytes < std::min(need, size_t(required) * size_t(m) * size_t(n) * sizeof(float)))
+        return PTB_ERR_WORKSPACE;
+      if (!aligned16(workspace)) return PTB_ERR_ALIGN;
+    }
+    if (room < need) p = make_plan(m, n, k, room, cu_count());
+  }
+  if (p.splits < 2) return ptb_gemm_bf16(a, b, residual, c, m, n, k, stream);   // one pass
+  if (!a || !b || !c) return PTB_ERR_NULL;
   // B and a tile's rows of A within 32-bit buffer offsets (the plan takes 64-row tiles past K = 2^23)
   if ((k + kRunAhead) * n * 2 >= (int64_t(1) << 32) || int64_t(64) * k * 2 >= (int64_t(1) << 32))
     return PTB_ERR_UNSUPPORTED;
-  if (!aligned16(a) || !aligned16(b) || !aligned16(c) || !aligned16(workspace) || (residual && !aligned16(residual)))
-    return PTB_ERR_ALIGN;
+  if (!aligned16(a) || !aligned16(b) || !aligned16(c) || (residual && !aligned16(residual))) return PTB_ERR_ALIGN;
   hipStream_t s = static_cast<hipStream_t>(stream);
   auto ap = static_cast<const uint16_t*>(a), bp = static_cast<const uint16_t*>(b);
   auto rp = static_cast<const uint16_t*>(residual);
@@ -1243,7 +1276,7 @@ PTB_EXPORT int ptb_gemm_swiglu_bf16(const void* a, const void* b, void* c, int64
   // 256x256 tiles throughout: 1 token of 4096 -> 12288 84 -> 46 us (96 workgroups of which one row is
   // wanted -> 192 of 64x128), 200 tokens 84.5 -> 65 (192 of 256x128), 640 167 -> 130 (128x256), 1024
   // 184 -> 171 (two even rounds of 256x192), 2048 unchanged.
-  const GemmPlan p = gemm_plan(m, n, k, false);
+  const GemmPlan p = gemm_plan(m, n, k, 0);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (p.wm == 4 && p.wn == 4) return launch_swiglu<4, 4>(a, b, c, m, n, k, s);
   if (p.wm == 4 && p.wn == 3) return launch_swiglu<4, 3>(a, b, c, m, n, k, s);

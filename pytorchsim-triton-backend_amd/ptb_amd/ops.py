@@ -207,8 +207,9 @@ def slice_add(x: torch.Tensor, first: int, count: int, s: float, out=None) -> to
 def gemm(a: torch.Tensor, b: torch.Tensor, residual: torch.Tensor | None = None, out=None,
          workspace: torch.Tensor | None = None, split_k: bool = True) -> torch.Tensor:
     """C = A[M,K] @ B[K,N] (+ residual[M,N]), bf16 operands, fp32 accumulation, bf16 C.  Shapes whose
-    output tiles would leave most CUs idle run split-K over a workspace (given, or allocated here);
-    split_k=False forces the single-pass kernel."""
+    output tiles would leave CUs idle run split-K over a workspace (given, or allocated here; a shorter
+    one than ptb_gemm_bf16_workspace_bytes gives fewer slices or a single pass, and is refused only
+    where ptb_gemm_bf16_ws says so); split_k=False forces the single-pass kernel."""
     _need(a, "a", BF16, 2)
     _need(b, "b", BF16, 2)
     m, k = a.shape

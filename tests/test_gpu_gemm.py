@@ -294,6 +294,52 @@ def test_no_split_below_1024(m, k, n):
     assert_close(got, want, RTOL, 2e-2 * float(want.float().abs().mean()), f"no split {m}x{k}x{n}")
 
 
+@pytest.mark.parametrize("m,k,n", [
+    (640, 12288, 4096),   # split in 2 or more, 160 tiles of 128x128
+    (768, 4096, 3072),
+    (2048, 4096, 1024),
+    (385, 4160, 4104),    # ragged
+])
+def test_gemm_ws_takes_the_workspace_there_is(m, k, n):
+    """Where splitting K only gains, any workspace does: none, a misaligned and a one-slice one give the
+    single pass bit for bit, a two-slice one at most two slices, and the bytes past it stay as they
+    were.  Integer operands: every form gives the same bits."""
+    lib = _lib.load()
+    need, slice_ = lib.ptb_gemm_bf16_workspace_bytes(m, n, k), 4 * m * n
+    assert need >= 2 * slice_
+    g = torch.Generator(device=DEV).manual_seed(m)
+    a, b = (torch.randint(-3, 4, s, generator=g, device=DEV).to(torch.bfloat16) for s in ((m, k), (k, n)))
+    want = ops.gemm(a, b, split_k=False)
+    ws = torch.full((need + 64,), 7, dtype=torch.uint8, device=DEV)
+    p, s = ws.data_ptr(), torch.cuda.current_stream().cuda_stream
+    for ptr, size in ((None, 0), (p, 0), (p, slice_), (p + 4, need), (p, 2 * slice_), (p, need)):
+        ws.fill_(7)
+        c = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+        st = lib.ptb_gemm_bf16_ws(a.data_ptr(), b.data_ptr(), None, c.data_ptr(), m, n, k, ptr, size, s)
+        assert st == _lib.PTB_OK, f"workspace of {size} bytes: status {st}"
+        assert torch.equal(c, want), f"workspace of {size} bytes"
+        used = size if ptr == p and size >= 2 * slice_ else 0
+        assert bool((ws[used:] == 7).all()), f"wrote past a workspace of {size} bytes"
+    assert torch.equal(ops.gemm(a, b, workspace=ws[:slice_]), want)
+
+
+def test_gemm_ws_refuses_where_the_slices_are_needed():
+    """Few 64x128 tiles and a long K: no workspace, one too short for their slices and a misaligned one
+    are refused as they always were."""
+    m, k, n = 128, 2048, 128
+    lib = _lib.load()
+    need = lib.ptb_gemm_bf16_workspace_bytes(m, n, k)
+    a = torch.zeros((m, k), dtype=torch.bfloat16, device=DEV)
+    b = torch.zeros((k, n), dtype=torch.bfloat16, device=DEV)
+    c = torch.empty((m, n), dtype=torch.bfloat16, device=DEV)
+    ws = torch.empty(need + 64, dtype=torch.uint8, device=DEV)
+    args, s = (a.data_ptr(), b.data_ptr(), None, c.data_ptr(), m, n, k), torch.cuda.current_stream().cuda_stream
+    assert lib.ptb_gemm_bf16_ws(*args, None, need, s) == _lib.PTB_ERR_NULL
+    assert lib.ptb_gemm_bf16_ws(*args, ws.data_ptr(), 4 * m * n, s) == _lib.PTB_ERR_WORKSPACE
+    assert lib.ptb_gemm_bf16_ws(*args, ws.data_ptr() + 4, need, s) == _lib.PTB_ERR_ALIGN
+    assert lib.ptb_gemm_bf16_ws(*args, ws.data_ptr(), need, s) == _lib.PTB_OK
+
+
 def test_split_k_exact_on_small_integers():
     """Small-integer operands make every partial and sum exact in fp32: split-K equals the oracle bit
     for bit, whatever the slicing."""
