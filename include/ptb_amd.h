@@ -298,6 +298,9 @@ int ptb_gemv_silu_parts_bf16(const float* gate_up_parts, int64_t gate_up_k, cons
  * Replaces: attention_decode_<HQ>x8x<S>_bf16/00__decode_kernel/_decode_kernel_triton.py:4-29 (and
  *           qwen3_8b_layer_decode_1x<S>_bf16/03__decode_kernel). */
 size_t ptb_attn_decode_workspace_bytes(int64_t nkv, int64_t group, int64_t seq);
+/* What such a call runs, for tests and tuning (no GPU work): plan[0..2] = 32-key steps a range and ranges a kv
+ * head (0 and 1 up to 256 keys), 1 if K and V go by the streaming policy (more than 300 MiB of them). */
+int ptb_attn_decode_plan(int64_t nkv, int64_t group, int64_t seq, int32_t* plan);
 int ptb_attn_decode_bf16(const void* q, const void* k, const void* v, void* o, int64_t nkv, int64_t group,
                          int64_t seq, int64_t head_dim, float scale, void* workspace,
                          size_t workspace_bytes, void* stream);

@@ -1013,17 +1013,13 @@ WavePlan wave_plan(int64_t seq) {
   return {int(steps), int((n + steps - 1) / steps)};
 }
 
-// K and V of more than the 256 MB last-level cache, which keeps none of them from one call to the next,
-// go by the streaming policy: 128 kv heads, 8192 keys, G = 4 (537 MB) 102 -> 96 us.  Smaller ones keep the
-// default, under which they may still be cached: 64 kv heads (268 MB), the same caches each call 45.1 us
-// against 48.5 streamed, other caches each call 52.9 against 50.0.
-constexpr int64_t kStreamBytes = int64_t(1) << 28;
+// K and V past kStreamBytes go by the streaming policy.
+bool streams(int64_t nkv, int64_t seq) { return nkv * seq * (2 * kD * 2) > kStreamBytes; }
 
 template <int G>
 void launch_attn_decode_mfma(const uint16_t* q, const uint16_t* k, const uint16_t* v, uint16_t* o, float* part,
                              int nkv, int seq, float c, const WavePlan& p, const QNorm& qn, hipStream_t s) {
-  const auto kernel =
-      int64_t(nkv) * seq * (2 * kD * 2) > kStreamBytes ? attn_decode_mfma<G, true> : attn_decode_mfma<G, false>;
+  const auto kernel = streams(nkv, seq) ? attn_decode_mfma<G, true> : attn_decode_mfma<G, false>;
   kernel<<<dim3(unsigned(p.records), unsigned(nkv)), dim3(64), 0, s>>>(
       q, k, v, o, part, seq, c, p.steps, qn.w, qn.cos, qn.sin, qn.eps);
   if (p.records > 1) attn_decode_merge<G><<<dim3(unsigned(nkv), unsigned(G)), dim3(256), 0, s>>>(part, o, p.records);
@@ -1090,6 +1086,18 @@ PTB_EXPORT int ptb_gemv_silu_parts_bf16(const float* gate_up_parts, int64_t gate
   const GemvSplit gs = gemv_split(gate_up_k, 2 * k);
   return launch_gemv<kSiluParts>(nullptr, nullptr, nullptr, nullptr, 0.f, w, res_a, res_b, y, k, n, workspace,
                                  workspace_bytes, stream, gate_up_parts, gs.splits);
+}
+
+PTB_EXPORT int ptb_attn_decode_plan(int64_t nkv, int64_t group, int64_t seq, int32_t* plan) {
+  if (!plan) return PTB_ERR_NULL;
+  if (nkv <= 0 || group <= 0 || seq <= 0) return PTB_ERR_SHAPE;
+  if (nkv > 65535 || seq >= (int64_t(1) << 30)) return PTB_ERR_GRID;
+  const bool waves = seq > kWaveMinSeq;
+  const WavePlan w = waves ? wave_plan(seq) : WavePlan{0, 1};
+  plan[0] = w.steps;
+  plan[1] = w.records;
+  plan[2] = waves && streams(nkv, seq);
+  return PTB_OK;
 }
 
 PTB_EXPORT size_t ptb_attn_decode_workspace_bytes(int64_t nkv, int64_t group, int64_t seq) {

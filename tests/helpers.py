@@ -3,6 +3,7 @@
 With PTB_REPORT_ERRORS=1 in the environment the checks also print, for checks that pass, the
 largest absolute error and the largest relative error over outputs at least the absolute floor in
 size (run pytest with -s to see them)."""
+import ctypes
 import os
 
 import torch
@@ -23,6 +24,13 @@ def randn(shape, seed, dtype=torch.bfloat16, std=1.0, mean=0.0):
     (validation/pytorchsim/*/..._spec.py:28-36), scaled and cast."""
     g = torch.Generator().manual_seed(seed)
     return (torch.randn(shape, generator=g) * std + mean).to(dtype)
+
+
+def plan(query, *sizes):
+    """What a plan query of the library (ptb_*_plan) says about these sizes: three numbers."""
+    out = (ctypes.c_int32 * 3)()
+    assert query(*sizes, ctypes.addressof(out)) == 0
+    return tuple(out)
 
 
 def rms(t) -> float:

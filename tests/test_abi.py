@@ -7,6 +7,7 @@ from pathlib import Path
 
 import pytest
 
+from helpers import plan
 from ptb_amd import _lib
 
 REPO = Path(__file__).resolve().parents[1]
@@ -110,6 +111,15 @@ def test_32bit_buffer_offset_limits_refused(lib):
     assert lib.ptb_attn_decode_workspace_bytes(1, 4, 1 << 30) == 0
     assert lib.ptb_attn_decode_bf16(P16, P16, P16, P16, 1, 4, 1 << 30, 128, 0.1, P16, 1 << 20, None) == _lib.PTB_ERR_GRID
     assert lib.ptb_attn_decode_workspace_bytes(1, 4, (1 << 30) - 1) > 0
+
+
+def test_streaming_starts_where_the_same_bytes_again_gain(lib):
+    """Caches a little past the last-level cache's 256 MB are still partly found in it by the next call: they keep
+    the default policy up to 300 MiB."""
+    for nkv, seq, streamed in [(64, 8192, 0), (64, 9011, 0), (64, 9600, 0), (64, 9601, 1), (128, 8192, 1), (1, 256, 0)]:
+        assert plan(lib.ptb_attn_decode_plan, nkv, 4, seq)[2] == streamed, (nkv, seq)
+    assert lib.ptb_attn_decode_plan(0, 4, 8192, P16) == _lib.PTB_ERR_SHAPE
+    assert lib.ptb_attn_decode_plan(1, 4, 8192, None) == _lib.PTB_ERR_NULL
 
 
 def test_gemv_parts_refusals(lib):

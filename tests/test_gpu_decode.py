@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import oracle
-from helpers import assert_close, bits_equal, randn
+from helpers import assert_close, bits_equal, plan, randn
 from ptb_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
@@ -154,10 +154,10 @@ def test_attention_decode_fused_qnorm_rope(nkv, g, s):
 
 @pytest.mark.parametrize("g", [1, 2, 3, 4, 6, 8])
 def test_attention_decode_streamed_cache(g):
-    """K and V just past the last-level cache's 256 MB take the streaming policy, the two halves of their heads
-    do not: the same bits, and a head of each end against the oracle."""
-    nkv, s = 70, 7501                            # a last step of 13 keys
-    assert nkv * s * 512 > 1 << 28 >= nkv // 2 * s * 512
+    """K and V just past 300 MiB take the streaming policy, the two halves of their heads do not: the same bits,
+    and a head of each end against the oracle."""
+    nkv, s = 70, 8781                            # a last step of 13 keys
+    assert [plan(_lib.load().ptb_attn_decode_plan, h, g, s)[2] for h in (nkv, nkv - 1, nkv // 2)] == [1, 0, 0]
     r = torch.Generator(device=DEV).manual_seed(g)
     q, k, v = (torch.randn(nkv, n, 128, generator=r, device=DEV).bfloat16() for n in (g, s, s))
     got = ops.attention_decode(q, k, v)
