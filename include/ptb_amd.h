@@ -441,6 +441,10 @@ int ptb_rms_broadcast_bf16(const void* x, const void* a, const float* ss, const 
 int ptb_grouped_gemm_bf16(const void* a, const void* b, const int32_t* group, const int32_t* start,
                           const int32_t* rows, void* c, int64_t nprog, int64_t ntab, int64_t a_rows,
                           int64_t nweights, int64_t k, int64_t n, int64_t weight_stride, void* stream);
+/* What such a call runs, for tests and tuning (no GPU work): plan[0..2] = tile rows, tile
+ * columns, 1 if the weights of groups with one row tile go by the streaming policy; groups = min(nprog, ntab,
+ * nweights). */
+int ptb_grouped_gemm_plan(int64_t groups, int64_t a_rows, int64_t k, int64_t n, int32_t* plan);
 /* The same grouped GEMM with a caller workspace of ptb_grouped_gemm_workspace_bytes(nprog, a_rows,
  * k, n) bytes (16-byte aligned), non-zero when a_rows <= 16: a split-K GEMV pass over each
  * program's weight (every weight row read once per 4 rows of A) and a pass that sums the slices,

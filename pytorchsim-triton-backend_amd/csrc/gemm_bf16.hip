@@ -639,8 +639,8 @@ constexpr int kMaxDedupGroups = 1024;   // group tables up to this size have rep
 // (768 -> 2048) together: 64 routed rows 91 -> 81 us, 512 203 -> 190, 2048 243 -> 226, 4096 273 -> 268,
 // 8192 315 -> 274, 16384 406 -> 320, 32768 617 -> 441.
 // STREAM (see grouped_plan): the weights of a group with one row tile go by the streaming policy.  On
-// another box, with skewed groups, both GEMMs without and with it: 128 routed rows 132 -> 118 us, 512 207 ->
-// 181, 2048 224 -> 201, 4096 239 -> 219, 8192 279 -> 256.
+// another box, with skewed groups, both GEMMs without and with it: 128 routed rows 132 -> 118 us, 256 183 ->
+// 165, 1024 214 -> 188, 4096 239 -> 219, 8192 279 -> 256.
 template <int WM, int WN, int NS, int WGS, bool STREAM>
 __global__ __launch_bounds__(kThreads, WGS) void grouped_gemm_kernel(const uint16_t* __restrict__ A,
                                                                    const uint16_t* __restrict__ B,
@@ -1213,12 +1213,15 @@ struct GroupedPlan {
   int tile;
   bool stream;
 };
-// The weights go by the streaming policy, tile by tile where a group has one row tile, if a group's mean
-// rows fit one and the table's weights are more than the 256 MB last-level cache, which then keeps
-// little of them from one call to the next.  128 experts, gate_up / down: 4 rows each 134.4 -> 119.2 /
-// 72.7 -> 63.1 us, 32 150.9 -> 139.2 / 88.0 -> 80.3, 128 204 -> 202 / 109 -> 104; at 200 rows 255 -> 262
-// / 145 -> 146.  Weights that do fit: 32 experts of 6 MB (201 MB), 4 rows, the same weights each call 31.6
-// -> 35.0, other weights each call 38.8 -> 35.7.
+// The weights go by the streaming policy, tile by tile where a group has one row tile, if
+// - a group's mean rows fit one (128 experts, gate_up / down: 4 rows each 137.0 -> 119.9 / 75.0 -> 65.4 us, 60
+//   156.4 -> 145.0 / 87.9 -> 80.6; at 200 rows 255 -> 262 / 145 -> 146);
+// - the table's weights pass kStreamBytes, so that the groups of the next call are not all in the cache; and
+// - those of the groups expected to be hit pass two thirds of it.  Few of them stay in the cache, up to a block's
+//   two GEMMs in turn: with other rows routed to the same weights each call, 17 rows over 128 experts' gate_up
+//   and down (146 MB of 1.2 GB) 36.9 us either way and by strongly skewed routing 33.4 -> 34.9, with the same
+//   rows 28.3 -> 35.8; 32 rows 54.6 -> 53.2, 45.1 -> 47.0 and 53.1 -> 53.8; past the line 48 rows (gate_up
+//   alone) 78.7 -> 70.9, 96 rows 117.5 -> 107.3, 61.1 -> 60.2 and 125.1 -> 114.0.
 GroupedPlan grouped_plan(int64_t groups, int64_t a_rows, int64_t n, int64_t k, int64_t cus) {
   struct {
     int bm, bn;
@@ -1239,8 +1242,8 @@ GroupedPlan grouped_plan(int64_t groups, int64_t a_rows, int64_t n, int64_t k, i
       best = i;
     }
   }
-  constexpr double kCacheBytes = double(int64_t(1) << 28);
-  return {best, mean <= tiles[best].bm && double(groups) * double(n) * double(k) * 2.0 > kCacheBytes};
+  const double bytes = double(n) * double(k) * 2.0, line = double(kStreamBytes);   // a group's weight
+  return {best, mean <= tiles[best].bm && double(groups) * bytes > line && 1.5 * hit * bytes > line};
 }
 
 // A workgroup for each of the tiles there can be, up to the CUs' WGS each.
@@ -1284,6 +1287,17 @@ PTB_EXPORT int ptb_gemm_swiglu_bf16(const void* a, const void* b, void* c, int64
   if (p.wm == 2 && p.wn == 4) return launch_swiglu<2, 4>(a, b, c, m, n, k, s);
   if (p.wm == 2) return launch_swiglu<2, 2>(a, b, c, m, n, k, s);
   return launch_swiglu<1, 2>(a, b, c, m, n, k, s);
+}
+
+PTB_EXPORT int ptb_grouped_gemm_plan(int64_t groups, int64_t a_rows, int64_t k, int64_t n, int32_t* plan) {
+  if (!plan) return PTB_ERR_NULL;
+  if (groups <= 0 || a_rows <= 0 || k <= 0 || n <= 0 || a_rows > 0x7fffffff || k > 0x7fffffff || n > 0x7fffffff)
+    return PTB_ERR_SHAPE;
+  const GroupedPlan p = grouped_plan(groups, a_rows, n, k, cu_count());
+  plan[0] = p.tile == 2 ? 64 : 128;
+  plan[1] = p.tile == 0 ? 256 : 128;
+  plan[2] = p.stream;
+  return PTB_OK;
 }
 
 PTB_EXPORT int ptb_grouped_gemm_bf16(const void* a, const void* b, const int32_t* group, const int32_t* start,

@@ -19,9 +19,10 @@ constexpr int kWave = 64;
 // Operands read once a launch go by the streaming policy (the nt bit) past this many bytes.  The last-level
 // cache holds 256 MB, and keeps enough of a read a little longer for the next call on the same bytes: decode
 // attention of 285 MB (64 kv heads, G = 4) 48.4 us by default and 52.1 streamed, 306 MB 56.7 / 56.4, 317 MB
-// 60.3 / 57.6, 336 MB 64.1 / 60.8, 537 MB 101.4 / 95.9.  So streaming starts where the same bytes in every call
-// gain as well.  Other bytes in every call gain below it too (285 MB 56.8 / 53.0), but a launch does not know
-// which of the two it is.
+// 60.3 / 57.6, 336 MB 64.1 / 60.8, 537 MB 101.4 / 95.9; the expert weights of a grouped GEMM at 277 MB 55.5 /
+// 58.0, 302 MB 62.4 / 60.4, 315 MB 66.1 / 61.8, 403 MB 74.4 / 66.1.  So streaming starts where the same bytes
+// in every call gain as well.  Other bytes in every call gain below it too (285 MB 56.8 / 53.0, 226 MB of
+// weights 43.5 / 39.0), but a launch does not know which of the two it is.
 constexpr int64_t kStreamBytes = int64_t(300) << 20;
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;

@@ -6,8 +6,8 @@ import pytest
 import torch
 
 import oracle
-from helpers import assert_close, bits_equal
-from ptb_amd import moe
+from helpers import assert_close, bits_equal, plan
+from ptb_amd import _lib, moe
 
 pytestmark = pytest.mark.gpu
 
@@ -422,17 +422,19 @@ def test_grouped_gemm_walk(groups, n, k_dim, div):
     assert torch.equal(got[gaps], c0.reshape(a_rows, n)[gaps])
 
 
-@pytest.mark.parametrize("groups,n,k_dim,sizes", [
-    (72, 1024, 2048, [0, 1, 3, 16, 63, 64, 65, 2]), (72, 1024, 2048, [0, 127, 64, 128, 65, 129, 33, 1]),
-    (72, 1024, 2048, [0, 257, 127, 128, 129, 65, 64, 1]), (130, 1096, 1024, [5, 64, 0, 63, 65, 40, 129, 2]),
+@pytest.mark.parametrize("groups,n,k_dim,sizes,tile", [
+    (88, 1024, 2048, [0, 1, 3, 16, 63, 64, 65, 2], (64, 128)),
+    (164, 1096, 1024, [0, 127, 64, 128, 65, 129, 33, 1], (128, 128)),
+    (88, 1024, 2048, [0, 257, 127, 128, 129, 65, 64, 1], (128, 256)),
+    (164, 1096, 1024, [5, 64, 0, 63, 65, 40, 129, 2], (64, 128)),
 ])
-def test_grouped_gemm_streamed_weights(groups, n, k_dim, sizes):
-    """Weights of more than the last-level cache's 256 MB, which groups of one row tile read by the streaming
-    policy and groups of two or three as usual, both in one walk, for each of the three tiles."""
-    assert groups * n * k_dim * 2 > 1 << 28
+def test_grouped_gemm_streamed_weights(groups, n, k_dim, sizes, tile):
+    """Weights of more than 300 MiB, which groups of one row tile read by the streaming policy and groups of two or
+    three as usual, both in one walk, for each of the three tiles."""
     rows = torch.tensor(sizes, dtype=I32)[(torch.arange(groups) * 5 + 3) % 8]
     starts = torch.cumsum(rows, 0).to(I32) - rows
     a_rows = int(rows.sum())
+    assert plan(_lib.load().ptb_grouped_gemm_plan, groups, a_rows, k_dim, n) == (*tile, 1)
     g = torch.Generator(device=DEV).manual_seed(44)
     a = (torch.randn(a_rows, k_dim, generator=g, device=DEV) / 8).to(BF16)
     b = (torch.randn(groups, k_dim, n, generator=g, device=DEV) / 8).to(BF16)
