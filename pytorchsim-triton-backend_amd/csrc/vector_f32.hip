@@ -220,7 +220,8 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_range(const float* p, int
 __device__ __forceinline__ float buffer_f32(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
 }
-// WIDE: byte offsets within a workgroup's rows of x or a slab of the weights may pass 2^32.
+// WIDE: byte offsets within a workgroup's rows of x or a slab of the weights may pass 2^32.  Its column blocks
+// run over the grid's x and z: a launch takes fewer than 2^32 threads along x.
 template <int WR, int WK, int KW, bool WIDE>
 __global__ __launch_bounds__(64 * WR * WK) void swiglu_f32(
     const float* __restrict__ x, const float* __restrict__ wg, const float* __restrict__ wu, float* __restrict__ o,
@@ -230,7 +231,10 @@ __global__ __launch_bounds__(64 * WR * WK) void swiglu_f32(
   __shared__ __attribute__((aligned(16))) float smem[Sh::kSmem];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wk = wave % WK, wr = wave / WK;
-  const int m0 = int(blockIdx.y) * Sh::BM, n0 = int(blockIdx.x) * Sh::BN;
+  const int m0 = int(blockIdx.y) * Sh::BM;
+  const int64_t nblock = WIDE ? int64_t(blockIdx.z) * gridDim.x + blockIdx.x : blockIdx.x;
+  if (WIDE && nblock * Sh::BN >= N) return;   // uniform over the workgroup
+  const int n0 = int(nblock * Sh::BN);
   const int col = lane & 31, h = lane >> 5;
 
   // Loads: thread -> k ka of rows ra0, ra0 + kThreads / KS, ... of x; column cb of rows kb0, kb0 +
@@ -356,9 +360,10 @@ int launch_swiglu_f32(const float* x, const float* wg, const float* wu, float* o
                       hipStream_t s) {
   using Sh = SwShape<WR, WK, KW>;
   const int64_t gx = (n + Sh::BN - 1) / Sh::BN, gy = (m + Sh::BM - 1) / Sh::BM;
-  if (gx > 0x7fffffff || gy > 65535) return PTB_ERR_GRID;
-  swiglu_f32<WR, WK, KW, WIDE><<<dim3(unsigned(gx), unsigned(gy)), dim3(Sh::kThreads), 0, s>>>(x, wg, wu, o, int(m),
-                                                                                            int(n), int(k));
+  if (gy > 65535) return PTB_ERR_GRID;
+  const int64_t bx = WIDE ? std::min<int64_t>(gx, 1 << 22) : gx;
+  swiglu_f32<WR, WK, KW, WIDE><<<dim3(unsigned(bx), unsigned(gy), unsigned((gx + bx - 1) / bx)), dim3(Sh::kThreads), 0,
+                                 s>>>(x, wg, wu, o, int(m), int(n), int(k));
   return launch_status();
 }
 

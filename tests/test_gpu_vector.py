@@ -260,6 +260,32 @@ def test_swiglu_f32_ragged(m, n, k):
 
 
 @pytest.mark.parametrize("m,n,k", [
+    (66, (1 << 24) + 17, 33),   # two row blocks, a slab and a tail of one k
+    (2, 1, (1 << 24) + 5),      # one output column, repeated 32 times in the block; a tail of five k
+    (1, (1 << 29) + 33, 1),     # column blocks past 2^32 threads along x
+])
+def test_swiglu_f32_wide(m, n, k):
+    """Sizes past 2^24, whose offsets take 64 bits.  Operands in {-1, 0, 1} and {-2 .. 2} / 1024 keep every partial
+    sum exact in fp32 (at most 2^25 of 2^-10 each), so only the gate's exponential, sum, quotient and product round,
+    within (|g| + 4) 2^-23 of the exact value; the exponential's own underflow, where |g| > 87, is 2^-126 of it.
+    First, last and middle columns are checked, and that every output is written."""
+    g = torch.Generator(device=DEV).manual_seed(m + k)
+    x = torch.randint(-1, 2, (m, k), generator=g, device=DEV).float()
+    wg, wu = (torch.randint(-2, 3, (k, n), generator=g, device=DEV, dtype=torch.int8).float().div_(1024) for _ in range(2))
+    guard = torch.full((m * n + 4096,), float("nan"), device=DEV)
+    o = guard[: m * n].view(m, n)
+    ops.swiglu_f32(x, wg, wu, out=o)
+    assert bool(guard[m * n:].isnan().all()), "the kernel wrote past o"
+    assert not any(bool(row.isnan().any()) for row in o.view(-1).split(1 << 28))
+    for c0 in sorted({0, max(0, n // 2 - 512), max(0, min(n, 1 << 27) - 1024), max(0, n - 1024)}):
+        cols = slice(c0, min(c0 + 1024, n))
+        gate, up = (x.cpu().double() @ w[:, cols].cpu().double() for w in (wg, wu))
+        want = gate / (1 + torch.exp(-gate)) * up
+        bound = (gate.abs() + 4) * 2.0 ** -23 * want.abs() + 2.0 ** -126 * up.abs()
+        assert bool(((o[:, cols].cpu().double() - want).abs() <= bound).all()), f"columns from {c0}"
+
+
+@pytest.mark.parametrize("m,n,k", [
     (1, 1, 1),            # one output, a tail of one k
     (33, 65, 64),         # eight waves a 32x32 block: one whole slab, ragged blocks
     (5, 31, 257),         # four slabs and a tail of one
