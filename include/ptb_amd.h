@@ -170,6 +170,9 @@ int ptb_gemm_bf16(const void* a, const void* b, const void* residual, void* c, i
  * misaligned (PTB_ERR_ALIGN).
  * Replaces: the same kernels as ptb_gemm_bf16 (the small M x N gemm_<M>x<K>x<N>_bf16 shapes). */
 size_t ptb_gemm_bf16_workspace_bytes(int64_t m, int64_t n, int64_t k);
+/* What such a call runs, for tests and tuning (no GPU work): plan[0..2] = tile rows, tile columns, K slices.
+ * split: with the workspace above; 0: ptb_gemm_bf16, and (n = 2 * inter) ptb_gemm_swiglu_bf16. */
+int ptb_gemm_bf16_plan(int64_t m, int64_t n, int64_t k, int split, int32_t* plan);
 int ptb_gemm_bf16_ws(const void* a, const void* b, const void* residual, void* c, int64_t m, int64_t n, int64_t k,
                      void* workspace, size_t workspace_bytes, void* stream);
 
@@ -210,6 +213,9 @@ int ptb_gemm_fp8_scaled(const void* aq, const float* sa, const void* wq_t, const
  * split; then ptb_gemm_fp8_scaled_ws is ptb_gemm_fp8_scaled and takes a NULL workspace.  A split shape
  * refuses a NULL workspace (PTB_ERR_NULL) or one shorter than that (PTB_ERR_WORKSPACE). */
 size_t ptb_gemm_fp8_workspace_bytes(int64_t m, int64_t n, int64_t k);
+/* What such a call runs, for tests and tuning (no GPU work): plan[0..2] = tile rows (0: the few-row kernel), tile
+ * columns, K slices.  split: with the workspace above; 0: ptb_gemm_fp8_scaled. */
+int ptb_gemm_fp8_plan(int64_t m, int64_t n, int64_t k, int split, int32_t* plan);
 int ptb_gemm_fp8_scaled_ws(const void* aq, const float* sa, const void* wq_t, const float* sw, void* c, int64_t m,
                            int64_t n, int64_t k, void* workspace, size_t workspace_bytes, void* stream);
 

@@ -1149,6 +1149,16 @@ size_t plan_workspace(const GemmPlan& p, int64_t m, int64_t n) {
 
 }  // namespace
 
+PTB_EXPORT int ptb_gemm_bf16_plan(int64_t m, int64_t n, int64_t k, int split, int32_t* plan) {
+  if (!plan) return PTB_ERR_NULL;
+  if (m <= 0 || n <= 0 || k <= 0 || m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff) return PTB_ERR_SHAPE;
+  const GemmPlan p = gemm_plan(m, n, k, split ? kAnyRoom : 0);
+  plan[0] = 64 * p.wm;
+  plan[1] = 64 * p.wn;
+  plan[2] = p.splits;
+  return PTB_OK;
+}
+
 PTB_EXPORT size_t ptb_gemm_bf16_workspace_bytes(int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || n <= 0 || k <= 0 || m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff) return 0;
   return plan_workspace(gemm_plan(m, n, k, kAnyRoom), m, n);

@@ -957,6 +957,16 @@ PTB_EXPORT int ptb_gemm_fp8_scaled(const void* aq, const float* sa, const void* 
   return launch_fp8_plan(fp8_plan(m, n, k, false), g, nullptr, static_cast<hipStream_t>(stream));
 }
 
+PTB_EXPORT int ptb_gemm_fp8_plan(int64_t m, int64_t n, int64_t k, int split, int32_t* plan) {
+  if (!plan) return PTB_ERR_NULL;
+  if (m <= 0 || n <= 0 || k <= 0 || m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff) return PTB_ERR_SHAPE;
+  const Fp8Plan p = fp8_plan(m, n, k, split != 0);
+  plan[0] = p.bm;
+  plan[1] = p.bn;
+  plan[2] = p.splits;
+  return PTB_OK;
+}
+
 PTB_EXPORT size_t ptb_gemm_fp8_workspace_bytes(int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || n <= 0 || k <= 0 || m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff) return 0;
   return fp8_workspace(fp8_plan(m, n, k, true), m, n);

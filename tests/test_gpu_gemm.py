@@ -12,13 +12,23 @@ import pytest
 import torch
 
 import oracle
-from helpers import assert_close, bits_equal, randn, rms
+from helpers import assert_close, bits_equal, plan, randn, rms
 from ptb_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda"
 RTOL = ATOL = 2e-2
+
+
+def gemm_plan(m, k, n, split=1):
+    """(tile rows, tile columns, K slices) of ops.gemm, or (split = 0) of one pass over K."""
+    return plan(_lib.load().ptb_gemm_bf16_plan, m, n, k, split)
+
+
+def fp8_plan(m, k, n):
+    """The same of ops.gemm_fp8; tile rows 0: the few-row kernel."""
+    return plan(_lib.load().ptb_gemm_fp8_plan, m, n, k, 1)
 
 
 def sample_rows(m, seed=0):
@@ -85,15 +95,20 @@ def test_gemm_ragged_residual_stays_inside_c(m, k, n):
     assert_close(c.cpu()[rows], oracle.gemm(a[rows], b, r[rows]), RTOL, ATOL, f"gemm+R {m}x{k}x{n}")
 
 
-@pytest.mark.parametrize("m,k,n", [
+WALKS = [
     (4096, 4096, 12288),   # three rounds of 256x256 tiles
-    (4300, 256, 8248),     # 561 tiles, ragged in M and N: some workgroups walk three tiles, most two
-])
+    (4100, 256, 8648),     # 578 tiles, ragged in M and N: 66 workgroups walk three tiles, the others two
+    (4300, 256, 12344),    # 833 tiles: 65 workgroups walk four, the others three
+]
+
+
+@pytest.mark.parametrize("m,k,n", WALKS)
 def test_gemm_persistent_walk_is_the_tile_by_tile_product(m, k, n):
     """Two or more rounds of 256x256 tiles run as one workgroup per CU walking its tiles, the next
     tile's first stage loading during the current tile's epilogue.  Every tile keeps its MFMA order
     over K, so each 256-row band equals the product of that band of A alone (a one-round shape,
     other tiles) bit for bit; the sampled rows against the oracle, and nothing written past C."""
+    assert gemm_plan(m, k, n) == (256, 256, 1) and -(-m // 256) * -(-n // 256) >= 2 * 256
     a = randn((m, k), 8, std=1.0 / 64)
     b = randn((k, n), 9, std=1.0 / 64)
     guard = torch.full((m * n + 8192,), float("nan"), dtype=torch.bfloat16, device=DEV)
@@ -119,26 +134,33 @@ def test_gemm_bundle_inputs_exact_products():
     assert bits_equal(c, oracle.gemm(a, b))
 
 
-@pytest.mark.parametrize("m,k,n,resid", [
-    (1308, 64, 5408, True),       # 128x256 tiles, one K step: every stage past the first runs past K
-    (1893, 128, 4176, False),     # 128x256 tiles, ragged in M and N, 255 tiles (not a multiple of 8)
-    (1849, 512, 4152, True),      # the same, eight steps of the three-step loop
-    (2357, 64, 792, False),       # 128x128 tiles, one step of the four-step loop
-    (1491, 320, 1896, True),      # 128x128 tiles, five steps: a remainder of one
-    (1, 640, 4512, False),        # 64x128 tiles, one row, ten steps: a remainder of two
-    (110, 896, 56, True),         # 64x128 tiles, one ragged column tile
-    (9, 2304, 8, True),           # 64x128 tiles split 8 ways, a single tile
-    (355, 1216, 16, False),       # split 7 ways, the last slice a step shorter
-    (72, 1792, 5480, True),       # 128x128 tiles split 4 ways, ragged
-    (385, 4160, 4104, True),      # 256x128 tiles split
-    (262, 4416, 3744, False),     # 128x256 tiles split 5 ways, 45 tiles a slice
-    (387, 7104, 5592, True),      # 256x256 tiles split 5 ways, 44 tiles a slice
-])
-def test_gemm_planned_tiles_stay_inside_c(m, k, n, resid):
+PLANNED = [
+    (1308, 64, 5408, True, (128, 256, 1)),     # one K step: every stage past the first runs past K
+    (1893, 128, 4176, False, (128, 256, 1)),   # ragged in M and N, 255 tiles (not a multiple of 8)
+    (1849, 512, 4152, True, (128, 256, 1)),    # eight steps of the three-step loop
+    (2357, 64, 792, False, (128, 128, 1)),     # one step of the four-step loop
+    (1491, 320, 1896, True, (128, 128, 1)),    # five steps: a remainder of one
+    (1, 640, 4512, False, (64, 128, 1)),       # one row, ten steps: a remainder of two
+    (110, 896, 56, True, (64, 128, 1)),        # one ragged column tile
+    (9, 2304, 8, True, (64, 128, 8)),          # a single tile
+    (355, 1216, 16, False, (64, 128, 7)),      # the last slice a step shorter
+    (5, 1088, 8, True, (64, 128, 6)),          # slices of three steps, the last of two
+    (72, 1792, 5480, True, (128, 128, 4)),     # ragged
+    (385, 4160, 4104, True, (256, 128, 3)),    # the last slice a step shorter
+    (387, 7104, 5592, True, (256, 128, 2)),    # 88 tiles a slice, the last one a step shorter
+    (262, 4416, 3744, False, (128, 256, 5)),   # 45 tiles a slice
+    (482, 10304, 5408, True, (256, 256, 5)),   # 44 tiles a slice, the last slice four steps shorter
+    (1054, 6144, 4088, False, (256, 256, 3)),  # 80 tiles a slice, ragged in M and N
+]
+
+
+@pytest.mark.parametrize("m,k,n,resid,tiles", PLANNED)
+def test_gemm_planned_tiles_stay_inside_c(m, k, n, resid, tiles):
     """Every tile shape and split of the plan at ragged sizes, step counts around the loops' turns and
     tile counts that do not divide by the XCDs: small-integer operands make every partial sum exact in
     fp32 (|sum| <= 9 * 12288 + 9 < 2^24), so the result is the oracle's bit for bit whatever the tiling,
     and a NaN-filled guard after C's last element stays NaN."""
+    assert gemm_plan(m, k, n) == tiles
     g = torch.Generator().manual_seed(m + n)
     a = torch.randint(-3, 4, (m, k), generator=g).to(torch.bfloat16)
     b = torch.randint(-3, 4, (k, n), generator=g).to(torch.bfloat16)
@@ -203,30 +225,39 @@ def test_gemm_fp8(m, k, n):
     assert_close(c[rows], want, RTOL, ATOL * scale, f"gemm_fp8 {m}x{k}x{n}")
 
 
-@pytest.mark.parametrize("m,k,n", [
-    (1, 128, 16),        # few rows: one step, seven waves idle
-    (16, 1024, 528),     # a step a wave
-    (7, 7296, 112),      # 57 steps: a whole batch of 6 a wave, then 9 more steps
-    (17, 4480, 80),      # two blocks of 16 rows, 35 steps
-    (32, 256, 848),
-    (33, 128, 64),       # 64x128 tiles, one step: three stages past K
-    (205, 384, 224),     # three steps, ragged in M and N
-    (419, 640, 32),      # five steps of the four-step loop
-    (40, 4224, 16),      # split 7 ways, one ragged tile
-    (67, 2176, 2368),    # split 3 ways, the last slice a step shorter
-    (398, 128, 4640),    # 128x128 tiles
-    (601, 384, 3488),
-    (463, 5120, 2112),   # 128x128 tiles split
-    (1026, 512, 3632),   # 256x128 tiles, an odd tile count for the XCDs
-    (397, 11008, 4112),  # 256x128 tiles split
-    (644, 8704, 5392),   # 256x256 tiles split
-    (1747, 1664, 4640),  # 256x256 tiles
-])
-def test_gemm_fp8_planned_tiles_stay_inside_c(m, k, n):
+FP8_PLANNED = [
+    (1, 128, 16, (0, 16, 1)),            # few rows: one step, seven waves idle
+    (16, 1024, 528, (0, 16, 1)),         # a step a wave
+    (1, 5248, 736, (0, 16, 1)),          # 41 steps: wave 0 takes a whole batch of six, the others single steps
+    (3, 5760, 1008, (0, 16, 1)),         # 45 steps: waves 0 to 4 a batch, the others single steps
+    (16, 6144, 2048, (0, 16, 1)),        # 48 steps: a batch a wave and nothing left
+    (17, 4480, 80, (0, 16, 1)),          # two blocks of 16 rows, 35 steps: batches of four, then single steps
+    (32, 5120, 1024, (0, 16, 1)),        # 40 steps: a batch of four and a single step a wave
+    (32, 256, 848, (0, 16, 1)),
+    (7, 7296, 112, (64, 128, 8)),        # 57 steps, the last slice a step of the others' eight
+    (33, 128, 64, (64, 128, 1)),         # one step: three stages past K
+    (205, 384, 224, (64, 128, 1)),       # three steps, ragged in M and N
+    (419, 640, 32, (64, 128, 1)),        # five steps of the four-step loop
+    (33, 1408, 16, (64, 128, 6)),        # slices of two steps, the last of one
+    (40, 4224, 16, (64, 128, 7)),        # one ragged tile
+    (67, 2176, 2368, (64, 128, 3)),      # the last slice a step shorter
+    (398, 128, 4640, (128, 128, 1)),
+    (601, 384, 3488, (128, 128, 1)),
+    (463, 5120, 2112, (128, 128, 3)),
+    (1026, 512, 3632, (256, 128, 1)),    # an odd tile count for the XCDs
+    (397, 11008, 4112, (256, 128, 3)),
+    (644, 8704, 5392, (256, 256, 3)),
+    (1747, 1664, 4640, (256, 256, 1)),
+]
+
+
+@pytest.mark.parametrize("m,k,n,tiles", FP8_PLANNED)
+def test_gemm_fp8_planned_tiles_stay_inside_c(m, k, n, tiles):
     """Every tile shape and split of the fp8 plan and the few-row kernel at ragged sizes and around
     their loops' step counts: small integers (exact in e4m3) and powers of two as scales make every sum
     exact in fp32 (|sum| <= 9 * 12288 < 2^24), so the result is the oracle's bit for bit; a NaN-filled
     guard after C's last element stays NaN."""
+    assert fp8_plan(m, k, n) == tiles
     g = torch.Generator().manual_seed(m + n)
     a = torch.randint(-3, 4, (m, k), generator=g).float().to(torch.float8_e4m3fn)
     w = torch.randint(-3, 4, (n, k), generator=g).float().to(torch.float8_e4m3fn)
@@ -351,19 +382,26 @@ def test_split_k_exact_on_small_integers():
     assert bits_equal(got, oracle.gemm(a, b))
 
 
-@pytest.mark.parametrize("m,k,n,resid", [(2048, 768, 768, False), (1000, 768, 264, True), (768, 3072, 1024, False),
-                                         (4000, 384, 512, True), (2048, 4096, 1024, True)])
-def test_gemm_64x128_tiles(m, k, n, resid):
-    """Mid-size shapes whose 128x128 tiles cover less than 3/4 of the CUs run 64x128 tiles (K split
-    when the plan's cost model says so: 768x3072x1024)."""
+MID_SIZES = [
+    (2048, 768, 768, False, (64, 128, 1)), (1000, 768, 264, True, (64, 128, 1)), (4000, 384, 512, True, (64, 128, 1)),
+    (768, 3072, 1024, False, (128, 128, 4)), (2048, 4096, 1024, True, (128, 128, 2)),
+]
+
+
+@pytest.mark.parametrize("m,k,n,resid,tiles", MID_SIZES)
+def test_gemm_mid_sizes(m, k, n, resid, tiles):
+    """Mid-size shapes whose 128x128 tiles cover less than 3/4 of the CUs: 64x128 tiles in one pass, or K
+    slices of 128x128 ones."""
+    assert gemm_plan(m, k, n) == tiles
     c, want = run_gemm(m, k, n, 41, 1 / 32, 1 / 16, resid)
-    assert_close(c, want, RTOL, 2e-2 * float(want.float().abs().mean()), f"64x128 {m}x{k}x{n}")
+    assert_close(c, want, RTOL, 2e-2 * float(want.float().abs().mean()), f"mid size {m}x{k}x{n}")
 
 
 @pytest.mark.parametrize("m,k,n,resid", [(6144, 1024, 1024, False), (6000, 768, 1000, True)])
 def test_gemm_256x128_tiles_from_three_quarters(m, k, n, resid):
     """256x128 tiles that cover 3/4 of the CUs or more run as one round of them (192 tiles here),
     ragged rows and columns included."""
+    assert gemm_plan(m, k, n) == (256, 128, 1)
     c, want = run_gemm(m, k, n, 43, 1 / 32, 1 / 16, resid)
     assert_close(c, want, RTOL, 2e-2 * float(want.float().abs().mean()), f"256x128 {m}x{k}x{n}")
 
@@ -401,18 +439,23 @@ def test_gemm_odd_step_count(m, k, n, resid):
     assert_close(got, want, RTOL, ATOL * rms(want), f"gemm {m}x{k}x{n}")
 
 
-@pytest.mark.parametrize("m,k,inter", [
-    (1, 64, 128),         # 64x128 tiles, one row, one step
-    (130, 320, 256),      # 64x128 tiles, five steps
-    (129, 320, 5504),     # 128x128 tiles, the second row tile one row
-    (1669, 320, 1280),    # 256x128 tiles
-    (515, 320, 5632),     # 128x256 tiles, the last row tile three rows
-    (2047, 448, 2176),    # 256x192 tiles (96 outputs each): the last one covers 64 of its 96
-    (2500, 192, 3200),    # 256x256 tiles
-])
-def test_gemm_swiglu_every_tile(m, k, inter):
+SWIGLU_TILES = [
+    (1, 64, 128, (64, 128)),         # one row, one step
+    (130, 320, 256, (64, 128)),      # five steps
+    (129, 320, 5504, (128, 128)),    # the second row tile one row
+    (1669, 320, 1280, (256, 128)),
+    (515, 320, 5632, (128, 256)),    # the last row tile three rows
+    (2047, 448, 2176, (256, 192)),   # tiles of 96 outputs: the last one covers 64 of its 96
+    (2500, 192, 3200, (256, 256)),
+    (768, 4096, 1536, (128, 128)),   # a size that ops.gemm splits in K
+]
+
+
+@pytest.mark.parametrize("m,k,inter,tile", SWIGLU_TILES)
+def test_gemm_swiglu_every_tile(m, k, inter, tile):
     """The SwiGLU epilogue of every tile shape of the plan, ragged in M and (256x192) in the outputs:
-    bit for bit the GEMM followed by silu_mul, and nothing past C."""
+    bit for bit the one-pass GEMM followed by silu_mul, and nothing past C."""
+    assert gemm_plan(m, k, 2 * inter, split=0) == (*tile, 1)
     a = randn((m, k), 61, std=1 / 16).to(DEV)
     b = randn((k, 2 * inter), 62, std=1 / 4).to(DEV)
     guard = torch.full((m * inter + 8192,), float("nan"), dtype=torch.bfloat16, device=DEV)
