@@ -66,7 +66,8 @@ typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 // to 39 us (1024x4096x4096).  Stage kt + DIST, DIST = NSA - 1 = 2 or 3, refills the slots of stage kt-1, which the barrier of step
 // kt-1 freed, so the stage's DMAs spread over all of step kt's MFMAs; with two B slots, its B part
 // waits for the barrier of step kt and spreads over the slice after it.
-template <int WM, int WN>
+// RING: NSA; 64x128 and 128x128 tiles also come in rings of 3 for short K ranges (see make_plan).
+template <int WM, int WN, int RING = (WM * WN >= 8 ? 3 : 4)>
 struct Shape {
   static constexpr int BK = 64;
   // A and B live in rings of their own: NSA and NSB slots.  256x256 and 256x192 tiles with 64-deep
@@ -74,7 +75,7 @@ struct Shape {
   // refills a slot only after the barrier that frees it (the "hybrid" schedule below); every other
   // ring is one slot deeper than its DMA distance.
   static constexpr bool kHybrid = WM * WN >= 12;
-  static constexpr int NSA = WM * WN >= 8 ? 3 : 4;
+  static constexpr int NSA = RING;
   static constexpr int NSB = kHybrid ? 2 : NSA;
   static constexpr int NS = NSA;
   static constexpr int DIST = NSA - 1;
@@ -134,16 +135,20 @@ __device__ __forceinline__ int swiglu_staged(int wn, int j, int n) {
 // swiglu_staged), and the epilogue stores bf16(silu(bf16(gate)) * bf16(up)), as a separate silu_mul
 // would compute it from the bf16 GEMM.
 enum { kPlain = 0, kSplit = 1, kSwiGLU = 2 };
+// Up to this many outputs the partials of 64x128 tiles leave straight from the accumulators, without the barrier
+// and the LDS pass: 348x2048x40 5.69 -> 5.42 us, 3x2816x8 5.54 -> 5.23, 544x1600x48 6.02 -> 5.78.  Past it whole
+// rows a store instruction are worth them: 1024x2048x128 7.74 us staged, 8.09 direct; 193x3008x576 7.51 / 7.84.
+constexpr int64_t kDirectPartials = 32768;
 
 
 // PERSIST (plain 256x256 tiles, no residual): one workgroup per CU walks the tiles
 // blockIdx.x, blockIdx.x + gridDim.x, ...; the next tile's first stage goes out halfway through the
 // current tile's epilogue, so its latency hides behind the stores (see the epilogue).
-template <int WM, int WN, bool RESID, int MODE, bool PERSIST = false>
+template <int WM, int WN, bool RESID, int MODE, bool PERSIST = false, int RING = Shape<WM, WN>::NSA>
 __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_kernel(
     const uint16_t* __restrict__ A_in, const uint16_t* __restrict__ B_in, const uint16_t* __restrict__ R,
     uint16_t* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n, float* __restrict__ part, int kchunk) {
-  using Sh = Shape<WM, WN>;
+  using Sh = Shape<WM, WN, RING>;
   constexpr int BM = Sh::BM, BN = Sh::BN, kABytes = Sh::kABytes;
   constexpr int BK = Sh::BK, NS = Sh::NS, DIST = Sh::DIST, NSA = Sh::NSA, NSB = Sh::NSB;
   constexpr bool kHybrid = Sh::kHybrid;
@@ -457,7 +462,8 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
   // residual is read the same way.  The region is the wave's own and LDS operations of a wave
   // complete in order, so no barrier separates its writes from its reads.  Rows past M and columns
   // past `cols` fall outside the buffer resources (stores dropped, loads 0): no branches.
-  __syncthreads();
+  const bool direct = MODE == kSplit && WM == 1 && int64_t(M) * N <= kDirectPartials;
+  if (!direct) __syncthreads();
   auto store_staged = [&](auto ng, auto value, uint16_t* out, int ldc, int cols, int col0) __attribute__((always_inline)) {
     constexpr int NG = decltype(ng)::value;
     constexpr int WC = NG * 8;            // columns of a wave's block
@@ -542,7 +548,21 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
       }
     }
   };
-  if constexpr (MODE == kSplit) {
+  if (direct) {
+#pragma unroll
+    for (int i = 0; i < WM; ++i) {
+      const int row = m0 + wm * (BM / 2) + i * 32 + fr;
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int col = n0 + wn * (BN / 2) + j * 32 + 8 * g + 4 * h;
+          if (row < M && col < N)   // N % 8 == 0: a 4-column group is all in or all out
+            *reinterpret_cast<f32x4v*>(part + int64_t(slice) * M * N + int64_t(row) * N + col) =
+                f32x4v{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+        }
+    }
+  } else if constexpr (MODE == kSplit) {
     // the slice's fp32 partial sums, staged the same way: whole rows of WN * 128 bytes a store
     // instruction (16 bytes into each of 32 rows straight from the accumulators)
     constexpr int WC = WN * 32, kPitch = WC * 4 + 16, LPR = WC / 4, RPI = 64 / LPR;
@@ -930,10 +950,10 @@ __global__ __launch_bounds__(kThreads, WGS) void grouped_gemm_kernel(const uint1
 
 int cu_count();
 
-template <int WM, int WN>
+template <int WM, int WN, int RING = Shape<WM, WN>::NSA>
 int launch_gemm(const void* a, const void* b, const void* residual, void* c, int64_t m, int64_t n, int64_t k,
                 hipStream_t s) {
-  using Sh = Shape<WM, WN>;
+  using Sh = Shape<WM, WN, RING>;
   const int64_t tm = (m + Sh::BM - 1) / Sh::BM, tn = (n + Sh::BN - 1) / Sh::BN;
   if (tm * tn > 0x7fffffff) return PTB_ERR_GRID;
   const dim3 grid(unsigned(tm * tn)), block(kThreads);
@@ -948,11 +968,11 @@ int launch_gemm(const void* a, const void* b, const void* residual, void* c, int
     }
   }
   if (residual)
-    gemm_bf16_kernel<WM, WN, true, kPlain><<<grid, block, 0, s>>>(
+    gemm_bf16_kernel<WM, WN, true, kPlain, false, RING><<<grid, block, 0, s>>>(
         static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), static_cast<const uint16_t*>(residual),
         static_cast<uint16_t*>(c), int(m), int(n), int(k), int(tm), int(tn), nullptr, 0);
   else
-    gemm_bf16_kernel<WM, WN, false, kPlain><<<grid, block, 0, s>>>(
+    gemm_bf16_kernel<WM, WN, false, kPlain, false, RING><<<grid, block, 0, s>>>(
         static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), nullptr, static_cast<uint16_t*>(c), int(m),
         int(n), int(k), int(tm), int(tn), nullptr, 0);
   return launch_status();
@@ -968,6 +988,7 @@ int cu_count() {
 struct GemmPlan {
   int wm, wn, splits;
   int64_t kchunk;   // K columns per split
+  int ring;         // slots of the ring (chosen for 64x128 and 128x128 tiles, given by the others' shape)
 };
 
 // Cost model of a plan, in us.  A round of workgroups (one a CU) costs `step` per 64-deep K step
@@ -1006,7 +1027,7 @@ GemmPlan make_plan(int64_t m, int64_t n, int64_t k, size_t room, int64_t cus) {
   const double mem = kMemUs + kMemUsPerMB * 2e-6 * (double(k) * double(n) + double(m) * (double(k) + double(n)));
   const double partial = kPartialUsPerMB * 8e-6 * double(m) * double(n);
   const bool tall = int64_t(256) * k * 2 < (int64_t(1) << 32);
-  GemmPlan best{1, 2, 1, k};
+  GemmPlan best{1, 2, 1, k, 4};
   double best_t = -1.0;
   for (const TileCost& c : kTiles) {
     if (c.wm > 1 && !tall) continue;
@@ -1025,10 +1046,19 @@ GemmPlan make_plan(int64_t m, int64_t n, int64_t k, size_t room, int64_t cus) {
       if (splits > 1) us += kFinishUs + partial * double(splits);
       if (best_t < 0.0 || us < best_t) {
         best_t = us;
-        best = GemmPlan{c.wm, c.wn, int(splits), kc};
+        best = GemmPlan{c.wm, c.wn, int(splits), kc, 4};
       }
     }
   }
+  // 64x128 tiles of few K steps, or of a moderate number on few CUs, take rings of 3 slots: the fourth one's 24 KB
+  // cost 0.3 us of a launch, which only longer ranges, with more of the chip asking for operands, make up for.
+  // 3 against 4 slots: 3x128x272 2.94 us / 3.26, 302x704x8 4.67 / 4.94, 2048x768x768 5.52 / 5.79, 330x832x1056 5.20
+  // / 5.48, 9x1600x120 6.99 / 7.22; but 2x896x7856 (62 workgroups of 14 steps) 6.35 / 5.65, 97x1728x8896 11.7 / 9.3.
+  const int64_t steps = (best.kchunk + 63) / 64, wgs = tiles(64, 128) * best.splits;
+  if (best.wm == 1 && (steps <= 12 || (steps <= 32 && wgs <= 48))) best.ring = 3;
+  // 128x128 tiles in one pass likewise (128 KB of LDS against 96): 727x64x2880 4.19 us / 4.40, 469x320x7120 5.74 /
+  // 6.07, 935x768x3072 7.25 / 7.46, 3301x1088x728 8.36 / 8.74; 137x2560x11712 (40 steps) 19.3 / 18.3.
+  if (best.wm == 2 && best.wn == 2 && best.splits == 1 && steps <= 16) best.ring = 3;
   return best;
 }
 
@@ -1073,7 +1103,9 @@ int launch_planned(const GemmPlan& p, const void* a, const void* b, const void* 
   if (p.wm == 4 && p.wn == 4) return launch_gemm<4, 4>(a, b, residual, c, m, n, k, s);
   if (p.wm == 4 && p.wn == 2) return launch_gemm<4, 2>(a, b, residual, c, m, n, k, s);
   if (p.wm == 2 && p.wn == 4) return launch_gemm<2, 4>(a, b, residual, c, m, n, k, s);
+  if (p.wm == 2 && p.wn == 2 && p.ring == 3) return launch_gemm<2, 2, 3>(a, b, residual, c, m, n, k, s);
   if (p.wm == 2 && p.wn == 2) return launch_gemm<2, 2>(a, b, residual, c, m, n, k, s);
+  if (p.ring == 3) return launch_gemm<1, 2, 3>(a, b, residual, c, m, n, k, s);
   return launch_gemm<1, 2>(a, b, residual, c, m, n, k, s);
 }
 
@@ -1121,12 +1153,12 @@ __global__ __launch_bounds__(256) void splitk_finish(const float* __restrict__ P
   *reinterpret_cast<u32x2*>(C + q) = u32x2{pack_bf16x2(acc.x, acc.y), pack_bf16x2(acc.z, acc.w)};
 }
 
-template <int WM, int WN>
+template <int WM, int WN, int RING = Shape<WM, WN>::NSA>
 int launch_split(const GemmPlan& p, const uint16_t* a, const uint16_t* b, const uint16_t* residual, uint16_t* c,
                  float* part, int64_t m, int64_t n, int64_t k, hipStream_t s) {
-  using Sh = Shape<WM, WN>;
+  using Sh = Shape<WM, WN, RING>;
   const int64_t tm = (m + Sh::BM - 1) / Sh::BM, tn = (n + Sh::BN - 1) / Sh::BN;   // at most a tile a CU
-  gemm_bf16_kernel<WM, WN, false, kSplit><<<dim3(unsigned(tm * tn * p.splits)), dim3(kThreads), 0, s>>>(
+  gemm_bf16_kernel<WM, WN, false, kSplit, false, RING><<<dim3(unsigned(tm * tn * p.splits)), dim3(kThreads), 0, s>>>(
       a, b, nullptr, nullptr, int(m), int(n), int(k), int(tm), int(tn), part, int(p.kchunk));
   const int64_t mn = m * n;
   const dim3 grid(unsigned((mn / 4 + 255) / 256)), block(256);
@@ -1196,6 +1228,7 @@ PTB_EXPORT int ptb_gemm_bf16_ws(const void* a, const void* b, const void* residu
   if (p.wm == 4) return launch_split<4, 2>(p, ap, bp, rp, cp, part, m, n, k, s);
   if (p.wm == 2 && p.wn == 4) return launch_split<2, 4>(p, ap, bp, rp, cp, part, m, n, k, s);
   if (p.wm == 2) return launch_split<2, 2>(p, ap, bp, rp, cp, part, m, n, k, s);
+  if (p.ring == 3) return launch_split<1, 2, 3>(p, ap, bp, rp, cp, part, m, n, k, s);
   return launch_split<1, 2>(p, ap, bp, rp, cp, part, m, n, k, s);
 }
 

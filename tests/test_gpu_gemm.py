@@ -145,12 +145,17 @@ PLANNED = [
     (9, 2304, 8, True, (64, 128, 8)),          # a single tile
     (355, 1216, 16, False, (64, 128, 7)),      # the last slice a step shorter
     (5, 1088, 8, True, (64, 128, 6)),          # slices of three steps, the last of two
-    (72, 1792, 5480, True, (128, 128, 4)),     # ragged
-    (385, 4160, 4104, True, (256, 128, 3)),    # the last slice a step shorter
+    (776, 3712, 1168, True, (128, 128, 3)),    # 70 tiles a slice, the last slice two steps shorter
+    (565, 6144, 2632, True, (256, 128, 4)),    # 63 tiles a slice, ragged in M and N
     (387, 7104, 5592, True, (256, 128, 2)),    # 88 tiles a slice, the last one a step shorter
     (262, 4416, 3744, False, (128, 256, 5)),   # 45 tiles a slice
     (482, 10304, 5408, True, (256, 256, 5)),   # 44 tiles a slice, the last slice four steps shorter
-    (1054, 6144, 4088, False, (256, 256, 3)),  # 80 tiles a slice, ragged in M and N
+    (535, 7680, 6536, False, (256, 256, 3)),   # 78 tiles a slice, ragged in M and N
+    (2105, 1088, 1120, False, (128, 128, 1)),  # a step past the rings of 3
+    (2105, 1024, 1120, False, (128, 128, 1)),  # rings of 3
+    (2048, 768, 776, False, (64, 128, 1)),     # 12 steps: rings of 3
+    (97, 832, 9104, False, (64, 128, 1)),      # 13 steps of 144 tiles: rings of 4
+    (330, 2048, 48, True, (64, 128, 8)),       # partials straight from the accumulators, ragged in M and N
 ]
 
 
@@ -326,10 +331,10 @@ def test_no_split_below_1024(m, k, n):
 
 
 @pytest.mark.parametrize("m,k,n", [
-    (640, 12288, 4096),   # split in 2 or more, 160 tiles of 128x128
-    (768, 4096, 3072),
-    (2048, 4096, 1024),
-    (385, 4160, 4104),    # ragged
+    (640, 12288, 4096),   # split in 3, 80 tiles of 128x256
+    (387, 7104, 5592),    # ragged
+    (565, 6144, 2632),
+    (482, 10304, 5408),
 ])
 def test_gemm_ws_takes_the_workspace_there_is(m, k, n):
     """Where splitting K only gains, any workspace does: none, a misaligned and a one-slice one give the
