@@ -147,7 +147,8 @@ constexpr int64_t kDirectPartials = 32768;
 template <int WM, int WN, bool RESID, int MODE, bool PERSIST = false, int RING = Shape<WM, WN>::NSA>
 __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_kernel(
     const uint16_t* __restrict__ A_in, const uint16_t* __restrict__ B_in, const uint16_t* __restrict__ R,
-    uint16_t* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n, float* __restrict__ part, int kchunk) {
+    uint16_t* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n, int by_xcd, float* __restrict__ part,
+    int kchunk) {
   using Sh = Shape<WM, WN, RING>;
   constexpr int BM = Sh::BM, BN = Sh::BN, kABytes = Sh::kABytes;
   constexpr int BK = Sh::BK, NS = Sh::NS, DIST = Sh::DIST, NSA = Sh::NSA, NSB = Sh::NSB;
@@ -177,7 +178,8 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
   int m0, n0;
   int Kl = K;    // the K columns this workgroup multiplies
   int slice = 0; // split-K: this workgroup's K slice
-  int pid = xcd_position(blockIdx.x, PERSIST ? ntiles : int(gridDim.x));
+  int pid = blockIdx.x;
+  if (PERSIST || MODE != kPlain || by_xcd) pid = xcd_position(pid, PERSIST ? ntiles : int(gridDim.x));
   if constexpr (MODE == kSplit) {
     slice = pid / ntiles;
     pid -= slice * ntiles;
@@ -952,7 +954,7 @@ int cu_count();
 
 template <int WM, int WN, int RING = Shape<WM, WN>::NSA>
 int launch_gemm(const void* a, const void* b, const void* residual, void* c, int64_t m, int64_t n, int64_t k,
-                hipStream_t s) {
+                bool by_xcd, hipStream_t s) {
   using Sh = Shape<WM, WN, RING>;
   const int64_t tm = (m + Sh::BM - 1) / Sh::BM, tn = (n + Sh::BN - 1) / Sh::BN;
   if (tm * tn > 0x7fffffff) return PTB_ERR_GRID;
@@ -963,18 +965,18 @@ int launch_gemm(const void* a, const void* b, const void* residual, void* c, int
     if (!residual && tm * tn >= 2 * cus) {
       gemm_bf16_kernel<4, 4, false, kPlain, true><<<dim3(unsigned(cus)), block, 0, s>>>(
           static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), nullptr, static_cast<uint16_t*>(c),
-          int(m), int(n), int(k), int(tm), int(tn), nullptr, 0);
+          int(m), int(n), int(k), int(tm), int(tn), 1, nullptr, 0);
       return launch_status();
     }
   }
   if (residual)
     gemm_bf16_kernel<WM, WN, true, kPlain, false, RING><<<grid, block, 0, s>>>(
         static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), static_cast<const uint16_t*>(residual),
-        static_cast<uint16_t*>(c), int(m), int(n), int(k), int(tm), int(tn), nullptr, 0);
+        static_cast<uint16_t*>(c), int(m), int(n), int(k), int(tm), int(tn), int(by_xcd), nullptr, 0);
   else
     gemm_bf16_kernel<WM, WN, false, kPlain, false, RING><<<grid, block, 0, s>>>(
         static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), nullptr, static_cast<uint16_t*>(c), int(m),
-        int(n), int(k), int(tm), int(tn), nullptr, 0);
+        int(n), int(k), int(tm), int(tn), int(by_xcd), nullptr, 0);
   return launch_status();
 }
 
@@ -989,7 +991,36 @@ struct GemmPlan {
   int wm, wn, splits;
   int64_t kchunk;   // K columns per split
   int ring;         // slots of the ring (chosen for 64x128 and 128x128 tiles, given by the others' shape)
+  bool by_xcd;      // consecutive tiles to one XCD (one pass; see xcd_order)
 };
+
+// Whether the tiles of one pass that fits one round go to the XCDs by consecutive runs.  A run is compact where
+// the tiles are many columns wide: an XCD then fetches few columns of B (178x704x10360 11.7 us in the order of the
+// workgroup ids, 6.4 by runs).  Over few columns a run reaches into two groups of kGroupM tile-rows, and the
+// ids' order, which gives an XCD the same row of every group, fetches less: 3146x2176x296 13.7 us by runs, 10.4 by
+// ids, 1067x5760x160 27.3 / 20.1, 2105x1088x1120 10.2 / 8.8.  By ids where the most rows and columns that one XCD
+// fetches are over 10% more by runs: of 26 such sizes 24 were faster by ids or within 0.5%, and nearly all others by
+// runs.  Tile counts that divide by 8 keep to runs.
+bool xcd_order(int bm, int bn, int tiles_m, int tiles_n, int64_t cus) {
+  const int n = tiles_m * tiles_n;
+  if (n % 8 == 0 || n > cus || tiles_m < 12 || tiles_m <= tiles_n || tiles_m > 256) return true;
+  int most[2] = {0, 0};   // by ids, by runs
+  for (int runs = 0; runs < 2; ++runs) {
+    for (int x = 0; x < 8; ++x) {
+      const int count = n / 8 + (x < n % 8 ? 1 : 0), first = x * (n / 8) + std::min(x, n % 8);
+      bool row[256] = {}, col[256] = {};
+      int fetched = 0;
+      for (int i = 0; i < count; ++i) {
+        const int pid = runs ? first + i : x + 8 * i, group = pid / (kGroupM * tiles_n), in = pid % (kGroupM * tiles_n);
+        const int rows = std::min(tiles_m - group * kGroupM, kGroupM), r = group * kGroupM + in % rows, c = in / rows;
+        fetched += (row[r] ? 0 : bm) + (col[c] ? 0 : bn);
+        row[r] = col[c] = true;
+      }
+      most[runs] = std::max(most[runs], fetched);
+    }
+  }
+  return 10 * most[1] <= 11 * most[0];
+}
 
 // Cost model of a plan, in us.  A round of workgroups (one a CU) costs `step` per 64-deep K step
 // plus `load` x (share of the CUs busy: they share the chip's power and L2 bandwidth) and `fixed` for
@@ -1027,7 +1058,7 @@ GemmPlan make_plan(int64_t m, int64_t n, int64_t k, size_t room, int64_t cus) {
   const double mem = kMemUs + kMemUsPerMB * 2e-6 * (double(k) * double(n) + double(m) * (double(k) + double(n)));
   const double partial = kPartialUsPerMB * 8e-6 * double(m) * double(n);
   const bool tall = int64_t(256) * k * 2 < (int64_t(1) << 32);
-  GemmPlan best{1, 2, 1, k, 4};
+  GemmPlan best{1, 2, 1, k, 4, true};
   double best_t = -1.0;
   for (const TileCost& c : kTiles) {
     if (c.wm > 1 && !tall) continue;
@@ -1046,7 +1077,7 @@ GemmPlan make_plan(int64_t m, int64_t n, int64_t k, size_t room, int64_t cus) {
       if (splits > 1) us += kFinishUs + partial * double(splits);
       if (best_t < 0.0 || us < best_t) {
         best_t = us;
-        best = GemmPlan{c.wm, c.wn, int(splits), kc, 4};
+        best = GemmPlan{c.wm, c.wn, int(splits), kc, 4, true};
       }
     }
   }
@@ -1059,6 +1090,9 @@ GemmPlan make_plan(int64_t m, int64_t n, int64_t k, size_t room, int64_t cus) {
   // 128x128 tiles in one pass likewise (128 KB of LDS against 96): 727x64x2880 4.19 us / 4.40, 469x320x7120 5.74 /
   // 6.07, 935x768x3072 7.25 / 7.46, 3301x1088x728 8.36 / 8.74; 137x2560x11712 (40 steps) 19.3 / 18.3.
   if (best.wm == 2 && best.wn == 2 && best.splits == 1 && steps <= 16) best.ring = 3;
+  if (best.splits == 1 && tiles(64 * best.wm, 64 * best.wn) <= cus)
+    best.by_xcd = xcd_order(64 * best.wm, 64 * best.wn, int((m + 64 * best.wm - 1) / (64 * best.wm)),
+                            int((n + 64 * best.wn - 1) / (64 * best.wn)), cus);
   return best;
 }
 
@@ -1099,14 +1133,14 @@ int required_slices(int64_t m, int64_t n, int64_t k) {
 
 int launch_planned(const GemmPlan& p, const void* a, const void* b, const void* residual, void* c, int64_t m,
                    int64_t n, int64_t k, hipStream_t s) {
-  if (p.wm == 4 && p.wn == 3) return launch_gemm<4, 3>(a, b, residual, c, m, n, k, s);
-  if (p.wm == 4 && p.wn == 4) return launch_gemm<4, 4>(a, b, residual, c, m, n, k, s);
-  if (p.wm == 4 && p.wn == 2) return launch_gemm<4, 2>(a, b, residual, c, m, n, k, s);
-  if (p.wm == 2 && p.wn == 4) return launch_gemm<2, 4>(a, b, residual, c, m, n, k, s);
-  if (p.wm == 2 && p.wn == 2 && p.ring == 3) return launch_gemm<2, 2, 3>(a, b, residual, c, m, n, k, s);
-  if (p.wm == 2 && p.wn == 2) return launch_gemm<2, 2>(a, b, residual, c, m, n, k, s);
-  if (p.ring == 3) return launch_gemm<1, 2, 3>(a, b, residual, c, m, n, k, s);
-  return launch_gemm<1, 2>(a, b, residual, c, m, n, k, s);
+  if (p.wm == 4 && p.wn == 3) return launch_gemm<4, 3>(a, b, residual, c, m, n, k, p.by_xcd, s);
+  if (p.wm == 4 && p.wn == 4) return launch_gemm<4, 4>(a, b, residual, c, m, n, k, p.by_xcd, s);
+  if (p.wm == 4 && p.wn == 2) return launch_gemm<4, 2>(a, b, residual, c, m, n, k, p.by_xcd, s);
+  if (p.wm == 2 && p.wn == 4) return launch_gemm<2, 4>(a, b, residual, c, m, n, k, p.by_xcd, s);
+  if (p.wm == 2 && p.wn == 2 && p.ring == 3) return launch_gemm<2, 2, 3>(a, b, residual, c, m, n, k, p.by_xcd, s);
+  if (p.wm == 2 && p.wn == 2) return launch_gemm<2, 2>(a, b, residual, c, m, n, k, p.by_xcd, s);
+  if (p.ring == 3) return launch_gemm<1, 2, 3>(a, b, residual, c, m, n, k, p.by_xcd, s);
+  return launch_gemm<1, 2>(a, b, residual, c, m, n, k, p.by_xcd, s);
 }
 
 }  // namespace
@@ -1159,7 +1193,7 @@ int launch_split(const GemmPlan& p, const uint16_t* a, const uint16_t* b, const 
   using Sh = Shape<WM, WN, RING>;
   const int64_t tm = (m + Sh::BM - 1) / Sh::BM, tn = (n + Sh::BN - 1) / Sh::BN;   // at most a tile a CU
   gemm_bf16_kernel<WM, WN, false, kSplit, false, RING><<<dim3(unsigned(tm * tn * p.splits)), dim3(kThreads), 0, s>>>(
-      a, b, nullptr, nullptr, int(m), int(n), int(k), int(tm), int(tn), part, int(p.kchunk));
+      a, b, nullptr, nullptr, int(m), int(n), int(k), int(tm), int(tn), 1, part, int(p.kchunk));
   const int64_t mn = m * n;
   const dim3 grid(unsigned((mn / 4 + 255) / 256)), block(256);
   static_assert(kMaxSplits == 8, "a finish kernel for every split count");
@@ -1241,7 +1275,7 @@ int launch_swiglu(const void* a, const void* b, void* c, int64_t m, int64_t n, i
   if (tm * tn > 0x7fffffff) return PTB_ERR_GRID;
   gemm_bf16_kernel<WM, WN, false, kSwiGLU><<<dim3(unsigned(tm * tn)), dim3(kThreads), 0, s>>>(
       static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), nullptr, static_cast<uint16_t*>(c), int(m),
-      int(n), int(k), int(tm), int(tn), nullptr, 0);
+      int(n), int(k), int(tm), int(tn), 1, nullptr, 0);
   return launch_status();
 }
 

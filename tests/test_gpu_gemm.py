@@ -151,8 +151,9 @@ PLANNED = [
     (262, 4416, 3744, False, (128, 256, 5)),   # 45 tiles a slice
     (482, 10304, 5408, True, (256, 256, 5)),   # 44 tiles a slice, the last slice four steps shorter
     (535, 7680, 6536, False, (256, 256, 3)),   # 78 tiles a slice, ragged in M and N
-    (2105, 1088, 1120, False, (128, 128, 1)),  # a step past the rings of 3
-    (2105, 1024, 1120, False, (128, 128, 1)),  # rings of 3
+    (2105, 1088, 1120, False, (128, 128, 1)),  # 17 x 9 tiles: by ids over the XCDs; a step past the rings of 3
+    (2105, 1024, 1120, False, (128, 128, 1)),  # the same in rings of 3
+    (1850, 2048, 544, True, (64, 128, 1)),     # 29 x 5 tiles: by ids over the XCDs
     (2048, 768, 776, False, (64, 128, 1)),     # 12 steps: rings of 3
     (97, 832, 9104, False, (64, 128, 1)),      # 13 steps of 144 tiles: rings of 4
     (330, 2048, 48, True, (64, 128, 8)),       # partials straight from the accumulators, ragged in M and N
