@@ -1042,8 +1042,32 @@ constexpr TileCost kTiles[] = {{4, 4, 0.830, 0.500, 6.29}, {4, 3, 0.620, 0.511, 
 // (256x256's step and load a little above the fit's 0.816 and 0.464: at 1664x12288x4096 the fit took two
 // slices of 256x256 tiles, 1.4% of the layer slower than one pass of 256x128 ones)
 constexpr double kMemUs = 3.3, kMemUsPerMB = 0.106, kFinishUs = 1.9, kPartialUsPerMB = 0.148;
+// A split that nobody has to bring a workspace for (required_slices) has to beat one pass by this factor.  Over 160
+// sizes at which the model saw a split ahead by less than 1.3, those it put less than 1.12 ahead ran 3% slower than
+// one pass (geometric mean; 3954x2368x160 11.7 -> 14.6 us, 492x2496x2304 13.0 -> 16.7), those further ahead 10% faster.
+constexpr double kSplitMargin = 1.12;
 constexpr int kMaxSplits = 8;
 constexpr int64_t kFitK = 16384;   // past it (the fit ends at 12288) splits keep to the narrow rule below
+
+// The K slices that ptb_gemm_bf16_ws asks a caller's workspace for: those of 64x128 tiles on at most half
+// of the CUs where a workgroup's operand stream (90 GB/s; 2.5 us to launch) gets shorter by more than the
+// finish launch (1.5 us) and the partials' traffic (2.5 TB/s) take.  Part of the call's contract, not of the plan: such a call is refused without
+// the room for them, and every other one runs with the room it has.
+int required_slices(int64_t m, int64_t n, int64_t k, int64_t cus) {
+  const int64_t t64 = ((m + 63) / 64) * ((n + 127) / 128);
+  auto stream = [&](int sp) { return 2.5 + double(k) / sp * (64 + 128) * 2 / 90e3; };
+  int best = 1;
+  double best_us = stream(1);
+  for (int sp = 2; sp <= 8 && k >= 1024 && k / sp >= 256 && t64 * sp <= cus; sp *= 2) {
+    const double us = stream(sp) + (1.5 + sp * double(m) * double(n) * 8 / 2.5e6);
+    if (us < best_us) {
+      best_us = us;
+      best = sp;
+    }
+  }
+  const int64_t kc = ((k + best - 1) / best + 63) / 64 * 64;
+  return int((k + kc - 1) / kc);
+}
 
 // The cheapest plan by the model.  Splits: K at least 1024 and slices at least 128 deep (below, the
 // finish launch costs more than the shorter slices save), all in one round of workgroups; a K past
@@ -1058,6 +1082,7 @@ GemmPlan make_plan(int64_t m, int64_t n, int64_t k, size_t room, int64_t cus) {
   const double mem = kMemUs + kMemUsPerMB * 2e-6 * (double(k) * double(n) + double(m) * (double(k) + double(n)));
   const double partial = kPartialUsPerMB * 8e-6 * double(m) * double(n);
   const bool tall = int64_t(256) * k * 2 < (int64_t(1) << 32);
+  const double margin = may_split && required_slices(m, n, k, cus) < 2 ? kSplitMargin : 1.0;
   GemmPlan best{1, 2, 1, k, 4, true};
   double best_t = -1.0;
   for (const TileCost& c : kTiles) {
@@ -1075,6 +1100,7 @@ GemmPlan make_plan(int64_t m, int64_t n, int64_t k, size_t room, int64_t cus) {
       const double body = double(full) * (steps * (c.step + c.load) + c.fixed) + steps * (c.step + c.load * last) + c.fixed;
       double us = std::sqrt(body * body + mem * mem);
       if (splits > 1) us += kFinishUs + partial * double(splits);
+      if (splits > 1) us *= margin;
       if (best_t < 0.0 || us < best_t) {
         best_t = us;
         best = GemmPlan{c.wm, c.wn, int(splits), kc, 4, true};
@@ -1109,26 +1135,6 @@ GemmPlan gemm_plan(int64_t m, int64_t n, int64_t k, size_t room) {
   if (last.m != m || last.n != n || last.k != k || last.room != room || last.cus != cus)
     last = Last{m, n, k, cus, room, make_plan(m, n, k, room, cus)};
   return last.plan;
-}
-
-// The K slices that ptb_gemm_bf16_ws asks a caller's workspace for: those of 64x128 tiles on at most half
-// of the CUs where a workgroup's operand stream (90 GB/s; 2.5 us to launch) gets shorter by more than the
-// finish launch (1.5 us) and the partials' traffic (2.5 TB/s) take.  Part of the call's contract, not of the plan: such a call is refused without
-// the room for them, and every other one runs with the room it has.
-int required_slices(int64_t m, int64_t n, int64_t k) {
-  const int64_t cus = cu_count(), t64 = ((m + 63) / 64) * ((n + 127) / 128);
-  auto stream = [&](int sp) { return 2.5 + double(k) / sp * (64 + 128) * 2 / 90e3; };
-  int best = 1;
-  double best_us = stream(1);
-  for (int sp = 2; sp <= 8 && k >= 1024 && k / sp >= 256 && t64 * sp <= cus; sp *= 2) {
-    const double us = stream(sp) + (1.5 + sp * double(m) * double(n) * 8 / 2.5e6);
-    if (us < best_us) {
-      best_us = us;
-      best = sp;
-    }
-  }
-  const int64_t kc = ((k + best - 1) / best + 63) / 64 * 64;
-  return int((k + kc - 1) / kc);
 }
 
 int launch_planned(const GemmPlan& p, const void* a, const void* b, const void* residual, void* c, int64_t m,
@@ -1238,7 +1244,7 @@ PTB_EXPORT int ptb_gemm_bf16_ws(const void* a, const void* b, const void* residu
   if (p.splits > 1) {
     const size_t need = plan_workspace(p, m, n);
     const size_t room = workspace && aligned16(workspace) ? workspace_bytes : 0;
-    const int required = required_slices(m, n, k);
+    const int required = required_slices(m, n, k, cu_count());
     if (required > 1) {
       if (!a || !b || !c || !workspace) return PTB_ERR_NULL;
       if (workspace_bytes < std::min(need, size_t(required) * size_t(m) * size_t(n) * sizeof(float)))

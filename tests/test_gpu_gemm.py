@@ -153,7 +153,7 @@ PLANNED = [
     (535, 7680, 6536, False, (256, 256, 3)),   # 78 tiles a slice, ragged in M and N
     (2105, 1088, 1120, False, (128, 128, 1)),  # 17 x 9 tiles: by ids over the XCDs; a step past the rings of 3
     (2105, 1024, 1120, False, (128, 128, 1)),  # the same in rings of 3
-    (1850, 2048, 544, True, (64, 128, 1)),     # 29 x 5 tiles: by ids over the XCDs
+    (3146, 2176, 296, True, (64, 128, 1)),     # 50 x 3 tiles: by ids over the XCDs
     (2048, 768, 776, False, (64, 128, 1)),     # 12 steps: rings of 3
     (97, 832, 9104, False, (64, 128, 1)),      # 13 steps of 144 tiles: rings of 4
     (330, 2048, 48, True, (64, 128, 8)),       # partials straight from the accumulators, ragged in M and N
@@ -390,7 +390,7 @@ def test_split_k_exact_on_small_integers():
 
 MID_SIZES = [
     (2048, 768, 768, False, (64, 128, 1)), (1000, 768, 264, True, (64, 128, 1)), (4000, 384, 512, True, (64, 128, 1)),
-    (768, 3072, 1024, False, (128, 128, 4)), (2048, 4096, 1024, True, (128, 128, 2)),
+    (768, 3072, 1024, False, (128, 128, 4)), (2048, 4096, 1024, True, (64, 128, 1)),
 ]
 
 
