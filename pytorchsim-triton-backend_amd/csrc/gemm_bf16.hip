@@ -1122,16 +1122,19 @@ GemmPlan make_plan(int64_t m, int64_t n, int64_t k, size_t room, int64_t cus) {
   return best;
 }
 
-// The plan of a size is asked for twice a call, by the workspace query and by the launch: a thread
-// keeps its last one.
+// The plan of a size is asked for twice a call, by the workspace query and by the launch (with other room where no
+// split is wanted), and a model comes back to a few sizes: a thread keeps the last plan of each of 64 places that
+// sizes are spread over.
 GemmPlan gemm_plan(int64_t m, int64_t n, int64_t k, size_t room) {
   struct Last {
     int64_t m = -1, n = 0, k = 0, cus = 0;
     size_t room = 0;
     GemmPlan plan{};
   };
-  static thread_local Last last;
+  static thread_local Last kept[64];
   const int64_t cus = cu_count();
+  const uint64_t h = (uint64_t(m) * 0x9e3779b97f4a7c15u + uint64_t(n)) * 0xc2b2ae3d27d4eb4fu + uint64_t(k) + room;
+  Last& last = kept[(h * 0x9e3779b97f4a7c15u) >> 58];
   if (last.m != m || last.n != n || last.k != k || last.room != room || last.cus != cus)
     last = Last{m, n, k, cus, room, make_plan(m, n, k, room, cus)};
   return last.plan;
