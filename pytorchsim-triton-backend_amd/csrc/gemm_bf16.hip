@@ -1288,13 +1288,24 @@ int launch_swiglu(const void* a, const void* b, void* c, int64_t m, int64_t n, i
   return launch_status();
 }
 
+// The groups that `rows` rows hit, spread over them at random with popularities of log-normal deviation `skew`
+// (0: all alike): the mean over eight equal shares of the groups.
+double groups_hit(double groups, double rows, double skew) {
+  static const double share[] = {-1.534, -0.887, -0.489, -0.157, 0.157, 0.489, 0.887, 1.534};   // normal quantiles
+  double sum = 0.0;
+  for (const double z : share) sum += 1.0 - std::exp(-rows / groups * std::exp(skew * z - 0.5 * skew * skew));
+  return groups * sum / 8.0;
+}
+
 // The tile of a grouped GEMM: 0 128x256, 1 128x128 (one workgroup a CU), 2 64x128 (two).  The host does
-// not see the row counts; rows spread at random over the groups hit about groups * (1 - e^(-rows /
-// groups)) of them, and a hit group of m rows takes m / BM + 1/2 row tiles, or one up to m = BM / 2.  The
-// plain GEMM's cost of those rounds (its step, load and fixed per tile; 128x128 steps 0.34 here) picks
-// within 0.5% (geometric mean) of the best of the three over 79 (groups, rows, n, k) points, 2 to 128
-// groups and 24 to 16384 rows, at worst 1.1% slower and on average 1.09x faster than one workgroup a
-// 128x128 tile.
+// not see the row counts: a hit group of m rows takes m / BM + 1/2 row tiles, or one up to m = BM / 2, and the
+// cost of those rounds is the plain GEMM's (its step, load and fixed per tile; 128x128 steps 0.34 here).  Nor does
+// it see how evenly the rows are routed: the tile that is cheapest for evenly popular groups gives way to the one
+// with the least product of costs for even and strongly skewed popularities where that product is less than
+// 1 / 1.3 of its own.  (By even popularities alone the wide tile ran where skewed rows hit too few groups to fill the
+// CUs with it: 32 rows of 16 groups, 4096 -> 2816, 6 of them hit, 56.8 us, now 42.0; 57 rows of 32, 2048 -> 1536,
+// 25.1, now 18.2.)  Over 1040 points (2 to 128 groups, 17 to 8192 rows, four weights, deviations of 0 to 1.5) the
+// pick runs within 1.6% (geometric mean) of the best tile and 12% faster than a workgroup a 128x128 tile.
 struct GroupedPlan {
   int tile;
   bool stream;
@@ -1315,19 +1326,22 @@ GroupedPlan grouped_plan(int64_t groups, int64_t a_rows, int64_t n, int64_t k, i
   } const tiles[] = {{128, 256, 0.592, 0.250, 3.92}, {128, 128, 0.340, 0.196, 2.42}, {64, 128, 0.296, 0.141, 1.68}};
   if (groups <= 0) return {2, false};
   const double hit = double(groups) * (1.0 - std::exp(-double(a_rows) / double(groups)));
+  const double hits[] = {hit, groups_hit(double(groups), double(a_rows), 2.0)};
   const double mean = double(a_rows) / hit, steps = double(k / 64);
-  int best = 0;
-  double best_t = -1.0;
+  double t[3][2];
+  int even = 0, both = 0;   // the cheapest for even popularities, and by the product
   for (int i = 0; i < 3; ++i) {
     const auto& c = tiles[i];
-    const double w = hit * (mean > c.bm / 2 ? mean / c.bm + 0.5 : 1.0) * double((n + c.bn - 1) / c.bn);
-    const double full = std::ceil(w / double(cus)) - 1.0, last = w / double(cus) - full;
-    const double t = full * (steps * (c.step + c.load) + c.fixed) + steps * (c.step + c.load * last) + c.fixed;
-    if (best_t < 0.0 || t < best_t) {
-      best_t = t;
-      best = i;
+    for (int j = 0; j < 2; ++j) {
+      const double m = double(a_rows) / hits[j];
+      const double w = hits[j] * (m > c.bm / 2 ? m / c.bm + 0.5 : 1.0) * double((n + c.bn - 1) / c.bn);
+      const double full = std::ceil(w / double(cus)) - 1.0, last = w / double(cus) - full;
+      t[i][j] = full * (steps * (c.step + c.load) + c.fixed) + steps * (c.step + c.load * last) + c.fixed;
     }
+    if (t[i][0] < t[even][0]) even = i;
+    if (t[i][0] * t[i][1] < t[both][0] * t[both][1]) both = i;
   }
+  const int best = t[even][0] * t[even][1] > 1.3 * t[both][0] * t[both][1] ? both : even;
   const double bytes = double(n) * double(k) * 2.0, line = double(kStreamBytes);   // a group's weight
   return {best, mean <= tiles[best].bm && double(groups) * bytes > line && 1.5 * hit * bytes > line};
 }

@@ -123,6 +123,10 @@ def test_streaming_starts_where_the_same_bytes_again_gain(lib):
         assert plan(lib.ptb_grouped_gemm_plan, groups, 8 * groups, 2048, 1536)[2] == streamed, groups
     for rows, streamed in [(17, 0), (36, 0), (40, 1)]:   # few rows read few of 128 groups: 200 MiB are 33.3
         assert plan(lib.ptb_grouped_gemm_plan, 128, rows, 2048, 1536)[2] == streamed, rows
+    # few rows, which skewed routing sends to few groups: no wide tiles that would leave the CUs idle
+    assert plan(lib.ptb_grouped_gemm_plan, 16, 32, 4096, 2816)[:2] == (64, 128)
+    assert plan(lib.ptb_grouped_gemm_plan, 32, 57, 2048, 1536)[:2] == (64, 128)
+    assert plan(lib.ptb_grouped_gemm_plan, 128, 8192, 2048, 1536)[:2] == (128, 256)
     assert lib.ptb_attn_decode_plan(0, 4, 8192, P16) == _lib.PTB_ERR_SHAPE
     assert lib.ptb_attn_decode_plan(1, 4, 8192, None) == _lib.PTB_ERR_NULL
     assert lib.ptb_grouped_gemm_plan(4, 0, 64, 64, P16) == _lib.PTB_ERR_SHAPE
