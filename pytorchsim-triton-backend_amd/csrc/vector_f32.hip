@@ -460,6 +460,10 @@ PTB_EXPORT int ptb_swiglu_f32(const float* x, const float* wg, const float* wu, 
   if (k >= (int64_t(1) << 24) || n >= (int64_t(1) << 24))
     return launch_swiglu_f32<2, 2, 16, true>(x, wg, wu, o, m, n, k, s);
   if (blocks <= 2 * int64_t(cus)) return launch_swiglu_f32<1, 8, 8, false>(x, wg, wu, o, m, n, k, s);
+  // Where K is short enough for the first of the waves that split it, the others only add the sum through the LDS:
+  // 128x32 outputs to four waves, each with all of K (no larger error).  4096x4096 outputs: K = 8 32.7 us before the
+  // matrix instruction, 43.9 split, 24.3 so, K = 16 33.0, 44.5, 29.6; 363x4230 outputs: K = 8 7.6, 8.3, 6.2.
+  if (k <= (blocks > 9 * int64_t(cus) ? 16 : 8)) return launch_swiglu_f32<4, 1, 8, false>(x, wg, wu, o, m, n, k, s);
   if (blocks <= 9 * int64_t(cus)) return launch_swiglu_f32<1, 4, 8, false>(x, wg, wu, o, m, n, k, s);
   return launch_swiglu_f32<2, 2, 16, false>(x, wg, wu, o, m, n, k, s);
 }

@@ -292,6 +292,10 @@ def test_swiglu_f32_wide(m, n, k):
     (700, 800, 40),       # four waves a block (550 blocks): a slab and a tail of eight
     (1500, 1601, 33),     # 64x32 outputs (2397 blocks): a slab and a tail of one, ragged both ways
     (2049, 1200, 96),     # the same, whole slabs only
+    (777, 1700, 7),       # 128x32 outputs (1350 blocks): a tail of seven
+    (4001, 2049, 15),     # the same (8190 blocks): a slab and a tail of seven, ragged both ways
+    (3000, 1500, 16),     # two whole slabs
+    (3000, 1500, 1),      # one k
 ])
 def test_swiglu_f32_blocks(m, n, k):
     """Every workgroup shape of the fp32 SwiGLU at ragged sizes and slab tails.  Operands in {-1, 0, 1}
