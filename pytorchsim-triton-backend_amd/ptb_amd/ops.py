@@ -236,7 +236,8 @@ def gemm(a: torch.Tensor, b: torch.Tensor, residual: torch.Tensor | None = None,
 
 def gemm_swiglu(a: torch.Tensor, b: torch.Tensor, out=None) -> torch.Tensor:
     """C[M, I] = silu(bf16(A @ B[:, :I])) * bf16(A @ B[:, I:]) for B [K, 2I]: the gate_up GEMM and the
-    SwiGLU gate in one kernel, equal bit for bit to ``silu_mul(gemm(a, b))``."""
+    SwiGLU gate in one kernel, equal bit for bit to ``silu_mul(gemm(a, b, split_k=False))``.  (``gemm``
+    alone may cut K into slices, whose sums it adds in another order.)"""
     _need(a, "a", BF16, 2)
     _need(b, "b", BF16, 2)
     m, k = a.shape

@@ -12,10 +12,11 @@ manifest.json lists 14 launches of 12 kernels, 00,01,02,03,04,03,05,06,07,08,00,
 
 K01 and the two K03 launches run as one GEMM over the concatenated weight [hidden, q|k|v] (one round
 of 256x256 tiles fills the chip; the separate k and v GEMMs have 128 tiles each and leave half the
-CUs idle), and K02, K04 and K05 read their column slices of its [T, q|k|v] output in place (the
-same per-element arithmetic as the separate products).  K09 and K10 run as one kernel (``ops.gemm_swiglu``: the gate_up GEMM with silu(g) * u in its
-epilogue, bit for bit the pair's result), so the [T, 2*I] gate_up product never goes to HBM, and
-K06 writes O token-major, [T, 32, 128], so K07's transpose is not launched.
+CUs idle), and K02, K04 and K05 read their column slices of its [T, q|k|v] output in place (the same
+products; where one of the GEMMs cuts K into slices and the other does not, their sums are added in
+another order).  K09 and K10 run as one kernel (``ops.gemm_swiglu``: the gate_up GEMM with silu(g) * u
+in its epilogue, bit for bit the pair's result with the GEMM in one pass over K), so the [T, 2*I] gate_up
+product never goes to HBM, and K06 writes O token-major, [T, 32, 128], so K07's transpose is not launched.
 
 (The data flow is read from each kernel's index arithmetic; the reference times these kernels
 separately and never runs the layer end to end, validation/gemm/simulate_shapes.py:279-302.)
