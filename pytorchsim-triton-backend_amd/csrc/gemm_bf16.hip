@@ -1028,7 +1028,8 @@ bool xcd_order(int bm, int bn, int tiles_m, int tiles_n, int64_t cus) {
 // two overlap partly, which their root sum of squares follows.  A split adds the finish launch,
 // kFinishUs, and writing and reading 4 bytes per output and slice at kPartialUsPerMB.  Fitted by
 // least squares to 3969 (shape, tile, split) times on MI355X over 239 shapes with M 1 .. 4096, K
-// 64 .. 12288 and N 128 .. 24576: 4.7% rms error, and the plans it picks run within 0.9% (geometric
+// 64 .. 12288 and N 128 .. 24576: 4.7% rms error, and the plans picked by the fit as it came out (before 256x256's
+// constants were raised, below, and splits had to beat one pass by kSplitMargin) ran within 0.9% (geometric
 // mean) of the best measured plan of each shape, 1.23x faster than the previous rule's plans (one
 // pass of 128x128 tiles where those covered 3/4 of the CUs, splits of 64x128 tiles only; both with
 // 32-deep stages): 640x12288x4096 147 -> 71 us, 1280x12288x4096 237 -> 114, 384x12288x4096 105 -> 50,
@@ -1042,9 +1043,9 @@ constexpr TileCost kTiles[] = {{4, 4, 0.830, 0.500, 6.29}, {4, 3, 0.620, 0.511, 
 // (256x256's step and load a little above the fit's 0.816 and 0.464: at 1664x12288x4096 the fit took two
 // slices of 256x256 tiles, 1.4% of the layer slower than one pass of 256x128 ones)
 constexpr double kMemUs = 3.3, kMemUsPerMB = 0.106, kFinishUs = 1.9, kPartialUsPerMB = 0.148;
-// A split that nobody has to bring a workspace for (required_slices) has to beat one pass by this factor.  Over 160
-// sizes at which the model saw a split ahead by less than 1.3, those it put less than 1.12 ahead ran 3% slower than
-// one pass (geometric mean; 3954x2368x160 11.7 -> 14.6 us, 492x2496x2304 13.0 -> 16.7), those further ahead 10% faster.
+// A split that nobody has to bring a workspace for (required_slices) has to beat one pass by this factor.  Of 128
+// sizes at which the model saw a split ahead by less than 1.3, the 54 that it put less than 1.12 ahead ran 4% slower
+// split (geometric mean; 3954x2368x160 11.7 -> 14.6 us, 492x2496x2304 13.0 -> 16.7), the others 11% faster.
 constexpr double kSplitMargin = 1.12;
 constexpr int kMaxSplits = 8;
 constexpr int64_t kFitK = 16384;   // past it (the fit ends at 12288) splits keep to the narrow rule below

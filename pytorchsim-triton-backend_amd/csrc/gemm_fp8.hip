@@ -362,10 +362,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
 // M <= 16 MB rows of A against 16 columns (rows of Wt) a workgroup: kRowWaves waves take every
 // kRowWaves-th 128-wide K step, each lane holding 32 bytes of one row of Wt (lane % 16) and of MB rows of
 // A per step straight from global memory (16 + 16 bytes 64 apart: the K order within a step is the same
-// for both operands, so it does not matter to the dot product), UN steps' loads issued before the first
-// MFMA.  The waves' sums meet in LDS in wave order.  Bound by the stream of W and, at 16 rows, by A from
-// L2 beside it (each workgroup reads all of A): 16x4096x4096 29.7 -> 6.7 us (5.7 at one row), 16x512x512
-// 7.1 -> 2.8 us against the 256x128 tiles that ran before; W is read once a call (streaming policy).
+// for both operands, so it does not matter to the dot product).  Where a wave has UN steps or more (K past 5120
+// at one block of rows, 3072 at two) their loads go out before the first MFMA, the steps left over one by one;
+// shorter K runs one by one throughout.  The waves' sums meet in LDS in wave order.  Bound by the stream of W and, at 16 rows, by A from
+// L2 beside it (each workgroup reads all of A): 16x4096x4096 (four steps a wave) 29.7 -> 6.7 us (5.7 at one row),
+// 16x512x512 7.1 -> 2.8 us against the 256x128 tiles that ran before; W is read once a call (streaming policy).
 // Waves with contiguous K ranges, or a K start rotated by workgroup, measured the same.
 constexpr int kRowWaves = 8;
 template <int MB>

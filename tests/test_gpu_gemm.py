@@ -453,7 +453,7 @@ SWIGLU_TILES = [
     (515, 320, 5632, (128, 256)),    # the last row tile three rows
     (2047, 448, 2176, (256, 192)),   # tiles of 96 outputs: the last one covers 64 of its 96
     (2500, 192, 3200, (256, 256)),
-    (768, 4096, 1536, (128, 128)),   # a size that ops.gemm splits in K
+    (300, 4096, 768, (64, 128)),     # a size that ops.gemm splits in K
 ]
 
 
@@ -461,7 +461,7 @@ SWIGLU_TILES = [
 def test_gemm_swiglu_every_tile(m, k, inter, tile):
     """The SwiGLU epilogue of every tile shape of the plan, ragged in M and (256x192) in the outputs:
     bit for bit the one-pass GEMM followed by silu_mul, and nothing past C."""
-    assert gemm_plan(m, k, 2 * inter, split=0) == (*tile, 1)
+    assert gemm_plan(m, k, 2 * inter, split=0) == (*tile, 1) and (gemm_plan(m, k, 2 * inter)[2] > 1) == (k > 1024)
     a = randn((m, k), 61, std=1 / 16).to(DEV)
     b = randn((k, 2 * inter), 62, std=1 / 4).to(DEV)
     guard = torch.full((m * inter + 8192,), float("nan"), dtype=torch.bfloat16, device=DEV)

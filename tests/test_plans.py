@@ -18,6 +18,7 @@ def test_bf16_walks(m, k, n):
 @pytest.mark.parametrize("m,k,inter,tile", gemms.SWIGLU_TILES)
 def test_swiglu_plans(m, k, inter, tile):
     assert gemms.gemm_plan(m, k, 2 * inter, split=0) == (*tile, 1)
+    assert (gemms.gemm_plan(m, k, 2 * inter)[2] > 1) == (k > 1024)
 
 
 @pytest.mark.parametrize("m,k,n,tiles", gemms.FP8_PLANNED)
