@@ -1043,10 +1043,12 @@ constexpr TileCost kTiles[] = {{4, 4, 0.830, 0.500, 6.29}, {4, 3, 0.620, 0.511, 
 // (256x256's step and load a little above the fit's 0.816 and 0.464: at 1664x12288x4096 the fit took two
 // slices of 256x256 tiles, 1.4% of the layer slower than one pass of 256x128 ones)
 constexpr double kMemUs = 3.3, kMemUsPerMB = 0.106, kFinishUs = 1.9, kPartialUsPerMB = 0.148;
-// A split that nobody has to bring a workspace for (required_slices) has to beat one pass by this factor.  Of 128
-// sizes at which the model saw a split ahead by less than 1.3, the 54 that it put less than 1.12 ahead ran 4% slower
-// split (geometric mean; 3954x2368x160 11.7 -> 14.6 us, 492x2496x2304 13.0 -> 16.7), the others 11% faster.
-constexpr double kSplitMargin = 1.12;
+// A split that nobody has to bring a workspace for (required_slices) has to beat one pass by these factors, taller
+// outputs than wide by the larger one: the fit took their one pass in an order over the XCDs that they no longer
+// run in.  Of 128 sizes at which the model saw a split ahead by less than 1.3, the 37 that it put less than this
+// ahead ran 7% slower split (geometric mean; 3954x2368x160 11.7 us in one pass, 14.6 split, 492x2496x2304 13.0 /
+// 16.7), the others 10% faster (270x7488x7720 52.6 / 48.0, 293x3520x2728 20.5 / 16.5).
+constexpr double kSplitMarginTall = 1.12, kSplitMargin = 1.07;
 constexpr int kMaxSplits = 8;
 constexpr int64_t kFitK = 16384;   // past it (the fit ends at 12288) splits keep to the narrow rule below
 
@@ -1083,7 +1085,7 @@ GemmPlan make_plan(int64_t m, int64_t n, int64_t k, size_t room, int64_t cus) {
   const double mem = kMemUs + kMemUsPerMB * 2e-6 * (double(k) * double(n) + double(m) * (double(k) + double(n)));
   const double partial = kPartialUsPerMB * 8e-6 * double(m) * double(n);
   const bool tall = int64_t(256) * k * 2 < (int64_t(1) << 32);
-  const double margin = may_split && required_slices(m, n, k, cus) < 2 ? kSplitMargin : 1.0;
+  const double margin = !may_split || required_slices(m, n, k, cus) > 1 ? 1.0 : m > n ? kSplitMarginTall : kSplitMargin;
   GemmPlan best{1, 2, 1, k, 4, true};
   double best_t = -1.0;
   for (const TileCost& c : kTiles) {
