@@ -135,7 +135,7 @@ __device__ __forceinline__ int swiglu_staged(int wn, int j, int n) {
 // swiglu_staged), and the epilogue stores bf16(silu(bf16(gate)) * bf16(up)), as a separate silu_mul
 // would compute it from the bf16 GEMM.
 enum { kPlain = 0, kSplit = 1, kSwiGLU = 2 };
-// Up to this many outputs the partials of 64x128 tiles leave straight from the accumulators, without the barrier
+// Up to this many outputs the partials of 64x128 tiles in rings of 3 leave straight from the accumulators, without the barrier
 // and the LDS pass: 348x2048x40 5.69 -> 5.42 us, 3x2816x8 5.54 -> 5.23, 544x1600x48 6.02 -> 5.78.  Past it whole
 // rows a store instruction are worth them: 1024x2048x128 7.74 us staged, 8.09 direct; 193x3008x576 7.51 / 7.84.
 constexpr int64_t kDirectPartials = 32768;
@@ -147,7 +147,7 @@ constexpr int64_t kDirectPartials = 32768;
 template <int WM, int WN, bool RESID, int MODE, bool PERSIST = false, int RING = Shape<WM, WN>::NSA>
 __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_kernel(
     const uint16_t* __restrict__ A_in, const uint16_t* __restrict__ B_in, const uint16_t* __restrict__ R,
-    uint16_t* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n, int by_xcd, float* __restrict__ part,
+    uint16_t* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n, int xcd_grid, float* __restrict__ part,
     int kchunk) {
   using Sh = Shape<WM, WN, RING>;
   constexpr int BM = Sh::BM, BN = Sh::BN, kABytes = Sh::kABytes;
@@ -178,8 +178,9 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
   int m0, n0;
   int Kl = K;    // the K columns this workgroup multiplies
   int slice = 0; // split-K: this workgroup's K slice
+  // xcd_grid: the workgroups of the launch (the tiles of a persistent walk), 0: positions by workgroup id
   int pid = blockIdx.x;
-  if (PERSIST || MODE != kPlain || by_xcd) pid = xcd_position(pid, PERSIST ? ntiles : int(gridDim.x));
+  if (MODE != kPlain || xcd_grid > 0) pid = xcd_position(pid, xcd_grid);
   if constexpr (MODE == kSplit) {
     slice = pid / ntiles;
     pid -= slice * ntiles;
@@ -464,7 +465,7 @@ __global__ __launch_bounds__(kThreads, (WM * WN >= 12 ? 1 : 2)) void gemm_bf16_k
   // residual is read the same way.  The region is the wave's own and LDS operations of a wave
   // complete in order, so no barrier separates its writes from its reads.  Rows past M and columns
   // past `cols` fall outside the buffer resources (stores dropped, loads 0): no branches.
-  const bool direct = MODE == kSplit && WM == 1 && int64_t(M) * N <= kDirectPartials;
+  const bool direct = MODE == kSplit && WM == 1 && RING == 3 && int64_t(M) * N <= kDirectPartials;
   if (!direct) __syncthreads();
   auto store_staged = [&](auto ng, auto value, uint16_t* out, int ldc, int cols, int col0) __attribute__((always_inline)) {
     constexpr int NG = decltype(ng)::value;
@@ -965,18 +966,18 @@ int launch_gemm(const void* a, const void* b, const void* residual, void* c, int
     if (!residual && tm * tn >= 2 * cus) {
       gemm_bf16_kernel<4, 4, false, kPlain, true><<<dim3(unsigned(cus)), block, 0, s>>>(
           static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), nullptr, static_cast<uint16_t*>(c),
-          int(m), int(n), int(k), int(tm), int(tn), 1, nullptr, 0);
+          int(m), int(n), int(k), int(tm), int(tn), int(tm * tn), nullptr, 0);
       return launch_status();
     }
   }
   if (residual)
     gemm_bf16_kernel<WM, WN, true, kPlain, false, RING><<<grid, block, 0, s>>>(
         static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), static_cast<const uint16_t*>(residual),
-        static_cast<uint16_t*>(c), int(m), int(n), int(k), int(tm), int(tn), int(by_xcd), nullptr, 0);
+        static_cast<uint16_t*>(c), int(m), int(n), int(k), int(tm), int(tn), by_xcd ? int(tm * tn) : 0, nullptr, 0);
   else
     gemm_bf16_kernel<WM, WN, false, kPlain, false, RING><<<grid, block, 0, s>>>(
         static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), nullptr, static_cast<uint16_t*>(c), int(m),
-        int(n), int(k), int(tm), int(tn), int(by_xcd), nullptr, 0);
+        int(n), int(k), int(tm), int(tn), by_xcd ? int(tm * tn) : 0, nullptr, 0);
   return launch_status();
 }
 
@@ -1205,7 +1206,8 @@ int launch_split(const GemmPlan& p, const uint16_t* a, const uint16_t* b, const 
   using Sh = Shape<WM, WN, RING>;
   const int64_t tm = (m + Sh::BM - 1) / Sh::BM, tn = (n + Sh::BN - 1) / Sh::BN;   // at most a tile a CU
   gemm_bf16_kernel<WM, WN, false, kSplit, false, RING><<<dim3(unsigned(tm * tn * p.splits)), dim3(kThreads), 0, s>>>(
-      a, b, nullptr, nullptr, int(m), int(n), int(k), int(tm), int(tn), 1, part, int(p.kchunk));
+      a, b, nullptr, nullptr, int(m), int(n), int(k), int(tm), int(tn), int(tm * tn * p.splits), part,
+      int(p.kchunk));
   const int64_t mn = m * n;
   const dim3 grid(unsigned((mn / 4 + 255) / 256)), block(256);
   static_assert(kMaxSplits == 8, "a finish kernel for every split count");
@@ -1287,7 +1289,7 @@ int launch_swiglu(const void* a, const void* b, void* c, int64_t m, int64_t n, i
   if (tm * tn > 0x7fffffff) return PTB_ERR_GRID;
   gemm_bf16_kernel<WM, WN, false, kSwiGLU><<<dim3(unsigned(tm * tn)), dim3(kThreads), 0, s>>>(
       static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), nullptr, static_cast<uint16_t*>(c), int(m),
-      int(n), int(k), int(tm), int(tn), 1, nullptr, 0);
+      int(n), int(k), int(tm), int(tn), int(tm * tn), nullptr, 0);
   return launch_status();
 }
 
