@@ -1319,11 +1319,11 @@ struct GroupedPlan {
 // - a group's mean rows fit one (128 experts, gate_up / down: 4 rows each 137.0 -> 119.9 / 75.0 -> 65.4 us, 60
 //   156.4 -> 145.0 / 87.9 -> 80.6; at 200 rows 255 -> 262 / 145 -> 146);
 // - the table's weights pass kStreamBytes, so that the groups of the next call are not all in the cache; and
-// - those of the groups expected to be hit pass two thirds of it.  Few of them stay in the cache, up to a block's
-//   two GEMMs in turn: with other rows routed to the same weights each call, 17 rows over 128 experts' gate_up
-//   and down (146 MB of 1.2 GB) 36.9 us either way and by strongly skewed routing 33.4 -> 34.9, with the same
-//   rows 28.3 -> 35.8; 32 rows 54.6 -> 53.2, 45.1 -> 47.0 and 53.1 -> 53.8; past the line 48 rows (gate_up
-//   alone) 78.7 -> 70.9, 96 rows 117.5 -> 107.3, 61.1 -> 60.2 and 125.1 -> 114.0.
+// - a fifth of the groups are expected to be hit.  Fewer stay in the cache up to the next call, through an expert
+//   block's two GEMMs in turn: with the same rows in each call 17 rows over 128 experts' gate_up and down (146 MB of
+//   1.2 GB) 28.3 -> 35.8 us, with other rows routed to the same weights 36.9 either way; past the line 32 rows (283
+//   MB) 53.1 -> 53.8 and 54.6 -> 53.2, 48 rows with other rows 73.0 -> 67.2, 96 rows 125.1 -> 114.0 and 117.5 ->
+//   107.3.  (A GEMM by itself on the same 100 to 250 MB in each call loses up to 9% of what the block gains.)
 GroupedPlan grouped_plan(int64_t groups, int64_t a_rows, int64_t n, int64_t k, int64_t cus) {
   struct {
     int bm, bn;
@@ -1347,8 +1347,8 @@ GroupedPlan grouped_plan(int64_t groups, int64_t a_rows, int64_t n, int64_t k, i
     if (t[i][0] * t[i][1] < t[both][0] * t[both][1]) both = i;
   }
   const int best = t[even][0] * t[even][1] > 1.3 * t[both][0] * t[both][1] ? both : even;
-  const double bytes = double(n) * double(k) * 2.0, line = double(kStreamBytes);   // a group's weight
-  return {best, mean <= tiles[best].bm && double(groups) * bytes > line && 1.5 * hit * bytes > line};
+  const double table = double(groups) * double(n) * double(k) * 2.0;
+  return {best, mean <= tiles[best].bm && table > double(kStreamBytes) && 5.0 * hit > double(groups)};
 }
 
 // A workgroup for each of the tiles there can be, up to the CUs' WGS each.

@@ -115,13 +115,13 @@ def test_32bit_buffer_offset_limits_refused(lib):
 
 def test_streaming_starts_where_the_same_bytes_again_gain(lib):
     """Caches and weights a little past the last-level cache's 256 MB are still partly found in it by the next
-    call, and so are the weights of few groups: they keep the default policy up to 300 MiB (two thirds of it for
-    the groups expected to be hit)."""
+    call, and so are the weights of few groups: they keep the default policy up to 300 MiB, and up to a fifth
+    of the groups."""
     for nkv, seq, streamed in [(64, 8192, 0), (64, 9011, 0), (64, 9600, 0), (64, 9601, 1), (128, 8192, 1), (1, 256, 0)]:
         assert plan(lib.ptb_attn_decode_plan, nkv, 4, seq)[2] == streamed, (nkv, seq)
     for groups, streamed in [(44, 0), (50, 0), (51, 1), (128, 1)]:   # weights of 6 MiB
         assert plan(lib.ptb_grouped_gemm_plan, groups, 8 * groups, 2048, 1536)[2] == streamed, groups
-    for rows, streamed in [(17, 0), (36, 0), (40, 1)]:   # few rows read few of 128 groups: 200 MiB are 33.3
+    for rows, streamed in [(17, 0), (28, 0), (29, 1)]:   # few rows read few of 128 groups, which the cache keeps
         assert plan(lib.ptb_grouped_gemm_plan, 128, rows, 2048, 1536)[2] == streamed, rows
     # few rows, which skewed routing sends to few groups: no wide tiles that would leave the CUs idle
     assert plan(lib.ptb_grouped_gemm_plan, 16, 32, 4096, 2816)[:2] == (64, 128)
